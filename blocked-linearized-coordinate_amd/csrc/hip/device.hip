@@ -33,28 +33,32 @@ constexpr uint64_t LDS_OUT_MAX = 48 * 1024;
 constexpr int LVL3_MAX_MODE_LENGTH = 100;     // src/utils.hpp:13
 constexpr int DEFAULT_TPW = 4;                // tiles of 64 per wave
 constexpr int SORTED_TPW = 16;                // tiles of 64 per wave, row-ordered kernel (most)
-constexpr uint64_t SORTED_TARGET_CHUNKS = 8192;
+constexpr int ROWS_LONG_TPW = 8;              // chunks from here on take k_mttkrp_rows' long rounds
 constexpr int DEFAULT_NPRTN = 1;
 constexpr uint32_t LVL3_CHUNKS_PER_WG = 64;
 constexpr uint32_t HOT_EXCLUDE = 64;  // hot rows kept out of the row windows
 
 static int value_size(int vdt) { return vdt == BLCO_F64 ? 8 : 4; }
 
-// Default tiles of 64 nonzeros per chunk of the row-ordered kernel.  A
-// tensor of up to 2^22 nonzeros takes shorter chunks, so that the grid keeps
-// 4096-8192 waves (2 tiles up to 2^20 nonzeros, 4 up to 2^21, 8 up to 2^22):
-// with 16 tiles such a tensor fills a fraction of the 256 CUs, and 2 tiles
-// ran tensors of 1e5-3e5 nonzeros in a third of the time (the total over
-// chunk targets from 2000 to 64000 differs by 2%).  From 2^22 nonzeros 16,
-// and 32 for FP64 rows of 256 bytes or more from 2^26 nonzeros: fewer
-// chunk ends, each of which adds its open rows to HBM (3-7% faster on the
-// 77M-nonzero modes, 0.5% on the 1.7B-nonzero ones; FP32 rows of that size
-// were faster at 16).
-static int sorted_tpw(const blco_dev* d, int rank, int ftype)
+// Default tiles of 64 nonzeros per chunk of the row-ordered kernel.  A chunk
+// of 2 tiles runs in one or two rounds of the kernel: the most waves and the
+// closest neighbours in L1.  Longer chunks pay where a chunk's end, which
+// adds its open row to HBM, is dear: rows of more than 128 bytes (FP64 at
+// rank 32: 2055 / 2130 us with 2 tiles, 1506 / 1522 with 16 on the
+// 77M-nonzero modes), and for tensors from 2^22 nonzeros hot rows whose adds
+// queue up (nnz * hot / (64 tpw) adds of 13 ns each to one row: 401 rows of a
+// Zipf(0.8) mode at 34M nonzeros 671 us with 2 tiles, 560 with 8).  FP32 at
+// rank 32: 1221 / 1162 / 1164 us with 2 tiles and 1298 / 1273 / 1274 with 16
+// on the 4.8M-row shape at 85M nonzeros, 820 / 820 / 778 and 819 / 811 / 785
+// on the 77M-nonzero modes, 81 and 141 for 2M nonzeros at rank 64.
+static int sorted_tpw(const blco_dev* d, int mode, int rank, int ftype)
 {
-    if (ftype == BLCO_F64 && rank >= 32 && d->nnz >= (1ull << 26)) return 32;
-    int t = 2;
-    while (t < SORTED_TPW && d->nnz > (uint64_t)WAVE * t * SORTED_TARGET_CHUNKS) t *= 2;
+    if (d->nnz < (1ull << 17)) return 1;  // 100k nonzeros: 5.4 us with 1, 6.3 with 2
+    if (d->nnz < (1ull << 22)) return 2;
+    const uint64_t row_bytes = (uint64_t)rank * (ftype == BLCO_F64 ? 8 : 4);
+    const uint64_t hottest = d->hot_cnt_h[mode].empty() ? 0 : d->hot_cnt_h[mode][0];
+    int t = row_bytes > 128 ? 8 : 2;
+    while (t < SORTED_TPW && hottest * row_bytes > (uint64_t)t * (2ull << 20) * 128) t *= 2;
     return t;
 }
 
@@ -655,10 +659,17 @@ static int ensure_row_ordered(blco_dev* d, int mode, int rank, int ftype)
 // Chunks of the row-ordered copy of a mode: within a group, a chunk closes at
 // the first row boundary once it holds 64 * tpw nonzeros, and never holds more
 // than twice that (a long row is cut), so most rows end inside a chunk while
-// every chunk stays short enough to spread a hot row over many waves.  A tiled
+// every chunk stays short enough to spread a hot row over many waves.  A row
+// of LONG_ROW nonzeros or more is cut into pieces of LONG_PIECE even where
+// chunks are shorter: it has waves enough so, and every piece ends in one add
+// per column to the same output row, which queue up (13 ns each) and, in
+// FP32, add their roundings (86,000 pieces of 128 nonzeros of one row: error
+// 1.6e-6 against 64 bits, 7,000 of 1500: 8e-7).  A tiled
 // copy pads every tile's chunk list with empty chunks to one common length, a
 // multiple of the waves per workgroup: the grid then has NUM_XCD equal ranges
 // of workgroups and the XCD-contiguous workgroup numbering puts tile t on XCD t.
+constexpr uint64_t LONG_ROW = 32768, LONG_PIECE = 2 * WAVE * SORTED_TPW;
+
 static const ChunkTab* sorted_chunk_table(blco_dev* d, int mode, int tpw)
 {
     for (auto& t : d->stabs[mode])
@@ -678,8 +689,14 @@ static const ChunkTab* sorted_chunk_table(blco_dev* d, int mode, int tpw)
         while (c0 < end) {
             const uint64_t run_end = (r + 1 < runs.size()) ? std::min(runs[r + 1], end) : end;
             if (run_end - c0 > cap) {  // inside a long row
-                emit(c0, c0 + cap);
-                c0 += cap;
+                const uint64_t run_len = run_end - std::max(runs[r], g.start);
+                const uint64_t piece = run_len >= LONG_ROW ? std::max(cap, LONG_PIECE) : cap;
+                const uint64_t end_piece = std::min(c0 + piece, run_end);
+                emit(c0, end_piece);
+                c0 = end_piece;
+                if (c0 < run_end) continue;
+                if (c0 == end) break;
+                ++r;
                 continue;
             }
             if (run_end - c0 >= base || run_end == end) {
@@ -694,13 +711,34 @@ static const ChunkTab* sorted_chunk_table(blco_dev* d, int mode, int tpw)
         }
     }
     std::vector<Chunk> h;
-    if (ntiles == 1) {
+    if (ntiles == 1 && cap < LONG_PIECE) {
+        // the pieces of long rows hold many times the nonzeros of the other
+        // chunks and lie together: they go to the XCDs with the fewest
+        // nonzeros, ahead of each one's equal share of the rest
+        std::vector<Chunk> rest, pieces;
+        for (const Chunk& c : tiles[0]) (c.len > cap ? pieces : rest).push_back(c);
+        if (!pieces.empty()) {
+            tiles.assign(NUM_XCD, {});
+            uint64_t held[NUM_XCD] = {};
+            const auto first = [&](int x) { return rest.size() * x / NUM_XCD; };
+            for (int x = 0; x < NUM_XCD; ++x)
+                for (size_t i = first(x); i < first(x + 1); ++i) held[x] += rest[i].len;
+            for (const Chunk& c : pieces) {
+                const int x = (int)(std::min_element(held, held + NUM_XCD) - held);
+                held[x] += c.len;
+                tiles[x].push_back(c);
+            }
+            for (int x = 0; x < NUM_XCD; ++x)
+                tiles[x].insert(tiles[x].end(), rest.begin() + first(x), rest.begin() + first(x + 1));
+        }
+    }
+    if (tiles.size() == 1) {
         h.swap(tiles[0]);
     } else {
         size_t most = 0;
         for (auto& tl : tiles) most = std::max(most, tl.size());
         most = (most + WAVES_PER_WG - 1) / WAVES_PER_WG * WAVES_PER_WG;
-        h.reserve(most * ntiles);
+        h.reserve(most * tiles.size());
         for (auto& tl : tiles) {
             h.insert(h.end(), tl.begin(), tl.end());
             h.resize(h.size() + (most - tl.size()), Chunk{0, 0, 0});
@@ -792,18 +830,23 @@ size_t rows_kernel_plan(blco_dev* d, int mode, int rank, int ftype, bool fib, Mt
     return lds;
 }
 
-// The windows cover, for the first two input modes (the inner and first
-// outer mode with fibers, 2/3 and 1/3 of HOT_TABLE_BYTES' rows; else
-// halves), the mode's consecutive rows with the most nonzeros; a window that
-// would hold fewer than 2% of the nonzeros is left out.  A workgroup fills
-// its windows once, so its waves take several chunks (as many as leave 1024
-// workgroups, at least half of the cap): up to 4 consecutive ones each in
-// the plain form, for rows of at most 128 bytes (FP64 rows of 256 bytes
-// were slower with windows); in the fiber form up to 8, with the grid walking the
-// chunks in step (chunk j of a wave is j grid widths on), and only when the
-// inner window holds a fifth of the nonzeros and the copy is not split into
-// XCD tiles -- the forms and counts that were faster on the 77M-nonzero
-// and 1.7B-nonzero workloads (a wave per chunk, no windows, otherwise).
+// k_mttkrp_rows takes one chunk per wave and keeps no windows.  The windowed
+// kernel (k_mttkrp_rows_lds) is slower wherever both were timed since the
+// former gathers with wide stream loads and coalesced adds: 40M nonzeros with
+// Zipf(1.2) modes, FP32 rank 32, 821 / 840 / 667 us with windows and 574 /
+// 577 / 531 without, FP64 rank 16 1003 / 1020 / 761 and 628 / 634 / 622; the
+// 4.8M-row shape at 85M nonzeros 2360 / 1899 / 1880 and 1420 / 1398 / 1399.
+// It runs only where BLCO_FIBERS forces a form.  There the windows cover, for
+// the first two input modes (the inner and first outer mode with fibers, 2/3
+// and 1/3 of HOT_TABLE_BYTES' rows; else halves), the mode's consecutive rows
+// with the most nonzeros; a window that would hold fewer than 2% of the
+// nonzeros is left out.  A workgroup fills its windows once, so its waves
+// take several chunks (as many as leave 1024 workgroups, at least half of the
+// cap): up to 4 consecutive ones each in the plain form, for rows of at most
+// 128 bytes; in the fiber form up to 8, with the grid walking the chunks in
+// step (chunk j of a wave is j grid widths on), and only when the inner
+// window holds a fifth of the nonzeros and the copy is not split into XCD
+// tiles.
 static size_t plan_rows(blco_dev* d, int mode, int rank, int ftype, bool fib, MttkrpArgs* a)
 {
     const uint32_t n = a->nchunks;
@@ -811,6 +854,7 @@ static size_t plan_rows(blco_dev* d, int mode, int rank, int ftype, bool fib, Mt
     a->cpw_interleave = 0;
     a->hot_lo[0] = a->hot_lo[1] = 0;
     a->hot_n[0] = a->hot_n[1] = 0;
+    if (!getenv("BLCO_FIBERS")) return 0;
     const uint64_t row_bytes = (uint64_t)rank * dtype_size(ftype);
     // up to 8 (fibers) or 4 chunks per wave while 1024 workgroups remain
     const uint32_t cap = fib ? 8 : 4, fit = n / (1024u * WAVES_PER_WG);
@@ -843,6 +887,10 @@ static size_t plan_rows(blco_dev* d, int mode, int rank, int ftype, bool fib, Mt
         progress("row-ordered kernel of mode %d: rows [%llu, %llu) of mode %d in LDS, %.1f%% of the nonzeros",
                  mode, (unsigned long long)lo[t], (unsigned long long)(lo[t] + h[t]), in[t],
                  100.0 * covered[t] / d->nnz);
+    }
+    if (!lds) {  // nothing to fill once per workgroup
+        a->cpw = 1;
+        a->cpw_interleave = 0;
     }
     return lds;
 }
@@ -913,7 +961,7 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
             break;
         case BLCO_K_ATOMIC: which = W_ATOMIC; break;
         case BLCO_K_SORTED:
-            which = W_SORTED;
+            which = W_ROWS;
             if (d->stream_data) {  // the copies are device-resident only
                 which = W_WINDOW;
                 kernel = BLCO_K_BATCHED2;
@@ -921,10 +969,10 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
             break;
         default: return fail(BLCO_EINVAL, "unknown kernel id %d", kernel);
     }
-    if (tpw <= 0) tpw = which == W_SORTED ? sorted_tpw(d, rank, ftype) : DEFAULT_TPW;
+    if (tpw <= 0) tpw = which == W_ROWS ? sorted_tpw(d, mode, rank, ftype) : DEFAULT_TPW;
     if (used_kernel) *used_kernel = kernel;
     if (d->nnz == 0) return BLCO_OK;
-    if (which == W_SORTED) {
+    if (which == W_ROWS) {
         int rc = ensure_row_ordered(d, mode, rank, ftype);
         if (rc == BLCO_ENOMEM && chosen) {  // no room for the copy: the row window
             d->sorted_failed[mode] = true;
@@ -1055,7 +1103,7 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
         if (!rc)
             rc = launch_window_reduce(out, d->part, wp->d_rows, wp->d_ptr, wp->d_idx, wp->nred, rank,
                                       otype, st);
-    } else if (which == W_SORTED) {
+    } else if (which == W_ROWS) {
         a.coords = d->d_scoords[mode];
         a.vals = d->d_svals[mode];
         a.coord_base = 0;
@@ -1066,22 +1114,27 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
         bool wide = false;
         for (int m = 0; m < d->nmodes; ++m)
             wide |= d->dims[m] * (uint64_t)rank * dtype_size(ftype) >= FACTOR_BYTES_MAX;
-        int kind = wide ? W_SORTED64 : W_SORTED;
-        if (d->sfiber[mode]) {
-            kind = wide ? W_FIBER64 : W_FIBER;
-            a.inner = d->sinner[mode];
-        }
-        if (kind == W_SORTED || kind == W_FIBER) {
+        const bool fib = d->sfiber[mode];
+        if (fib) a.inner = d->sinner[mode];
+        if (wide) {
+            rc = launch_range(d, fib ? W_FIBER64 : W_SORTED64, a, stab, 0, stab->n, ftype, st);
+        } else if (stab->n) {
             a.chunks = stab->d;
             a.chunk0 = 0;
             a.nchunks = stab->n;
-            const size_t lds = rows_kernel_plan(d, mode, rank, ftype, kind == W_FIBER, &a);
+            const size_t lds = rows_kernel_plan(d, mode, rank, ftype, fib, &a);
             // the form with LDS windows only where the plan holds some
-            if (lds) kind = kind == W_FIBER ? W_FIBER_LDS : W_SORTED_LDS;
+            int kind = fib ? W_FIBER_LDS : W_SORTED_LDS;
+            if (!lds) {
+                kind = tpw >= ROWS_LONG_TPW ? W_ROWS : W_ROWS_SHORT;
+                int j = 0;
+                if (fib) a.order[j++] = a.inner;
+                for (int m = 0; m < d->nmodes; ++m)
+                    if (m != mode && !(fib && m == a.inner)) a.order[j++] = m;
+                a.order[j] = mode;
+            }
             const uint32_t per_wg = WAVES_PER_WG * a.cpw;
-            if (stab->n) rc = launch_mttkrp(kind, a, ftype, (stab->n + per_wg - 1) / per_wg, lds, st);
-        } else {
-            rc = launch_range(d, kind, a, stab, 0, stab->n, ftype, st);
+            rc = launch_mttkrp(kind, a, ftype, (stab->n + per_wg - 1) / per_wg, lds, st);
         }
     } else if (!d->stream_data) {
         a.coords = d->d_coords;

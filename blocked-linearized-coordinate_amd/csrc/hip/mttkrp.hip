@@ -115,7 +115,8 @@ __global__ __launch_bounds__(WG) void k_fill(T* __restrict__ x, uint64_t n, T v)
 
 const void* mttkrp_kernel(int which, int nmodes, int ftype, int rank, int* C, int* L)
 {
-    Shape s = pick_shape(rank, dtype_size(ftype));
+    const bool rows = which == W_ROWS || which == W_ROWS_SHORT;
+    const Shape s = rows ? rows_shape(rank, dtype_size(ftype)) : pick_shape(rank, dtype_size(ftype));
     *C = s.C;
     *L = s.L;
     if (ftype == BLCO_F64) return mttkrp_kernel_f64(nmodes, s, which);

@@ -54,8 +54,10 @@ struct MttkrpArgs {
     const uint64_t* sc_poff;   // [entry + 1]: the entry's window is partial rows [poff[e], poff[e+1])
     uint64_t hot_poff;         // first partial row of the hot areas (entry e: + e * hot_rows)
     void* part;                // partial rows (rank wide), reduced by k_window_reduce
-    // fiber kernel only: the input mode gathered per nonzero
+    // fiber-ordered copies: the mode that varies within a fiber
     int inner;
+    // k_mttkrp_rows: the input modes in gather order, then the output mode
+    int order[BLCO_MAX_MODES];
     // row-ordered kernels: chunks per wave (consecutive, or with
     // cpw_interleave one grid width apart), and for the first two input
     // modes (the inner and first outer mode with fibers) a window of rows
@@ -75,8 +77,8 @@ struct RowsPlan {
     size_t lds;
 };
 
-enum { W_LVL1 = 0, W_LVL3 = 1, W_ATOMIC = 2, W_WINDOW = 3, W_WINDOW64 = 4, W_SORTED = 5, W_SORTED64 = 6,
-       W_FIBER = 7, W_FIBER64 = 8, W_SORTED_LDS = 9, W_FIBER_LDS = 10 };
+enum { W_LVL1 = 0, W_LVL3 = 1, W_ATOMIC = 2, W_WINDOW = 3, W_WINDOW64 = 4, W_SORTED64 = 5, W_FIBER64 = 6,
+       W_SORTED_LDS = 7, W_FIBER_LDS = 8, W_ROWS = 9, W_ROWS_SHORT = 10 };
 
 // The row-ordered and fiber kernels take 31-bit byte offsets into factors
 // of fewer bytes than this (bit 31 marks an offset into an LDS window).

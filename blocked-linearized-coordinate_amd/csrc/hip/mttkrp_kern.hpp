@@ -812,9 +812,346 @@ __global__ __launch_bounds__(WG) void k_mttkrp_fiber(MttkrpArgs a)
     }
 }
 
-// MTTKRP over a row-ordered copy with every round's decoded nonzeros staged
-// in LDS (the form of kernel 14 for factors of fewer than FACTOR_BYTES_MAX
-// bytes; k_mttkrp_sorted and k_mttkrp_fiber remain for larger ones).  Slots
+// Value of lane K of every group of L lanes (L 4, 8 or 16), by DPP: a quad
+// permute, or row_newbcast over the 16-lane rows (twice, one half of the row
+// each, for groups of 8).  No LDS access, unlike __shfl.
+template <int K, int L>
+__device__ __forceinline__ uint32_t group_bcast(uint32_t x)
+{
+    static_assert(L == 4 || L == 8 || L == 16, "DPP groups");
+    constexpr int ROW_NEWBCAST = 0x150;
+    if constexpr (L == 4) {
+        return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, K | K << 2 | K << 4 | K << 6, 0xf, 0xf, true);
+    } else if constexpr (L == 8) {
+        const int t = __builtin_amdgcn_update_dpp(0, (int)x, ROW_NEWBCAST + K, 0xf, 0x3, false);
+        return (uint32_t)__builtin_amdgcn_update_dpp(t, (int)x, ROW_NEWBCAST + 8 + K, 0xf, 0xc, false);
+    } else {
+        return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, ROW_NEWBCAST + K, 0xf, 0xf, true);
+    }
+}
+
+template <int K, int L>
+__device__ __forceinline__ float group_bcast(float x)
+{
+    return __uint_as_float(group_bcast<K, L>(__float_as_uint(x)));
+}
+
+template <int K, int L>
+__device__ __forceinline__ double group_bcast(double x)
+{
+    const uint64_t u = (uint64_t)__double_as_longlong(x);
+    const uint32_t lo = group_bcast<K, L>((uint32_t)u), hi = group_bcast<K, L>((uint32_t)(u >> 32));
+    return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+}
+
+// f(integral_constant<0>) ... f(integral_constant<E - 1>)
+template <int E, int I = 0, typename F>
+__device__ __forceinline__ void unrolled(F&& f)
+{
+    if constexpr (I < E) {
+        f(std::integral_constant<int, I>{});
+        unrolled<E, I + 1>(f);
+    }
+}
+
+// Q consecutive elements from p (aligned to their own size only)
+template <int Q, typename T>
+__device__ __forceinline__ void load_run(const T* p, T (&x)[Q])
+{
+    if constexpr (Q * sizeof(T) <= 16) {
+        struct __attribute__((packed, aligned(sizeof(T)))) V { T e[Q]; };
+        const V v = *reinterpret_cast<const V*>(p);
+        #pragma unroll
+        for (int k = 0; k < Q; ++k) x[k] = v.e[k];
+    } else {
+        T lo[Q / 2], hi[Q / 2];
+        load_run<Q / 2>(p, lo);
+        load_run<Q / 2>(p + Q / 2, hi);
+        #pragma unroll
+        for (int k = 0; k < Q / 2; ++k) {
+            x[k] = lo[k];
+            x[Q / 2 + k] = hi[k];
+        }
+    }
+}
+
+// MTTKRP over a row-ordered copy, for factors of fewer than FACTOR_BYTES_MAX
+// bytes (k_mttkrp_sorted and k_mttkrp_fiber remain for larger ones).  A wave
+// takes a chunk in rounds of up to 64 Q consecutive nonzeros: each lane loads
+// and decodes Q of them (wide loads of whole cache lines) into byte offsets
+// of the input factor rows.  Slot s of L lanes then walks its L Q consecutive
+// positions of the round in order, each position's offsets and value
+// broadcast to the slot's lanes by DPP, with the gathers of PB positions
+// issued together.  The S = 64 / L slots stay within one round of each other,
+// so neighbouring nonzeros share the input rows in L1.  Lane sub of a slot
+// holds C consecutive columns from min(C sub, width - C) on: any rank runs
+// 16-byte gathers (the last lanes' columns may repeat the ones before).
+// Positions past a slot's share gather at an offset beyond the resource's
+// range, which returns zeros.
+//
+// While a round brings no new output row, every slot keeps adding into its
+// own partial sums of the current row.  In a round that does, the partial
+// sums are first combined in slot 0, a slot stages a row when its walk leaves
+// it, and a segmented scan over the slots joins the rows that run over
+// several of them; the round's last row stays in slot 0.
+//
+// Bound: the gathers' address path (about 17 cycles a CU for each 1 KiB
+// gather instruction when the rows come from L2), and for rows of few
+// nonzeros the adds into HBM.  A finished row is not added by its slot's
+// lanes (C adds of 4 bytes each, 16 bytes apart: 2.6e9 128-byte rows/s on
+// the whole GPU) but staged in LDS; once S rows are staged, they are added
+// with consecutive lanes on consecutive columns, one memory request per 128
+// bytes: 10.2e9 rows/s.  Against the form with records of the decoded
+// nonzeros in LDS, 8-byte loads along each slot's own run and per-slot adds:
+// 77M nonzeros 12092 x 9184 x 28818, rank 32, 1049 / 1038 / 1000 -> 784 / 783
+// / 766 us a mode (FP32) and 2017 / 2032 / 1978 -> 1511 / 1532 / 1575 us
+// (FP64); 85M nonzeros on 4.8M x 1.8M x 1.8M 2361 / 1896 / 1878 -> 1296 /
+// 1206 / 1207 us; 10M nonzeros with BF16 factors 306 / 313 / 413 -> 110 / 118
+// / 109 us; 3.3M nonzeros at FP64 rank 10 117 -> 52 us.
+template <int N, typename FT, typename VT, int C, int L, int Q>
+__global__ __launch_bounds__(WG) void k_mttkrp_rows(MttkrpArgs a)
+{
+    using AT = typename Acc<FT>::type;
+    static_assert(C * L <= WAVE, "a staged row is added by at most one wave");
+    constexpr int S = WAVE / L;
+    constexpr int P = L * Q;                // positions of a slot per round
+    // positions whose gathers are issued together: up to 32 registers of rows
+    constexpr int ROW_REGS = (N - 1) * C * (int)sizeof(AT) / 4;
+    constexpr int PB = ROW_REGS <= 8 ? 4 : ROW_REGS <= 16 ? 2 : 1;
+    constexpr int KS = PB < Q ? PB : Q;     // of one lane
+    constexpr int LS = PB / KS;             // of consecutive lanes
+    constexpr int CAP = 2 * S;              // staged rows
+    constexpr uint32_t NONE = 0x80000000u;  // past every factor: gathers zeros
+    __shared__ AT s_stage[WAVES_PER_WG][CAP][C * L];
+    __shared__ uint32_t s_row[WAVES_PER_WG][CAP];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint32_t c = (uint32_t)__builtin_amdgcn_readfirstlane(
+        (int)(xcd_remap(blockIdx.x, gridDim.x) * WAVES_PER_WG + w));
+    if (c >= a.nchunks) return;  // whole wave leaves; no block barriers below
+    const Chunk ch = a.chunks[a.chunk0 + c];
+    if (ch.len == 0) return;
+    const int R = a.rank;
+    const uint32_t row_bytes = (uint32_t)R * (uint32_t)sizeof(FT);
+    // in the order of a.order: the input modes, then the output mode
+    __amdgpu_buffer_rsrc_t rs[N - 1];
+    uint32_t bc[N];
+    uint64_t mk[N];
+    int ps[N];
+    #pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const int m = a.order[j];
+        if (j < N - 1) rs[j] = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.f[m]), 0, NONE, 0x00020000);
+        bc[j] = (uint32_t)a.bcoords[(uint64_t)ch.block * N + m];
+        mk[j] = a.mask[m];
+        ps[j] = a.pos[m];
+    }
+    const int slot = lane / L, sub = lane % L;
+    AT* out = reinterpret_cast<AT*>(a.out);
+    const VT* vals = reinterpret_cast<const VT*>(a.vals) + (ch.begin - a.coord_base);
+    const uint64_t* words = a.coords + (ch.begin - a.coord_base);
+    // lanes of the slots below this one
+    const uint64_t below_slots = ((1ull << (slot * L)) - 1);
+
+    for (int cb = 0; cb < R; cb += C * L) {
+        const int width = min(R - cb, C * L);
+        const int c0 = min(sub * C, width - C);  // may lie before cb: R >= C
+        const uint32_t colb = (uint32_t)(cb + c0) * (uint32_t)sizeof(FT);
+        int gsh = 2;  // lanes per row of the staged adds: 4 to 64
+        while ((1 << gsh) < width) ++gsh;
+        AT acc[C];
+        #pragma unroll
+        for (int cc = 0; cc < C; ++cc) acc[cc] = 0;
+        int staged = 0;
+        auto add_staged = [&]() {
+            wave_lds_sync();
+            for (int i = 0; i < staged; i += WAVE >> gsh) {
+                const int r = i + (lane >> gsh), col = lane & ((1 << gsh) - 1);
+                if (r < staged && col < width)
+                    atomic_add_global(out + (uint64_t)s_row[w][r] * R + cb + col, s_stage[w][r][col]);
+            }
+            wave_lds_sync();
+            staged = 0;
+        };
+        uint32_t cur = 0;  // the row of acc
+        // stages the sums of the slots whose lanes are in `lanes`
+        auto stage = [&](uint64_t lanes) {
+            if (lanes >> lane & 1) {
+                const int at = staged + (int)__popcll(lanes & below_slots) / L;
+                #pragma unroll
+                for (int cc = 0; cc < C; ++cc)
+                    if (c0 + cc >= 0) s_stage[w][at][c0 + cc] = acc[cc];
+                if (sub == 0) s_row[w][at] = cur;
+            }
+            staged += (int)__popcll(lanes) / L;
+        };
+        // every slot's acc summed into slot 0, the others cleared
+        auto gather_slots = [&]() {
+            #pragma unroll
+            for (int d = L; d < WAVE; d <<= 1) {
+                #pragma unroll
+                for (int cc = 0; cc < C; ++cc) acc[cc] += __shfl_xor(acc[cc], d);
+            }
+            #pragma unroll
+            for (int cc = 0; cc < C; ++cc) acc[cc] = slot == 0 ? acc[cc] : (AT)0;
+        };
+        uint64_t word[Q];
+        VT val[Q];
+        // the round of `run` positions a slot from `base`
+        auto fetch = [&](uint32_t base, uint32_t run) {
+            const uint32_t q = base + slot * run + sub * Q;
+            if (q + Q <= ch.len) {
+                load_run<Q>(words + q, word);
+                load_run<Q>(vals + q, val);
+            } else {
+                #pragma unroll
+                for (int k = 0; k < Q; ++k) {
+                    const uint32_t e = min(q + k, ch.len - 1);
+                    word[k] = words[e];
+                    val[k] = vals[e];
+                }
+            }
+        };
+        // a full round, or the rest of the chunk over all slots
+        auto share = [&](uint32_t base) { return min((uint32_t)P, (ch.len - base + S - 1) / S); };
+        uint32_t base = 0, run = share(0);
+        fetch(0, run);
+        uint32_t carry = 0;   // the current row
+        bool spread = false;  // every slot holds a partial sum of it, not slot 0 alone
+        for (bool first = true; base < ch.len; first = false) {
+            const uint32_t q = base + slot * run + sub * Q;
+            uint32_t off[Q][N - 1], row[Q];
+            AT v[Q];
+            // positions of this lane in the round (none: 0 or less)
+            const int left = min((int)run - sub * Q, (int)ch.len - (int)q);
+            #pragma unroll
+            for (int k = 0; k < Q; ++k) {
+                const bool valid = k < left;
+                #pragma unroll
+                for (int j = 0; j < N - 1; ++j) {
+                    const uint32_t i = (uint32_t)((word[k] >> ps[j]) & mk[j]) | bc[j];
+                    off[k][j] = valid ? i * row_bytes : NONE;
+                }
+                row[k] = (uint32_t)((word[k] >> ps[N - 1]) & mk[N - 1]) | bc[N - 1];
+                v[k] = valid ? (AT)val[k] : (AT)0;
+            }
+            if (first) carry = (uint32_t)__builtin_amdgcn_readfirstlane((int)row[0]);
+            const uint32_t next_base = base + S * run;
+            const uint32_t lim = run;
+            const bool have = base + slot * run < ch.len;
+            if (next_base < ch.len) {  // in flight during this round's gathers
+                run = share(next_base);
+                fetch(next_base, run);
+            }
+            base = next_base;
+            bool other = false;
+            #pragma unroll
+            for (int k = 0; k < Q; ++k) other = other || (k < left && row[k] != carry);
+            const bool changed = __ballot(other) != 0;
+            // positions whose output row differs from the slot's one before
+            uint64_t change[Q];
+            #pragma unroll
+            for (int k = 0; k < Q; ++k) change[k] = 0;
+            if (changed) {
+                if (spread) gather_slots();
+                const uint32_t before = __shfl(row[Q - 1], sub > 0 ? lane - 1 : lane);
+                const uint32_t start = __shfl(row[0], slot * L);
+                cur = slot == 0 ? carry : start;
+                #pragma unroll
+                for (int k = 0; k < Q; ++k) {
+                    const uint32_t prev = k > 0 ? row[k > 0 ? k - 1 : 0] : sub > 0 ? before : cur;
+                    change[k] = __ballot(k < left && prev != row[k]);
+                }
+            }
+            constexpr uint64_t SUB0 = L == 4 ? 0x1111111111111111ull : L == 8 ? 0x0101010101010101ull
+                                                                              : 0x0001000100010001ull;
+            unrolled<L / LS>([&](auto g) {
+                if (g * LS * Q < lim) {
+                    #pragma unroll
+                    for (int kb = 0; kb < Q; kb += KS) {
+                        AT x[PB][N - 1][C];
+                        unrolled<LS>([&](auto s) {
+                            constexpr int ln = g * LS + s;
+                            #pragma unroll
+                            for (int k = 0; k < KS; ++k) {
+                                #pragma unroll
+                                for (int j = 0; j < N - 1; ++j)
+                                    load_row_buf<FT, C>(rs[j], group_bcast<ln, L>(off[kb + k][j]) + colb,
+                                                        x[s * KS + k][j]);
+                            }
+                        });
+                        unrolled<LS>([&](auto s) {
+                            constexpr int ln = g * LS + s;
+                            #pragma unroll
+                            for (int k = 0; k < KS; ++k) {
+                                const uint64_t f = change[kb + k] >> ln & SUB0;
+                                if (f) {  // uniform
+                                    const uint64_t lanes = (f << L) - f;  // every lane of the changing slots
+                                    const uint32_t next = group_bcast<ln, L>(row[kb + k]);
+                                    stage(lanes);
+                                    if (lanes >> lane & 1) {
+                                        #pragma unroll
+                                        for (int cc = 0; cc < C; ++cc) acc[cc] = 0;
+                                        cur = next;
+                                    }
+                                    if (staged >= S) add_staged();
+                                }
+                                const AT vb = group_bcast<ln, L>(v[kb + k]);
+                                #pragma unroll
+                                for (int cc = 0; cc < C; ++cc) {
+                                    AT t = vb;
+                                    #pragma unroll
+                                    for (int j = 0; j + 1 < N - 1; ++j) t *= x[s * KS + k][j][cc];
+                                    acc[cc] += t * x[s * KS + k][N - 2][cc];
+                                }
+                            }
+                        });
+                    }
+                }
+            });
+            spread = !changed;
+            if (changed) {
+                // the slots' last rows, joined by an inclusive segmented scan
+                const uint64_t alive = __ballot(have);
+                const int below = lane - L, above = lane + L;
+                const uint32_t prev_cur = __shfl(cur, below < 0 ? lane : below);
+                bool head = slot == 0 || !have || prev_cur != cur;
+                #pragma unroll
+                for (int d = 1; d < S; d <<= 1) {
+                    const int from = lane - d * L < 0 ? lane : lane - d * L;
+                    const bool pf = __shfl(head, from);
+                    AT pa[C];
+                    #pragma unroll
+                    for (int cc = 0; cc < C; ++cc) pa[cc] = __shfl(acc[cc], from);
+                    if (slot >= d) {
+                        if (!head) {
+                            #pragma unroll
+                            for (int cc = 0; cc < C; ++cc) acc[cc] += pa[cc];
+                        }
+                        head = head || pf;
+                    }
+                }
+                // slots 0 .. last hold positions; all but the last one's row are done
+                const int last = __popcll(alive) / L - 1;
+                const uint32_t next_cur = __shfl(cur, above >= WAVE ? lane : above);
+                stage(__ballot(slot < last && next_cur != cur));
+                if (staged >= S) add_staged();
+                carry = (uint32_t)__builtin_amdgcn_readlane((int)cur, last * L);
+                #pragma unroll
+                for (int cc = 0; cc < C; ++cc) {
+                    const AT t = __shfl(acc[cc], last * L + sub);
+                    acc[cc] = slot == 0 ? t : (AT)0;
+                }
+            }
+        }
+        if (spread) gather_slots();
+        cur = carry;
+        stage((1ull << L) - 1);  // slot 0
+        add_staged();
+    }
+}
+
+// MTTKRP over a row-ordered copy with the hot rows of two input modes in LDS
+// windows and every round's decoded nonzeros staged in LDS.  Slots
 // and rounds are those of k_mttkrp_sorted: each lane decodes the nonzero of
 // its own position once and writes one record -- the output row (with the
 // fiber-start bit when FIB), the 32-bit byte offsets of the input factor
@@ -830,8 +1167,8 @@ __global__ __launch_bounds__(WG) void k_mttkrp_fiber(MttkrpArgs a)
 //   starts a fiber, and their product scales the fiber's terms.
 // The flush and the final segmented scan over the slots are those of
 // k_mttkrp_sorted.
-template <int N, typename FT, typename VT, int C, int L, bool EXACT, bool FIB, bool HOT>
-__global__ __launch_bounds__(WG) void k_mttkrp_rows(MttkrpArgs a)
+template <int N, typename FT, typename VT, int C, int L, bool EXACT, bool FIB>
+__global__ __launch_bounds__(WG) void k_mttkrp_rows_lds(MttkrpArgs a)
 {
     using AT = typename Acc<FT>::type;
     constexpr int S = WAVE / L;
@@ -860,9 +1197,9 @@ __global__ __launch_bounds__(WG) void k_mttkrp_rows(MttkrpArgs a)
         for (int m = 0; m < N; ++m)
             if (m != mode && !(FIB && m == a.inner) && j < N - 1) in[j++] = m;
     }
-    constexpr int NT = !HOT ? 0 : N - 1 < 2 ? N - 1 : 2;  // input modes with a window
-    uint32_t tab_off[NT > 0 ? NT : 1] = {};
-    if (HOT) {
+    constexpr int NT = N - 1 < 2 ? N - 1 : 2;  // input modes with a window
+    uint32_t tab_off[NT] = {};
+    {
         uint32_t o = 0;
         #pragma unroll
         for (int t = 0; t < NT; ++t) {
@@ -875,7 +1212,7 @@ __global__ __launch_bounds__(WG) void k_mttkrp_rows(MttkrpArgs a)
             o += nb;
         }
     }
-    if (HOT) __syncthreads();  // the only block barrier: waves leave independently below
+    __syncthreads();  // the only block barrier: waves leave independently below
     const int slot = lane / L, sub = lane % L;
     AT* out = reinterpret_cast<AT*>(a.out);
     const VT* vals = reinterpret_cast<const VT*>(a.vals);
@@ -917,7 +1254,7 @@ __global__ __launch_bounds__(WG) void k_mttkrp_rows(MttkrpArgs a)
         // a row piece from the factor, or (offset with bit 31 set) from its
         // LDS window
         auto row_piece = [&](int m, uint32_t byte_off, AT (&x)[C]) {
-            if (HOT && (byte_off >> 31)) {
+            if (byte_off >> 31) {
                 const unsigned char* t = s_tab + (byte_off & 0x7fffffffu);
                 if (EXACT || col + C <= R) {
                     load_row<FT, C>(reinterpret_cast<const FT*>(t + colb), x);
@@ -1179,22 +1516,66 @@ inline const void* kernel_ptr(int which)
     if (which == W_LVL3) return (const void*)&k_mttkrp_lvl3<N, FT, VT, C, L, EX>;
     if (which == W_WINDOW) return (const void*)&k_mttkrp_window<N, FT, VT, C, L, EX, uint32_t>;
     if (which == W_WINDOW64) return (const void*)&k_mttkrp_window<N, FT, VT, C, L, EX, uint64_t>;
-    if (which == W_SORTED) return (const void*)&k_mttkrp_rows<N, FT, VT, C, L, EX, false, false>;
-    if (which == W_SORTED_LDS) return (const void*)&k_mttkrp_rows<N, FT, VT, C, L, EX, false, true>;
+    if (which == W_SORTED_LDS) return (const void*)&k_mttkrp_rows_lds<N, FT, VT, C, L, EX, false>;
     if (which == W_SORTED64) return (const void*)&k_mttkrp_sorted<N, FT, VT, C, L, EX, uint64_t>;
-    if (which == W_FIBER || which == W_FIBER64 || which == W_FIBER_LDS) {
+    if (which == W_FIBER64 || which == W_FIBER_LDS) {
         if constexpr (N >= 3)
-            return which == W_FIBER       ? (const void*)&k_mttkrp_rows<N, FT, VT, C, L, EX, true, false>
-                   : which == W_FIBER_LDS ? (const void*)&k_mttkrp_rows<N, FT, VT, C, L, EX, true, true>
-                                          : (const void*)&k_mttkrp_fiber<N, FT, VT, C, L, EX, uint64_t>;
+            return which == W_FIBER_LDS ? (const void*)&k_mttkrp_rows_lds<N, FT, VT, C, L, EX, true>
+                                        : (const void*)&k_mttkrp_fiber<N, FT, VT, C, L, EX, uint64_t>;
         return nullptr;  // an order-2 tensor has no fibers
     }
     return (const void*)&k_mttkrp_atomic<N, FT, VT, C, L, EX>;
 }
 
+// Columns per lane and lanes per nonzero of k_mttkrp_rows: 16-byte gathers
+// (an 8-byte one costs the address path as much; a 4-byte one a third, which
+// serves ranks of at most 8 best) over the fewest lanes that hold the rank.
+// An odd rank's bf16 rows are only 2-byte aligned: single elements.
+inline Shape rows_shape(int rank, int esize)
+{
+    // at most 64 columns a pass: a staged row is added by one wave
+    const auto lanes = [&](int C) { return rank <= 4 * C ? 4 : rank <= 8 * C || C == 8 ? 8 : 16; };
+    if (esize == 2 && rank % 2) return {1, lanes(1), false};
+    const int C = esize == 8 ? (rank <= 4 ? 1 : rank <= 8 ? 2 : 4)
+                : esize == 4 ? (rank <= 8 ? 1 : 4)
+                             : (rank <= 4 ? 1 : rank <= 8 ? 2 : rank <= 16 ? 4 : 8);
+    return {C, lanes(C), false};
+}
+
+template <int N, typename FT, typename VT, int C, int L>
+inline const void* rows_ptr(int which)
+{
+    // short runs take rounds of fewer positions
+    if (which == W_ROWS_SHORT) return (const void*)&k_mttkrp_rows<N, FT, VT, C, L, L == 16 ? 1 : 2>;
+    return (const void*)&k_mttkrp_rows<N, FT, VT, C, L, L == 16 ? 2 : 4>;
+}
+
+template <int N, typename FT, typename VT>
+inline const void* select_rows(const Shape& s, int which)
+{
+    if (s.C == 1 && s.L == 4) return rows_ptr<N, FT, VT, 1, 4>(which);
+    if constexpr (sizeof(FT) <= 4) {
+        if (s.C == 1 && s.L == 8) return rows_ptr<N, FT, VT, 1, 8>(which);
+    }
+    if (s.C == 4 && s.L == 4) return rows_ptr<N, FT, VT, 4, 4>(which);
+    if constexpr (sizeof(FT) != 4) {
+        if (s.C == 2 && s.L == 4) return rows_ptr<N, FT, VT, 2, 4>(which);
+    }
+    if constexpr (sizeof(FT) >= 4) {
+        if (s.C == 4 && s.L == 8) return rows_ptr<N, FT, VT, 4, 8>(which);
+        if (s.C == 4 && s.L == 16) return rows_ptr<N, FT, VT, 4, 16>(which);
+    } else {
+        if (s.C == 1 && s.L == 16) return rows_ptr<N, FT, VT, 1, 16>(which);
+        if (s.C == 8 && s.L == 4) return rows_ptr<N, FT, VT, 8, 4>(which);
+        if (s.C == 8 && s.L == 8) return rows_ptr<N, FT, VT, 8, 8>(which);
+    }
+    return nullptr;
+}
+
 template <int N, typename FT, typename VT>
 inline const void* select_shape(const Shape& s, int which)
 {
+    if (which == W_ROWS || which == W_ROWS_SHORT) return select_rows<N, FT, VT>(s, which);
     if (s.exact) {
         if (s.C == 1 && s.L == 8) return kernel_ptr<N, FT, VT, 1, 8, true>(which);
         if (s.C == 2 && s.L == 8) return kernel_ptr<N, FT, VT, 2, 8, true>(which);
