@@ -20,14 +20,15 @@
 //              in (f64, or f32 for the f32 / bf16 factor forms).
 //              On success the explicit inverse V^{-1} = L^{-T} L^{-1} is
 //              formed (so both outcomes leave one R x R matrix F).
-//   solve rows a group of R lanes per row: u = F m with the row of M staged
-//              in LDS; the same pass forms per-workgroup column statistics
-//              for the norm (sum of squares, or max).
-//   solve+gram the CP-ALS update of a mode in one pass on MFMA (k_solve_gram):
-//              the solve's result registers feed the Gram tiles directly.
+//   solve rows U = M F on f64 MFMA, a wave per 16 rows.
+//   als update the CP-ALS update of a mode in one pass on MFMA (k_als_update):
+//              the solve's result registers feed the Gram tiles directly, with
+//              the column statistics for the norm beside; k_als_finish turns
+//              the partial sums into lambda, Gram and fit and factors the next
+//              mode's V.
 //   lambda     lambda_r = sqrt(sum) (L2) or max(1, max) (max norm,
 //              src/kruskal_model.cpp:183-223), and 1/lambda (0 for a zero
-//              column), from the statistics folded in two passes.
+//              column).
 //   fit        one workgroup: fit = 1 - r / ||X|| with
 //              r^2 = ||X||^2 + |sum_ij l_i l_j prod_n G_n(i,j)| - 2 sum_r l_r ip_r
 //              (include/cpd.hpp:190-272).
@@ -179,124 +180,113 @@ static int fold_parts(double* part, int nparts, int W, int which, int* rows_left
 }
 
 // Pass 2 of the Gram reduction: G (R*R) and ip (R) from the P2 folded rows
-// of (R*R + R).  With inv (the new lambda's inverse), G is that of the
-// factor scaled by inv, G_ij = inv_i inv_j sum, and ip_r = inv_r c_r sum,
-// where c (colscale, may be null: ones) is the column scale the MTTKRP
-// result carries relative to that of the normalised factors.
+// of (R*R + R).
 __global__ __launch_bounds__(WAVE) void k_gram_finish(const double* __restrict__ part, int p2, int R,
-                                                      const double* __restrict__ inv,
-                                                      const double* __restrict__ colscale,
                                                       double* __restrict__ G, double* __restrict__ ip)
 {
     const int e = blockIdx.x * WAVE + threadIdx.x, W = R * R + R;
     if (e >= W) return;
     double s = part[e];
     for (int y = 1; y < p2; ++y) s += part[(uint64_t)y * W + e];
-    if (e < R * R) {
-        if (inv) s *= inv[e / R] * inv[e % R];
-        G[e] = s;
-    } else if (ip) {
-        const int r = e - R * R;
-        if (inv) s *= inv[r] * (colscale ? colscale[r] : 1.0);
-        ip[r] = s;
-    }
+    if (e < R * R) G[e] = s;
+    else if (ip) ip[e - R * R] = s;
 }
 
 // ------------------------------------------------------------- factorize
 
-// status: 0 V^{-1} in fac (by Cholesky), 1 pseudo-inverse in fac.
-// The Cholesky factor is formed right-looking (all trailing entries updated
-// in parallel after each column), which subtracts the terms of every entry
-// in the same order k = 0, 1, ... as dpotf2's column dot products.  L^{-1}
-// is formed row by row with the same parallel pattern, then
-// V^{-1} = L^{-T} L^{-1}.
-__global__ __launch_bounds__(WG) void k_factorize(GramSet gs, int nmodes, int mode, int R,
-                                                  double eps, double* __restrict__ fac,
-                                                  double* __restrict__ work,
-                                                  int* __restrict__ status,
-                                                  const double* __restrict__ dinv,
-                                                  double* __restrict__ colscale)
+__device__ __forceinline__ double lane_value(double x, int lane)
 {
-    extern __shared__ double s_a[];  // R x R: V, then L (lower); then R x R X = L^{-1}
-    double* s_x = s_a + R * R;
-    const int tid = threadIdx.x;
-    // the column scale of this mode's MTTKRP result: the product of the other
-    // factors' pending inverse scales (their stored columns carry lambda)
-    if (colscale)
-        for (int k = tid; k < R; k += WG) {
-            double c = 1.0;
-            for (int m = 0; m < nmodes; ++m)
-                if (m != mode) c *= dinv[m * R + k];
-            colscale[k] = c;
+    const uint64_t u = (uint64_t)__double_as_longlong(x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
+    return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+}
+
+// X = L^{-1} (lower, row-major in s_x) of the Cholesky factor L of s_a, by one
+// wave and in registers (R <= RP): lane i holds row i of the matrix while it
+// is factored, then column i of X.  Right-looking in both parts, so every
+// entry's terms are subtracted in the order of dpotf2's column dot products.
+// No barriers (by a workgroup in LDS the factorisation took 42 us at R = 32
+// and 16 us at R = 16).
+// False when a pivot falls to `floor_piv` or below (the same for every lane).
+template <int RP>
+__device__ __forceinline__ bool chol_inverse_wave(const double* s_a, double* s_x, int R, double floor_piv)
+{
+    const int lane = threadIdx.x & 63;
+    double a[RP];
+    #pragma unroll
+    for (int k = 0; k < RP; ++k) a[k] = (lane < R && k < R) ? s_a[lane * R + k] : (lane == k ? 1.0 : 0.0);
+    #pragma unroll
+    for (int j = 0; j < RP; ++j) {
+        if (j < R) {
+            const double ajj = lane_value(a[j], j);
+            if (!(ajj > floor_piv)) return false;
+            const double piv = sqrt(ajj);
+            a[j] = lane > j ? a[j] / piv : lane == j ? piv : 0.0;
+            #pragma unroll
+            for (int k = j + 1; k < RP; ++k) a[k] -= a[j] * lane_value(a[j], k);
         }
-    for (int e = tid; e < R * R; e += WG) {
-        double v = 1.0;
-        for (int m = 0; m < nmodes; ++m)
-            if (m != mode) v *= gs.g[m][e];
-        s_a[e] = v;
-        work[e] = v;  // keep V for the fallback
-        s_x[e] = (e / R == e % R) ? 1.0 : 0.0;
     }
+    double x[RP];
+    #pragma unroll
+    for (int k = 0; k < RP; ++k) x[k] = lane == k ? 1.0 : 0.0;
+    #pragma unroll
+    for (int k = 0; k < RP; ++k) {
+        if (k < R) {
+            x[k] /= lane_value(a[k], k);
+            #pragma unroll
+            for (int i = k + 1; i < RP; ++i) x[i] -= lane_value(a[k], i) * x[k];
+            if (lane < R) s_x[k * R + lane] = x[k];
+        }
+    }
+    return true;
+}
+
+// The same by the whole workgroup in LDS (s_a is overwritten), for ranks
+// whose rows do not fit a lane's registers.
+__device__ __forceinline__ bool chol_inverse_lds(double* s_a, double* s_x, int R, double floor_piv)
+{
+    const int tid = threadIdx.x, nt = blockDim.x;
+    for (int e = tid; e < R * R; e += nt) s_x[e] = (e / R == e % R) ? 1.0 : 0.0;
     __syncthreads();
-    // A pivot at or below R * eps * max_i V_ii means V is singular to working
-    // precision its Grams carry: its Cholesky factor would carry pivots of
-    // rounding noise (and the solve factors of that size), so the
-    // pseudo-inverse takes over -- the threshold the Jacobi fallback uses for
-    // eigenvalues.  eps is that of the Grams' accumulation (2^-52 for f64
-    // factors, 2^-23 for f32 / bf16 ones: an f32 V that is singular to f32
-    // precision clears an f64 floor or not depending on the summation order).
-    // dpotrf's own test (a pivot <= 0) is the special case of an exactly
-    // singular V.
-    double dmax = 0.0;
-    for (int i = 0; i < R; ++i) dmax = fmax(dmax, s_a[i * R + i]);
-    const double floor_piv = R * eps * dmax;
-    bool ok = true;
     for (int j = 0; j < R; ++j) {
         const double ajj = s_a[j * R + j];
-        if (!(ajj > floor_piv)) {  // every thread reads the same value: a uniform exit
-            ok = false;
-            break;
-        }
+        if (!(ajj > floor_piv)) return false;  // every thread reads the same value: a uniform exit
         const double piv = sqrt(ajj);
         __syncthreads();  // all have read a_jj
-        for (int i = j + 1 + tid; i < R; i += WG) s_a[i * R + j] /= piv;
+        for (int i = j + 1 + tid; i < R; i += nt) s_a[i * R + j] /= piv;
         if (tid == 0) s_a[j * R + j] = piv;
         __syncthreads();
         const int n = R - 1 - j;
-        for (int t = tid; t < n * n; t += WG) {
+        for (int t = tid; t < n * n; t += nt) {
             const int i = j + 1 + t / n, k = j + 1 + t % n;
             if (k <= i) s_a[i * R + k] -= s_a[i * R + j] * s_a[k * R + j];
         }
         __syncthreads();
     }
-    if (ok) {
-        for (int k = 0; k < R; ++k) {
-            const double lkk = s_a[k * R + k];
-            for (int c = tid; c <= k; c += WG) s_x[k * R + c] /= lkk;
-            __syncthreads();
-            const int n = R - 1 - k, w = k + 1;
-            for (int t = tid; t < n * w; t += WG) {
-                const int i = k + 1 + t / w, c = t % w;
-                s_x[i * R + c] -= s_a[i * R + k] * s_x[k * R + c];
-            }
-            __syncthreads();
+    for (int k = 0; k < R; ++k) {
+        const double lkk = s_a[k * R + k];
+        for (int c = tid; c <= k; c += nt) s_x[k * R + c] /= lkk;
+        __syncthreads();
+        const int n = R - 1 - k, w = k + 1;
+        for (int t = tid; t < n * w; t += nt) {
+            const int i = k + 1 + t / w, c = t % w;
+            s_x[i * R + c] -= s_a[i * R + k] * s_x[k * R + c];
         }
-        for (int e = tid; e < R * R; e += WG) {
-            int a = e / R, b = e % R;
-            int k0 = a > b ? a : b;
-            double t = 0.0;
-            for (int k = k0; k < R; ++k) t += s_x[k * R + a] * s_x[k * R + b];
-            fac[e] = t;
-        }
-        if (tid == 0) *status = 0;
-        return;
+        __syncthreads();
     }
-    __syncthreads();
+    return true;
+}
+
+// V^+ of the symmetric V in work (R x R, destroyed) into fac by cyclic Jacobi.
+__device__ void jacobi_pinv(int R, double eps, double* __restrict__ work, double* __restrict__ fac)
+{
+    const int tid = threadIdx.x, nt = blockDim.x;
     // ---- fallback: symmetric pseudo-inverse by cyclic Jacobi
     double* A = work;          // R x R, V (destroyed)
     double* Q = work + R * R;  // R x R eigenvectors (columns)
     double* wv = work + 2 * R * R;
-    for (int e = tid; e < R * R; e += WG) Q[e] = (e / R == e % R) ? 1.0 : 0.0;
+    for (int e = tid; e < R * R; e += nt) Q[e] = (e / R == e % R) ? 1.0 : 0.0;
     // s_done (sweep converged) and s_skip (one pair's rotation skipped) are
     // separate flags, and every thread has read s_done before thread 0 can
     // write either again, so no wave acts on a flag of another step.
@@ -335,14 +325,14 @@ __global__ __launch_bounds__(WG) void k_factorize(GramSet gs, int nmodes, int mo
                 __syncthreads();
                 if (s_skip) { __syncthreads(); continue; }
                 const double c = s_c, s = s_s;
-                for (int k = tid; k < R; k += WG) {
+                for (int k = tid; k < R; k += nt) {
                     double akp = A[k * R + p], akq = A[k * R + qq];
                     A[k * R + p] = c * akp - s * akq;
                     A[k * R + qq] = s * akp + c * akq;
                 }
                 __threadfence_block();
                 __syncthreads();
-                for (int k = tid; k < R; k += WG) {
+                for (int k = tid; k < R; k += nt) {
                     double apk = A[p * R + k], aqk = A[qq * R + k];
                     A[p * R + k] = c * apk - s * aqk;
                     A[qq * R + k] = s * apk + c * aqk;
@@ -367,13 +357,74 @@ __global__ __launch_bounds__(WG) void k_factorize(GramSet gs, int nmodes, int mo
     }
     __threadfence_block();
     __syncthreads();
-    for (int e = tid; e < R * R; e += WG) {
+    for (int e = tid; e < R * R; e += nt) {
         int i = e / R, j = e % R;
         double s = 0.0;
         for (int k = 0; k < R; ++k) s += Q[i * R + k] * wv[k] * Q[j * R + k];
         fac[e] = s;
     }
+}
+
+// The whole workgroup: V = s_a (R x R, also kept in work), then fac = V^{-1}
+// = L^{-T} L^{-1} with status 0, or V^+ with status 1.
+// A pivot at or below R * eps * max_i V_ii means V is singular to the working
+// precision its Grams carry: its Cholesky factor would carry pivots of
+// rounding noise (and the solve factors of that size), so the pseudo-inverse
+// takes over -- the threshold the Jacobi fallback uses for eigenvalues.  eps
+// is that of the Grams' accumulation (2^-52 for f64 factors, 2^-23 for f32 /
+// bf16 ones: an f32 V that is singular to f32 precision clears an f64 floor
+// or not depending on the summation order).  dpotrf's own test (a pivot <= 0)
+// is the special case of an exactly singular V.
+__device__ __forceinline__ void factorize_block(double* s_a, double* s_x, int R, double eps, double* fac, double* work,
+                                                int* status)
+{
+    __shared__ int s_ok;
+    const int tid = threadIdx.x, nt = blockDim.x;
+    __syncthreads();
+    double dmax = 0.0;
+    for (int i = 0; i < R; ++i) dmax = fmax(dmax, s_a[i * R + i]);
+    const double floor_piv = R * eps * dmax;
+    bool ok;
+    if (R <= 32) {
+        if (tid < WAVE) {
+            const bool r = R <= 16 ? chol_inverse_wave<16>(s_a, s_x, R, floor_piv)
+                                   : chol_inverse_wave<32>(s_a, s_x, R, floor_piv);
+            if (tid == 0) s_ok = r;
+        }
+        __syncthreads();
+        ok = s_ok != 0;
+    } else {
+        ok = chol_inverse_lds(s_a, s_x, R, floor_piv);
+    }
+    if (ok) {
+        for (int e = tid; e < R * R; e += nt) {
+            const int a = e / R, b = e % R;
+            double t = 0.0;
+            for (int k = a > b ? a : b; k < R; ++k) t += s_x[k * R + a] * s_x[k * R + b];
+            fac[e] = t;
+        }
+        if (tid == 0) *status = 0;
+        return;
+    }
+    __syncthreads();
+    jacobi_pinv(R, eps, work, fac);
     if (tid == 0) *status = 1;
+}
+
+// status: 0 V^{-1} in fac (by Cholesky), 1 pseudo-inverse in fac.
+__global__ __launch_bounds__(WG) void k_factorize(GramSet gs, int nmodes, int mode, int R, double eps,
+                                                  double* __restrict__ fac, double* __restrict__ work,
+                                                  int* __restrict__ status)
+{
+    extern __shared__ double s_a[];  // R x R: V, then R x R: L^{-1}
+    for (int e = threadIdx.x; e < R * R; e += WG) {
+        double v = 1.0;
+        for (int m = 0; m < nmodes; ++m)
+            if (m != mode) v *= gs.g[m][e];
+        s_a[e] = v;
+        work[e] = v;  // keep V for the fallback
+    }
+    factorize_block(s_a, s_a + R * R, R, eps, fac, work, status);
 }
 
 // --------------------------------------------------------- pseudo-inverse
@@ -464,59 +515,50 @@ __global__ __launch_bounds__(WG) void k_pinv_general(double* __restrict__ A, int
 
 // ------------------------------------------------------------ solve rows
 
-// U = M F with F = V^{-1} (or V^+), row by row, written as the factor dtype,
-// and per-workgroup column statistics (which 0: sum of squares, 1: max
-// seeded with 1) into stats[blockIdx][R].  A group of G lanes (G = R rounded
-// up to a power of two) takes one row: lane j holds row j of F in registers
-// and forms u_j = sum_k F[j][k] m_k, with the row of M staged in LDS (a
-// coalesced load).  The workgroup walks rows with a grid stride.
-template <typename MT, typename UT, int G>
-__global__ __launch_bounds__(WG) void k_solve_rows(const MT* __restrict__ M, UT* __restrict__ U,
-                                                   uint64_t rows, int R,
-                                                   const double* __restrict__ fac, int which,
-                                                   double* __restrict__ stats)
+// U = M F with F = V^{-1} (or V^+), a wave per 16-row tile on f64 MFMA: the
+// solve half of k_als_update.  Bound by HBM (M read and U written once): 1.8M
+// rows at rank 32, FP32, 327 us with a group of 32 lanes per row and the row
+// of M in LDS.
+template <typename MT, typename UT, int T>
+__global__ __launch_bounds__(WG) void k_solve_rows(const MT* __restrict__ M, UT* __restrict__ U, uint64_t rows, int R,
+                                                   const double* __restrict__ fac)
 {
-    constexpr int SLOTS = WG / G;
-    constexpr int RPS = 4;  // rows per slot per step: four loads in flight per lane
-    __shared__ double s_m[SLOTS * RPS][G + 1];
-    __shared__ double s_st[SLOTS][G];
-    const int j = threadIdx.x % G, slot = threadIdx.x / G;
-    const bool col = j < R;
-    double f[G];
+    constexpr int KS = 4 * T;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int i16 = lane & 15, k4 = lane >> 4;
+    double b[T][KS];
     #pragma unroll
-    for (int k = 0; k < G; ++k) f[k] = (col && k < R) ? fac[j * R + k] : 0.0;
-    double st = which == 0 ? 0.0 : 1.0;
-    const uint64_t step = (uint64_t)gridDim.x * SLOTS * RPS;
-    // every lane runs the same number of iterations: the barriers below are uniform
-    const uint64_t iters = (rows + step - 1) / step;
-    for (uint64_t it = 0; it < iters; ++it) {
-        // rows base + q * SLOTS + slot: each q a run of SLOTS consecutive rows
-        const uint64_t base = it * step + (uint64_t)blockIdx.x * SLOTS * RPS;
+    for (int ct = 0; ct < T; ++ct)
         #pragma unroll
-        for (int q = 0; q < RPS; ++q) {
-            const uint64_t row = base + (uint64_t)q * SLOTS + slot;
-            s_m[q * SLOTS + slot][j] = (row < rows && col) ? (double)M[row * (uint64_t)R + j] : 0.0;
+        for (int ks = 0; ks < KS; ++ks) {
+            const int k = 4 * ks + k4, j = 16 * ct + i16;
+            b[ct][ks] = (k < R && j < R) ? fac[j * R + k] : 0.0;
         }
-        __syncthreads();
+    const uint64_t tiles = (rows + 15) / 16, stride = (uint64_t)gridDim.x * WAVES_PER_WG;
+    for (uint64_t tile = (uint64_t)blockIdx.x * WAVES_PER_WG + w; tile < tiles; tile += stride) {
+        const uint64_t r0 = tile * 16, ra = r0 + i16;
+        d4 d[T];
         #pragma unroll
-        for (int q = 0; q < RPS; ++q) {
-            const uint64_t row = base + (uint64_t)q * SLOTS + slot;
-            double t = 0.0;
+        for (int ct = 0; ct < T; ++ct) d[ct] = d4{0, 0, 0, 0};
+        double m[KS];
+        #pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const int k = 4 * ks + k4;
+            m[ks] = (ra < rows && k < R) ? (double)M[ra * (uint64_t)R + k] : 0.0;
+        }
+        #pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
             #pragma unroll
-            for (int k = 0; k < G; ++k) t += f[k] * s_m[q * SLOTS + slot][k];
-            if (row < rows && col) {
-                U[row * (uint64_t)R + j] = from_f64<UT>(t);
-                st = which == 0 ? st + t * t : fmax(st, t);
+            for (int ct = 0; ct < T; ++ct) d[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(m[ks], b[ct][ks], d[ct], 0, 0, 0);
+        #pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const uint64_t row = r0 + k4 + 4 * v;
+            #pragma unroll
+            for (int ct = 0; ct < T; ++ct) {
+                const int col = 16 * ct + i16;
+                if (row < rows && col < R) U[row * (uint64_t)R + col] = from_f64<UT>(d[ct][v]);
             }
         }
-        __syncthreads();
-    }
-    s_st[slot][j] = st;
-    __syncthreads();
-    if (threadIdx.x < G && col) {
-        double x = s_st[0][j];
-        for (int q = 1; q < SLOTS; ++q) x = which == 0 ? x + s_st[q][j] : fmax(x, s_st[q][j]);
-        stats[(uint64_t)blockIdx.x * R + j] = x;
     }
 }
 
@@ -536,13 +578,27 @@ __global__ __launch_bounds__(WG) void k_solve_rows(const MT* __restrict__ M, UT*
 // Rows past the end load as 0 and give 0 rows of U (not stored).  Each
 // workgroup's waves take tiles with a fixed stride; its partial Gram (and
 // ip) and column statistics are combined in LDS in wave order and written to
-// part[blockIdx] (R*R + R) and stats[blockIdx] (R): deterministic.
+// part[block] (R*R + R) and stats[block] (R): deterministic.  A tile of M is
+// cleared once it is used: the next mode's MTTKRP adds into zeros without a
+// fill of its own.  One launch updates a mode of every task (the tensors of
+// a batch, or one): workgroup b belongs to the last task with first <= b.
 template <typename MT, typename UT, int T>
-__global__ __launch_bounds__(WG) void k_solve_gram(const MT* __restrict__ M, UT* __restrict__ U, uint64_t rows,
-                                                   int R, const double* __restrict__ fac,
-                                                   const double* __restrict__ colscale, int which, bool want_ip,
-                                                   double* __restrict__ stats, double* __restrict__ part)
+__global__ __launch_bounds__(WG) void k_als_update(const AlsTask* __restrict__ tasks, int ntasks, int R, int which)
 {
+    int lo = 0;
+    for (int hi = ntasks; hi - lo > 1;) {
+        const int mid = (lo + hi) >> 1;
+        if (tasks[mid].first <= blockIdx.x) lo = mid;
+        else hi = mid;
+    }
+    const AlsTask& tk = tasks[lo];
+    MT* __restrict__ M = static_cast<MT*>(tk.M);
+    UT* __restrict__ U = static_cast<UT*>(tk.U);
+    const uint64_t rows = tk.rows;
+    const double* __restrict__ fac = tk.fac;
+    const double* __restrict__ colscale = tk.colscale;
+    const bool want_ip = tk.last != 0;
+    const uint32_t block = blockIdx.x - tk.first, blocks = tk.parts;
     constexpr bool F64 = std::is_same<UT, double>::value;
     using AT = typename std::conditional<F64, double, float>::type;
     using VT = typename std::conditional<F64, d4, f4>::type;
@@ -557,7 +613,7 @@ __global__ __launch_bounds__(WG) void k_solve_gram(const MT* __restrict__ M, UT*
         #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             const int k = 4 * ks + k4, j = 16 * ct + i16;
-            b[ct][ks] = (k < R && j < R) ? fac[j * R + k] * (colscale ? colscale[k] : 1.0) : 0.0;
+            b[ct][ks] = (k < R && j < R) ? fac[j * R + k] * colscale[k] : 0.0;
         }
     VT g[NT];
     #pragma unroll
@@ -569,8 +625,8 @@ __global__ __launch_bounds__(WG) void k_solve_gram(const MT* __restrict__ M, UT*
         ipa[ct] = 0.0;
     }
     const uint64_t tiles = (rows + 15) / 16;
-    const uint64_t stride = (uint64_t)gridDim.x * WAVES_PER_WG;
-    for (uint64_t tile = (uint64_t)blockIdx.x * WAVES_PER_WG + w; tile < tiles; tile += stride) {
+    const uint64_t stride = (uint64_t)blocks * WAVES_PER_WG;
+    for (uint64_t tile = (uint64_t)block * WAVES_PER_WG + w; tile < tiles; tile += stride) {
         const uint64_t r0 = tile * 16;
         d4 d[T];
         #pragma unroll
@@ -579,9 +635,9 @@ __global__ __launch_bounds__(WG) void k_solve_gram(const MT* __restrict__ M, UT*
         #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             const int k = 4 * ks + k4;
-            const double a = (ra < rows && k < R) ? (double)M[ra * (uint64_t)R + k] : 0.0;
+            const double m = (ra < rows && k < R) ? (double)M[ra * (uint64_t)R + k] : 0.0;
             #pragma unroll
-            for (int ct = 0; ct < T; ++ct) d[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b[ct][ks], d[ct], 0, 0, 0);
+            for (int ct = 0; ct < T; ++ct) d[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(m, b[ct][ks], d[ct], 0, 0, 0);
         }
         #pragma unroll
         for (int v = 0; v < 4; ++v) {
@@ -615,6 +671,8 @@ __global__ __launch_bounds__(WG) void k_solve_gram(const MT* __restrict__ M, UT*
                     ++q;
                 }
         }
+        const uint64_t e1 = min((r0 + 16) * (uint64_t)R, rows * (uint64_t)R);
+        for (uint64_t e = r0 * (uint64_t)R + lane; e < e1; e += WAVE) M[e] = (MT)0;
     }
     // combine the waves: Gram tiles as in k_gram; statistics and ip over the
     // four row groups (k4) of a wave, then over the waves, in order
@@ -649,7 +707,7 @@ __global__ __launch_bounds__(WG) void k_solve_gram(const MT* __restrict__ M, UT*
         }
     }
     __syncthreads();
-    double* out = part + (uint64_t)blockIdx.x * (uint64_t)(R * R + R);
+    double* out = tk.part + (uint64_t)block * (uint64_t)(R * R + R);
     for (int e = threadIdx.x; e < R * R; e += WG) {
         const int i = e / R, j = e % R;
         out[e] = ((s_g[0][i][j] + s_g[1][i][j]) + s_g[2][i][j]) + s_g[3][i][j];
@@ -658,16 +716,148 @@ __global__ __launch_bounds__(WG) void k_solve_gram(const MT* __restrict__ M, UT*
         out[R * R + e] = ((s_v[0][1][e] + s_v[1][1][e]) + s_v[2][1][e]) + s_v[3][1][e];
         double a = s_v[0][0][e];
         for (int x = 1; x < WAVES_PER_WG; ++x) a = which == 0 ? a + s_v[x][0][e] : fmax(a, s_v[x][0][e]);
-        stats[(uint64_t)blockIdx.x * R + e] = a;
+        tk.stats[(uint64_t)block * R + e] = a;
     }
 }
 
+// First fold of the partial rows of tasks with more than FINISH_PARTS of them
+// (blockIdx.z: task; as k_fold_parts, sums of part and of stats by `which`).
+constexpr int FINISH_PARTS = 32;
+
+__global__ __launch_bounds__(WG) void k_als_fold(const AlsTask* __restrict__ tasks, int R, int which)
+{
+    const AlsTask& tk = tasks[blockIdx.z];
+    const int nparts = (int)tk.parts;
+    if (nparts <= FINISH_PARTS) return;
+    __shared__ double s_sum[WAVES_PER_WG][WAVE];
+    const int W = R * R + R, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int gx = (W + WAVE - 1) / WAVE;  // further columns of blocks fold the statistics
+    const bool st = (int)blockIdx.x >= gx;
+    const int e = ((int)blockIdx.x - (st ? gx : 0)) * WAVE + lane, width = st ? R : W, y = blockIdx.y, P2 = gridDim.y;
+    double* part = st ? tk.stats : tk.part;
+    const int op = st ? which : 0;
+    const double seed = op == 0 ? 0.0 : 1.0;
+    double a0 = seed, a1 = seed;
+    if (e < width) {
+        int p = y + P2 * w;
+        for (; p + WAVES_PER_WG * P2 < nparts; p += 2 * WAVES_PER_WG * P2) {
+            a0 = fold_op(op, a0, part[(uint64_t)p * width + e]);
+            a1 = fold_op(op, a1, part[(uint64_t)(p + WAVES_PER_WG * P2) * width + e]);
+        }
+        if (p < nparts) a0 = fold_op(op, a0, part[(uint64_t)p * width + e]);
+    }
+    s_sum[w][lane] = fold_op(op, a0, a1);
+    __syncthreads();
+    if (w == 0 && e < width)
+        part[(uint64_t)y * width + e] =
+            fold_op(op, fold_op(op, fold_op(op, s_sum[0][lane], s_sum[1][lane]), s_sum[2][lane]), s_sum[3][lane]);
+}
+
+// The end of a mode's update, one workgroup per task: lambda, 1/lambda and
+// the scaled Gram (and ip, and the sweep's fit after its last mode) from the
+// partial rows, then the factorisation for the mode that comes next.  One
+// launch in place of six and of a factorisation on a side stream: a sweep of
+// a small tensor is bound by its launches, and the factorisation takes a few
+// microseconds (chol_inverse_wave).  With nothing to finish (update = 0) only
+// the factorisation, for the first mode of the first sweep.
+constexpr int FINISH_WG = 512;
+
+__global__ __launch_bounds__(FINISH_WG) void k_als_finish(const AlsTask* __restrict__ tasks, int R, int which,
+                                                          double eps, int update)
+{
+    const AlsTask& tk = tasks[blockIdx.x];
+    extern __shared__ double s_dyn[];  // R x R: G, then L^{-1}; R x R: V; lambda, 1/lambda, ip (R each)
+    double *s_g = s_dyn, *s_v = s_dyn + R * R, *s_lam = s_v + R * R, *s_inv = s_lam + R, *s_ip = s_inv + R;
+    __shared__ double s_red[FINISH_WG / WAVE];
+    const int tid = threadIdx.x, W = R * R + R;
+    const int np = (int)tk.parts <= FINISH_PARTS ? (int)tk.parts : RED_SPLIT;
+    const int mode = tk.mode, nmodes = tk.nmodes;
+    if (update) {
+        for (int c = tid; c < R; c += FINISH_WG) {
+            double y = tk.stats[c];
+            for (int p = 1; p < np; ++p) y = fold_op(which, y, tk.stats[(uint64_t)p * R + c]);
+            if (which == 0) y = sqrt(y);
+            const double iv = (y == 0.0) ? 0.0 : 1.0 / y;
+            s_lam[c] = y;
+            s_inv[c] = iv;
+            tk.lambda[c] = y;
+            tk.dinv[mode * R + c] = iv;
+        }
+        __syncthreads();
+        for (int e = tid; e < W; e += FINISH_WG) {
+            double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+            int p = 0;
+            for (; p + 4 <= np; p += 4) {
+                const double* q = tk.part + (uint64_t)p * W + e;
+                s0 += q[0];
+                s1 += q[W];
+                s2 += q[2 * W];
+                s3 += q[3 * W];
+            }
+            for (; p < np; ++p) s0 += tk.part[(uint64_t)p * W + e];
+            double g = (s0 + s1) + (s2 + s3);
+            if (e < R * R) {
+                g *= s_inv[e / R] * s_inv[e % R];
+                tk.G[mode][e] = g;
+                s_g[e] = g;
+            } else {
+                const int r = e - R * R;
+                s_ip[r] = g * s_inv[r] * tk.colscale[r];
+            }
+        }
+        __syncthreads();
+        if (tk.last) {
+            // fit = 1 - r / ||X||, as k_fit
+            double sum = 0.0;
+            for (int e = tid; e < R * R; e += FINISH_WG) {
+                const int i = e / R, j = e % R;
+                if (j > i) continue;
+                double t = s_lam[i] * s_lam[j];
+                for (int m = 0; m < nmodes; ++m) t *= m == mode ? s_g[e] : tk.G[m][e];
+                sum += j < i ? 2.0 * t : t;
+            }
+            #pragma unroll
+            for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+            if ((tid & 63) == 0) s_red[tid >> 6] = sum;
+            __syncthreads();
+            if (tid == 0) {
+                double model = 0.0, inner = 0.0;
+                for (int i = 0; i < FINISH_WG / WAVE; ++i) model += s_red[i];
+                for (int r = 0; r < R; ++r) inner += s_ip[r] * s_lam[r];
+                model = fabs(model);
+                const double x2 = *tk.normX2;
+                double res = x2 + model - 2.0 * inner;
+                if (res > 0.0) res = sqrt(res);
+                tk.fit[0] = 1.0 - res / sqrt(x2);
+                tk.fit[1] = inner;
+                tk.fit[2] = model;
+            }
+        }
+    }
+    // the next mode's V, and the column scale its MTTKRP result carries: the
+    // product of the other factors' pending inverse scales
+    const int next = tk.next;
+    for (int k = tid; k < R; k += FINISH_WG) {
+        double c = 1.0;
+        for (int m = 0; m < nmodes; ++m)
+            if (m != next) c *= update && m == mode ? s_inv[k] : tk.dinv[m * R + k];
+        tk.colscale[k] = c;
+    }
+    for (int e = tid; e < R * R; e += FINISH_WG) {
+        double v = 1.0;
+        for (int m = 0; m < nmodes; ++m)
+            if (m != next) v *= update && m == mode ? s_g[e] : tk.G[m][e];
+        s_v[e] = v;
+        tk.work[e] = v;  // for the fallback
+    }
+    factorize_block(s_v, s_g, R, eps, tk.fac, tk.work, tk.status);
+}
+
 // lambda and 1/lambda (0 for a zero column) from the P2 folded rows of the
-// column statistics; dinv (may be null) receives 1/lambda too.
+// column statistics.
 __global__ __launch_bounds__(WAVE) void k_lambda_finish(const double* __restrict__ stats, int p2, int R,
                                                         int which, double* __restrict__ lambda,
-                                                        double* __restrict__ inv,
-                                                        double* __restrict__ dinv)
+                                                        double* __restrict__ inv)
 {
     const int c = blockIdx.x * WAVE + threadIdx.x;
     if (c >= R) return;
@@ -677,7 +867,6 @@ __global__ __launch_bounds__(WAVE) void k_lambda_finish(const double* __restrict
     const double iv = (y == 0.0) ? 0.0 : 1.0 / y;
     lambda[c] = y;
     inv[c] = iv;
-    if (dinv) dinv[c] = iv;
 }
 
 // ------------------------------------------------------------------- fit
@@ -731,13 +920,26 @@ __global__ __launch_bounds__(WG) void k_sumsq(const T* __restrict__ x, uint64_t 
     if (threadIdx.x == 0) part[blockIdx.x] = ((s[0] + s[1]) + s[2]) + s[3];
 }
 
-__global__ void k_sum_parts(const double* __restrict__ part, int n, double* __restrict__ out)
+// out[0] = sum of n parts, in a fixed order (61 us for 1024 by one thread).
+__global__ __launch_bounds__(WG) void k_sum_parts(const double* __restrict__ part, int n, double* __restrict__ out)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        double s = 0.0;
-        for (int i = 0; i < n; ++i) s += part[i];
-        out[0] = s;
-    }
+    __shared__ double s[WAVES_PER_WG];
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < n; i += WG) acc += part[i];
+    #pragma unroll
+    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
+    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) out[0] = ((s[0] + s[1]) + s[2]) + s[3];
+}
+
+// out = U diag(inv) in f64.
+template <typename UT>
+__global__ __launch_bounds__(WG) void k_export(const UT* __restrict__ U, uint64_t cells, int R,
+                                               const double* __restrict__ inv, double* __restrict__ out)
+{
+    for (uint64_t e = (uint64_t)blockIdx.x * WG + threadIdx.x; e < cells; e += (uint64_t)gridDim.x * WG)
+        out[e] = as_f64(U[e]) * inv[e % R];
 }
 
 __global__ __launch_bounds__(WG) void k_hadamard(double* __restrict__ x, const double* __restrict__ y,
@@ -837,8 +1039,7 @@ int launch_gram(const void* U, int dtype, uint64_t rows, int R, const void* M,
     int p2 = 0;
     rc = fold_parts(part, nparts, W, 0, &p2, st);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_gram_finish, dim3((W + WAVE - 1) / WAVE), dim3(WAVE), 0, st, part, p2, R, nullptr, nullptr,
-                       G, ip);
+    hipLaunchKernelGGL(k_gram_finish, dim3((W + WAVE - 1) / WAVE), dim3(WAVE), 0, st, part, p2, R, G, ip);
     HIP_TRY(hipGetLastError());
     return BLCO_OK;
 }
@@ -849,49 +1050,38 @@ double gram_eps(int factor_dtype)
 }
 
 int launch_factorize(const GramSet& gs, int nmodes, int mode, int R, double eps, double* fac,
-                     double* work, int* status, hipStream_t st, const double* dinv, double* colscale)
+                     double* work, int* status, hipStream_t st)
 {
     if (R < 1 || R > 64) return fail(BLCO_EUNSUPPORTED, "rank %d outside [1, 64] in the factorisation", R);
     size_t lds = sizeof(double) * 2 * (size_t)R * R;
     if (lds > 64 * 1024) HIP_TRY(hipFuncSetAttribute((const void*)k_factorize,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(k_factorize, dim3(1), dim3(WG), lds, st, gs, nmodes, mode, R, eps, fac, work, status,
-                       dinv, colscale);
+    hipLaunchKernelGGL(k_factorize, dim3(1), dim3(WG), lds, st, gs, nmodes, mode, R, eps, fac, work, status);
     HIP_TRY(hipGetLastError());
     return BLCO_OK;
 }
 
 template <typename MT, typename UT>
-static int solve_rows_t(const MT* M, UT* U, uint64_t rows, int R, const double* fac,
-                        int which, double* stats, hipStream_t st)
+static int solve_rows_t(const MT* M, UT* U, uint64_t rows, int R, const double* fac, hipStream_t st)
 {
     if (rows == 0) return BLCO_OK;
-    const uint32_t grid = solve_parts(rows);
-    if (R > 64) return fail(BLCO_EUNSUPPORTED, "rank %d > 64 in the row solve", R);
-    const int g = R <= 8 ? 8 : R <= 16 ? 16 : R <= 32 ? 32 : 64;
-    switch (g) {
-        case 8: hipLaunchKernelGGL((k_solve_rows<MT, UT, 8>), dim3(grid), dim3(WG), 0, st, M, U, rows, R, fac, which, stats); break;
-        case 16: hipLaunchKernelGGL((k_solve_rows<MT, UT, 16>), dim3(grid), dim3(WG), 0, st, M, U, rows, R, fac, which, stats); break;
-        case 32: hipLaunchKernelGGL((k_solve_rows<MT, UT, 32>), dim3(grid), dim3(WG), 0, st, M, U, rows, R, fac, which, stats); break;
-        default: hipLaunchKernelGGL((k_solve_rows<MT, UT, 64>), dim3(grid), dim3(WG), 0, st, M, U, rows, R, fac, which, stats); break;
+    const uint32_t grid = solve_gram_parts(rows);
+    switch ((R + 15) / 16) {
+        case 1: hipLaunchKernelGGL((k_solve_rows<MT, UT, 1>), dim3(grid), dim3(WG), 0, st, M, U, rows, R, fac); break;
+        case 2: hipLaunchKernelGGL((k_solve_rows<MT, UT, 2>), dim3(grid), dim3(WG), 0, st, M, U, rows, R, fac); break;
+        case 3: hipLaunchKernelGGL((k_solve_rows<MT, UT, 3>), dim3(grid), dim3(WG), 0, st, M, U, rows, R, fac); break;
+        case 4: hipLaunchKernelGGL((k_solve_rows<MT, UT, 4>), dim3(grid), dim3(WG), 0, st, M, U, rows, R, fac); break;
+        default: return fail(BLCO_EUNSUPPORTED, "rank %d > 64 in the row solve", R);
     }
     HIP_TRY(hipGetLastError());
     return BLCO_OK;
 }
 
-int launch_solve_rows(const void* M, void* U, int dtype, uint64_t rows, int R, const double* fac,
-                      int which, double* stats, hipStream_t st)
+int launch_solve_rows(const void* M, void* U, int dtype, uint64_t rows, int R, const double* fac, hipStream_t st)
 {
-    if (dtype == BLCO_F64) return solve_rows_t<double, double>((const double*)M, (double*)U, rows, R, fac, which, stats, st);
-    if (dtype == BLCO_F32) return solve_rows_t<float, float>((const float*)M, (float*)U, rows, R, fac, which, stats, st);
-    return solve_rows_t<float, bf16>((const float*)M, (bf16*)U, rows, R, fac, which, stats, st);
-}
-
-// Workgroups of the row solve (each walks rows with a grid stride).
-uint32_t solve_parts(uint64_t rows)
-{
-    const uint64_t p = (rows + 127) / 128;
-    return (uint32_t)(p < 1 ? 1 : p > 2048 ? 2048 : p);
+    if (dtype == BLCO_F64) return solve_rows_t<double, double>((const double*)M, (double*)U, rows, R, fac, st);
+    if (dtype == BLCO_F32) return solve_rows_t<float, float>((const float*)M, (float*)U, rows, R, fac, st);
+    return solve_rows_t<float, bf16>((const float*)M, (bf16*)U, rows, R, fac, st);
 }
 
 uint32_t solve_gram_parts(uint64_t rows)
@@ -901,47 +1091,45 @@ uint32_t solve_gram_parts(uint64_t rows)
 }
 
 template <typename MT, typename UT>
-static int solve_gram_t(const MT* M, UT* U, uint64_t rows, int R, const double* fac, const double* cs, int which,
-                        bool ip, double* stats, double* part, uint32_t grid, hipStream_t st)
+static void als_update_t(const AlsTask* tasks, int ntasks, int R, int which, uint32_t grid, hipStream_t st)
 {
     switch ((R + 15) / 16) {
-        case 1: hipLaunchKernelGGL((k_solve_gram<MT, UT, 1>), dim3(grid), dim3(WG), 0, st, M, U, rows, R, fac, cs, which, ip, stats, part); break;
-        case 2: hipLaunchKernelGGL((k_solve_gram<MT, UT, 2>), dim3(grid), dim3(WG), 0, st, M, U, rows, R, fac, cs, which, ip, stats, part); break;
-        case 3: hipLaunchKernelGGL((k_solve_gram<MT, UT, 3>), dim3(grid), dim3(WG), 0, st, M, U, rows, R, fac, cs, which, ip, stats, part); break;
-        case 4: hipLaunchKernelGGL((k_solve_gram<MT, UT, 4>), dim3(grid), dim3(WG), 0, st, M, U, rows, R, fac, cs, which, ip, stats, part); break;
-        default: return fail(BLCO_EUNSUPPORTED, "rank %d > 64 in the fused solve", R);
+        case 1: hipLaunchKernelGGL((k_als_update<MT, UT, 1>), dim3(grid), dim3(WG), 0, st, tasks, ntasks, R, which); break;
+        case 2: hipLaunchKernelGGL((k_als_update<MT, UT, 2>), dim3(grid), dim3(WG), 0, st, tasks, ntasks, R, which); break;
+        case 3: hipLaunchKernelGGL((k_als_update<MT, UT, 3>), dim3(grid), dim3(WG), 0, st, tasks, ntasks, R, which); break;
+        default: hipLaunchKernelGGL((k_als_update<MT, UT, 4>), dim3(grid), dim3(WG), 0, st, tasks, ntasks, R, which); break;
     }
+}
+
+static int als_finish(const AlsTask* d_tasks, int ntasks, int R, int which, double eps, int update, hipStream_t st)
+{
+    const size_t lds = sizeof(double) * (2 * (size_t)R * R + 3 * R);
+    if (lds > 64 * 1024) HIP_TRY(hipFuncSetAttribute((const void*)k_als_finish,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(k_als_finish, dim3(ntasks), dim3(FINISH_WG), lds, st, d_tasks, R, which, eps, update);
     HIP_TRY(hipGetLastError());
     return BLCO_OK;
 }
 
-int launch_solve_gram(const void* M, void* U, int dtype, uint64_t rows, int R, const double* fac,
-                      const double* colscale, int which, bool want_ip, double* stats, double* part, double* lambda,
-                      double* inv, double* dinv, double* G, double* ip, hipStream_t st)
+int launch_als_update(const AlsLaunch& l, int dtype, int R, int which, double eps, hipStream_t st)
 {
-    if (R < 1 || R > 64) return fail(BLCO_EUNSUPPORTED, "rank %d outside [1, 64] in the fused solve", R);
-    if (rows == 0) return fail(BLCO_EINVAL, "fused solve of 0 rows");
-    const uint32_t grid = solve_gram_parts(rows);
-    int rc;
-    if (dtype == BLCO_F64)
-        rc = solve_gram_t<double, double>((const double*)M, (double*)U, rows, R, fac, colscale, which, want_ip, stats,
-                                          part, grid, st);
-    else if (dtype == BLCO_F32)
-        rc = solve_gram_t<float, float>((const float*)M, (float*)U, rows, R, fac, colscale, which, want_ip, stats, part,
-                                        grid, st);
-    else
-        rc = solve_gram_t<float, bf16>((const float*)M, (bf16*)U, rows, R, fac, colscale, which, want_ip, stats, part,
-                                       grid, st);
-    if (!rc) rc = launch_lambda(stats, (int)grid, R, which, lambda, inv, st, dinv);
-    if (rc) return rc;
-    const int W = R * R + R;
-    int p2 = 0;
-    rc = fold_parts(part, (int)grid, W, 0, &p2, st);
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_gram_finish, dim3((W + WAVE - 1) / WAVE), dim3(WAVE), 0, st, part, p2, R, inv, colscale, G,
-                       want_ip ? ip : nullptr);
+    if (R < 1 || R > 64) return fail(BLCO_EUNSUPPORTED, "rank %d outside [1, 64] in the ALS update", R);
+    if (!l.ntasks) return BLCO_OK;
+    if (dtype == BLCO_F64) als_update_t<double, double>(l.d_tasks, l.ntasks, R, which, l.blocks, st);
+    else if (dtype == BLCO_F32) als_update_t<float, float>(l.d_tasks, l.ntasks, R, which, l.blocks, st);
+    else als_update_t<float, bf16>(l.d_tasks, l.ntasks, R, which, l.blocks, st);
     HIP_TRY(hipGetLastError());
-    return BLCO_OK;
+    if (l.most_parts > (uint32_t)FINISH_PARTS) {
+        const int gx = (R * R + R + WAVE - 1) / WAVE + (R + WAVE - 1) / WAVE;
+        hipLaunchKernelGGL(k_als_fold, dim3(gx, RED_SPLIT, l.ntasks), dim3(WG), 0, st, l.d_tasks, R, which);
+        HIP_TRY(hipGetLastError());
+    }
+    return als_finish(l.d_tasks, l.ntasks, R, which, eps, 1, st);
+}
+
+int launch_als_begin(const AlsLaunch& l, int R, double eps, hipStream_t st)
+{
+    return l.ntasks ? als_finish(l.d_tasks, l.ntasks, R, 0, eps, 0, st) : BLCO_OK;
 }
 
 int launch_pinv_general(double* A, int n, int* info, hipStream_t st)
@@ -953,14 +1141,13 @@ int launch_pinv_general(double* A, int n, int* info, hipStream_t st)
     return BLCO_OK;
 }
 
-int launch_lambda(double* stats, int nparts, int R, int which, double* lambda, double* inv, hipStream_t st,
-                  double* dinv)
+int launch_lambda(double* stats, int nparts, int R, int which, double* lambda, double* inv, hipStream_t st)
 {
     int p2 = 0;
     int rc = fold_parts(stats, nparts, R, which, &p2, st);
     if (rc) return rc;
     hipLaunchKernelGGL(k_lambda_finish, dim3((R + WAVE - 1) / WAVE), dim3(WAVE), 0, st, stats, p2, R, which, lambda,
-                       inv, dinv);
+                       inv);
     HIP_TRY(hipGetLastError());
     return BLCO_OK;
 }
@@ -980,7 +1167,7 @@ int launch_sumsq(const void* x, int dtype, uint64_t n, double* part, int nparts,
         hipLaunchKernelGGL(k_sumsq<double>, dim3(nparts), dim3(WG), 0, st, (const double*)x, n, part);
     else
         hipLaunchKernelGGL(k_sumsq<float>, dim3(nparts), dim3(WG), 0, st, (const float*)x, n, part);
-    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(64), 0, st, part, nparts, out);
+    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(WG), 0, st, part, nparts, out);
     HIP_TRY(hipGetLastError());
     return BLCO_OK;
 }
@@ -1025,6 +1212,18 @@ int launch_scale(void* U, int dtype, uint64_t rows, int R, const double* inv, hi
     if (dtype == BLCO_F64) hipLaunchKernelGGL(k_scale<double>, dim3(grid), dim3(WG), 0, st, (double*)U, cells, R, inv);
     else if (dtype == BLCO_F32) hipLaunchKernelGGL(k_scale<float>, dim3(grid), dim3(WG), 0, st, (float*)U, cells, R, inv);
     else hipLaunchKernelGGL(k_scale<bf16>, dim3(grid), dim3(WG), 0, st, (bf16*)U, cells, R, inv);
+    HIP_TRY(hipGetLastError());
+    return BLCO_OK;
+}
+
+int launch_export(const void* U, int dtype, uint64_t rows, int R, const double* inv, double* out, hipStream_t st)
+{
+    const uint64_t cells = rows * (uint64_t)R;
+    const uint32_t grid = (uint32_t)std::min<uint64_t>((cells + WG - 1) / WG, 8192);
+    if (grid == 0) return BLCO_OK;
+    if (dtype == BLCO_F64) hipLaunchKernelGGL(k_export<double>, dim3(grid), dim3(WG), 0, st, (const double*)U, cells, R, inv, out);
+    else if (dtype == BLCO_F32) hipLaunchKernelGGL(k_export<float>, dim3(grid), dim3(WG), 0, st, (const float*)U, cells, R, inv, out);
+    else hipLaunchKernelGGL(k_export<bf16>, dim3(grid), dim3(WG), 0, st, (const bf16*)U, cells, R, inv, out);
     HIP_TRY(hipGetLastError());
     return BLCO_OK;
 }

@@ -10,11 +10,14 @@
 // factor type) by timing the candidates on the batch itself.
 //
 // The CP-ALS driver keeps one solver state per tensor (cpals.hpp) and runs a
-// sweep as: per mode, clear every output (one stream per tensor), the
-// persistent MTTKRP (batch stream), then every tensor's ALS step on its own
-// stream; the fit of every tensor at the end.  After iteration 0 the sweep is
-// captured once into a hipGraph (the per-tensor streams fork from and join
-// the capturing stream through events) and replayed.  The reference
+// sweep on one stream, per mode: the MTTKRP of all tensors of each order in
+// one launch of kernel 14 over their row-ordered copies (k_mttkrp_rows_batch;
+// the persistent kernel where a copy does not fit), then the ALS update of
+// all tensors in two or three launches (launch_als_update), the fits among
+// them.  After iteration 0 the sweep is captured once into a hipGraph and
+// replayed.  32 tensors of 14.4M nonzeros in all, FP64, rank 16: one stream
+// and seven launches per tensor and mode took 75 ms for six sweeps and their
+// set-up.  The reference
 // decomposes one tensor per run (src/main.cpp:322-390); this has no
 // counterpart there.
 #include <algorithm>
@@ -42,14 +45,6 @@ struct BatchTensor {
     const void* f[BLCO_MAX_MODES];
     void* out;
     int nmodes;
-};
-
-struct BatchChunk {
-    uint64_t begin;
-    uint32_t len;
-    uint32_t block;
-    uint32_t tensor;  // index into the launch's descriptor array
-    uint32_t pad;
 };
 
 constexpr int BATCH_MAX_WAVES = 8;
@@ -195,12 +190,24 @@ int num_cus()
 
 using namespace blco;
 
+namespace blco {
+// The chunks of the tensors of one order for a mode of kernel 14, valid for
+// the copies named by `copies`.
+struct RowsList {
+    int mode, order;
+    std::vector<uint64_t> copies;
+    BatchChunk* d = nullptr;
+    uint32_t n = 0;
+};
+}  // namespace blco
+
 struct blco_batch {
     std::vector<blco_dev*> devs;
     int maxN = 0;
     int device = 0;
     hipStream_t st = nullptr;
     std::list<ChunkList> lists;
+    std::list<RowsList> rows_lists;
     std::vector<Tuned> tuned;
     BatchTensor* d_tens = nullptr;  // descriptors of blco_batch_mttkrp calls
     size_t tens_cap = 0;
@@ -346,6 +353,53 @@ int tune(blco_batch* b, const BatchTensor* d_tens, int mode, int rank, int ftype
     return BLCO_OK;
 }
 
+// The chunk list of the tensors `who` (all of one order) for kernel 14.
+const RowsList* rows_list(blco_batch* b, int mode, int order, const std::vector<int>& who)
+{
+    constexpr int TPW = 2;  // as for single tensors of these sizes
+    std::vector<uint64_t> copies;
+    for (int t : who) copies.push_back(b->devs[t]->copy_id[mode]);
+    for (auto it = b->rows_lists.begin(); it != b->rows_lists.end(); ++it)
+        if (it->mode == mode && it->order == order) {
+            if (it->copies == copies) return &*it;
+            if (it->d) (void)hipFree(it->d);  // a copy was rebuilt
+            b->rows_lists.erase(it);
+            break;
+        }
+    RowsList l{mode, order, copies};
+    std::vector<BatchChunk> h;
+    for (size_t k = 0; k < who.size(); ++k)
+        for (const Chunk& c : rows_batch_chunks(b->devs[who[k]], mode, TPW))
+            if (c.len) h.push_back(BatchChunk{c.begin, c.len, c.block, (uint32_t)k, 0});
+    l.n = (uint32_t)h.size();
+    if (l.n) {
+        if (hipMalloc(&l.d, sizeof(BatchChunk) * l.n) != hipSuccess) {
+            fail(BLCO_ENOMEM, "device allocation of the batch chunk list failed");
+            return nullptr;
+        }
+        if (hipMemcpy(l.d, h.data(), sizeof(BatchChunk) * l.n, hipMemcpyHostToDevice) != hipSuccess) {
+            (void)hipFree(l.d);
+            fail(BLCO_EHIP, "upload of the batch chunk list failed");
+            return nullptr;
+        }
+    }
+    b->rows_lists.push_back(l);
+    return &b->rows_lists.back();
+}
+
+int launch_rows_batch(const RowsList* l, const MttkrpArgs* d_args, int rank, int ftype, hipStream_t st)
+{
+    if (!l->n) return BLCO_OK;
+    int C, L;
+    const void* k = mttkrp_kernel(W_ROWS_BATCH, l->order, ftype, rank, &C, &L);
+    if (!k) return fail(BLCO_EUNSUPPORTED, "no batch MTTKRP kernel for %d modes, rank %d", l->order, rank);
+    const BatchChunk* chunks = l->d;
+    uint32_t n = l->n;
+    void* params[] = {(void*)&d_args, (void*)&chunks, &n};
+    HIP_TRY(hipLaunchKernel(k, dim3((n + WAVES_PER_WG - 1) / WAVES_PER_WG), dim3(WG), params, 0, st));
+    return BLCO_OK;
+}
+
 int check_call(const blco_batch* b, int mode, int rank, int ftype)
 {
     if (!b) return fail(BLCO_EINVAL, "null batch");
@@ -404,6 +458,8 @@ void blco_batch_free(blco_batch* b)
     if (!b) return;
     if (b->st) (void)hipStreamSynchronize(b->st);
     for (auto& l : b->lists)
+        if (l.d) (void)hipFree(l.d);
+    for (auto& l : b->rows_lists)
         if (l.d) (void)hipFree(l.d);
     if (b->d_tens) (void)hipFree(b->d_tens);
     if (b->st) (void)hipStreamDestroy(b->st);
@@ -476,50 +532,116 @@ int blco_batch_cpals(blco_batch* b, const blco_cpals_opts* o, double* const* U, 
     o2.verbose = 0;
     std::vector<blco_cpals_state*> S(T, nullptr);
     std::vector<BatchTensor*> d_desc(b->maxN, nullptr);
-    std::vector<double*> own_fitbuf(T, nullptr);
-    double* d_fits = nullptr;
-    double* h_fits = nullptr;
-    hipEvent_t fork = nullptr, it0 = nullptr, it1 = nullptr;
-    std::vector<hipEvent_t> join(T, nullptr);
+    char* d_pack = nullptr;     // kernel arguments and ALS tasks of every mode
+    double *d_fits = nullptr, *h_fits = nullptr;
+    double* d_export = nullptr;  // every tensor's factors and lambda, f64
+    hipEvent_t it0 = nullptr, it1 = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     auto cleanup = [&](int code) {
         if (b->st) (void)hipStreamSynchronize(b->st);
         if (gexec) (void)hipGraphExecDestroy(gexec);
         if (graph) (void)hipGraphDestroy(graph);
-        for (int t = 0; t < T; ++t) {
-            if (S[t]) {
-                S[t]->fitbuf = own_fitbuf[t];
-                blco_cpals_free(S[t]);
-            }
-            if (join[t]) (void)hipEventDestroy(join[t]);
-        }
+        for (blco_cpals_state* s : S)
+            if (s) blco_cpals_free(s);
         for (BatchTensor* p : d_desc)
             if (p) (void)hipFree(p);
+        if (d_pack) (void)hipFree(d_pack);
         if (d_fits) (void)hipFree(d_fits);
+        if (d_export) (void)hipFree(d_export);
         if (h_fits) (void)hipHostFree(h_fits);
-        for (hipEvent_t e : {fork, it0, it1})
+        for (hipEvent_t e : {it0, it1})
             if (e) (void)hipEventDestroy(e);
         return code;
     };
     for (int t = 0; t < T; ++t) {
-        rc = blco_cpals_create(b->devs[t], &o2, (const double* const*)(U + (size_t)t * BLCO_MAX_MODES), &S[t]);
+        rc = cpals_state_create(b->devs[t], &o2, (const double* const*)(U + (size_t)t * BLCO_MAX_MODES), false, &S[t]);
         if (rc) return cleanup(rc);
-        own_fitbuf[t] = S[t]->fitbuf;
-        if (hipEventCreateWithFlags(&join[t], hipEventDisableTiming) != hipSuccess)
-            return cleanup(fail(BLCO_EHIP, "event creation failed"));
+        rc = launch_fill(S[t]->Mbuf, S[t]->m_bytes / (S[t]->mt == BLCO_F64 ? 8 : 4), S[t]->mt, 0.0, S[t]->st);
+        if (rc) return cleanup(rc);
     }
     // every tensor's fit lands in one array: one read-back per iteration
+    std::vector<uint64_t> export_at(T + 1, 0);
+    for (int t = 0; t < T; ++t) {
+        export_at[t + 1] = export_at[t] + R;
+        for (int m = 0; m < S[t]->N; ++m) export_at[t + 1] += S[t]->d->dims[m] * (uint64_t)R;
+    }
     if (hipMalloc((void**)&d_fits, sizeof(double) * 4 * T) != hipSuccess ||
+        hipMalloc((void**)&d_export, sizeof(double) * export_at[T]) != hipSuccess ||
         hipHostMalloc((void**)&h_fits, sizeof(double) * 4 * T, hipHostMallocDefault) != hipSuccess)
-        return cleanup(fail(BLCO_ENOMEM, "fit buffers"));
-    for (int t = 0; t < T; ++t) S[t]->fitbuf = d_fits + 4 * t;
-    if (hipEventCreateWithFlags(&fork, hipEventDisableTiming) != hipSuccess || hipEventCreate(&it0) != hipSuccess ||
-        hipEventCreate(&it1) != hipSuccess)
+        return cleanup(fail(BLCO_ENOMEM, "batch result buffers"));
+    if (hipEventCreate(&it0) != hipSuccess || hipEventCreate(&it1) != hipSuccess)
         return cleanup(fail(BLCO_EHIP, "event creation failed"));
-    // per-mode descriptors (the solver buffers do not move) and launch shapes
+    // per mode: the tensors of each order through kernel 14 over their copies,
+    // or the mode's members through the tuned persistent kernel when a copy
+    // cannot be had; then the members' update tasks
+    struct Group { const RowsList* list; size_t args; };
+    std::vector<std::vector<Group>> groups(b->maxN);
+    std::vector<bool> by_rows(b->maxN, true);
     std::vector<Tuned> shape(b->maxN);
+    std::vector<char> pack;
+    auto append = [&](const void* p, size_t bytes) {
+        const size_t at = (pack.size() + 63) / 64 * 64;
+        pack.resize(at + bytes);
+        std::memcpy(pack.data() + at, p, bytes);
+        return at;
+    };
+    std::vector<AlsLaunch> upd(b->maxN);
+    std::vector<size_t> task_at(b->maxN + 1);
     for (int n = 0; n < b->maxN; ++n) {
+        const std::vector<int> mem = members(b, n);
+        for (int t : mem) {
+            rc = rows_batch_prepare(b->devs[t], n, R, ft);
+            if (rc == BLCO_ENOMEM || rc == BLCO_EUNSUPPORTED) by_rows[n] = false;
+            else if (rc) return cleanup(rc);
+            if (!by_rows[n]) break;
+        }
+        std::vector<AlsTask> tasks;
+        for (int t : mem) {
+            AlsTask k = S[t]->tasks[n];
+            k.fit = d_fits + 4 * t;
+            k.first = upd[n].blocks;
+            upd[n].blocks += k.parts;
+            upd[n].most_parts = std::max(upd[n].most_parts, k.parts);
+            tasks.push_back(k);
+        }
+        upd[n].ntasks = (int)tasks.size();
+        task_at[n] = append(tasks.data(), sizeof(AlsTask) * tasks.size());
+        if (!by_rows[n]) continue;
+        for (int order = 2; order <= BLCO_MAX_MODES; ++order) {
+            std::vector<int> who;
+            for (int t : mem)
+                if (b->devs[t]->nmodes == order) who.push_back(t);
+            if (who.empty()) continue;
+            std::vector<MttkrpArgs> args;
+            for (int t : who) {
+                MttkrpArgs a = rows_batch_args(b->devs[t], n, R);
+                for (int m = 0; m < order; ++m) a.f[m] = S[t]->U[m];
+                a.out = S[t]->Mbuf;
+                args.push_back(a);
+            }
+            const RowsList* l = rows_list(b, n, order, who);
+            if (!l) return cleanup(BLCO_ENOMEM);
+            groups[n].push_back(Group{l, append(args.data(), sizeof(MttkrpArgs) * args.size())});
+        }
+    }
+    // the tasks of every tensor's last mode, whose successor is mode 0
+    AlsLaunch begin;
+    {
+        std::vector<AlsTask> tasks;
+        for (int t = 0; t < T; ++t) tasks.push_back(S[t]->tasks[S[t]->N - 1]);
+        begin.ntasks = T;
+        task_at[b->maxN] = append(tasks.data(), sizeof(AlsTask) * tasks.size());
+    }
+    if (hipMalloc((void**)&d_pack, pack.size()) != hipSuccess) return cleanup(fail(BLCO_ENOMEM, "batch descriptors"));
+    if (hipMemcpy(d_pack, pack.data(), pack.size(), hipMemcpyHostToDevice) != hipSuccess)
+        return cleanup(fail(BLCO_EHIP, "descriptor upload failed"));
+    for (int n = 0; n < b->maxN; ++n) upd[n].d_tasks = reinterpret_cast<const AlsTask*>(d_pack + task_at[n]);
+    begin.d_tasks = reinterpret_cast<const AlsTask*>(d_pack + task_at[b->maxN]);
+    for (int t = 0; t < T; ++t)
+        if (hipStreamSynchronize(S[t]->st) != hipSuccess) return cleanup(fail(BLCO_EHIP, "setup failed"));
+    for (int n = 0; n < b->maxN; ++n) {
+        if (by_rows[n]) continue;
         std::vector<void*> F((size_t)T * BLCO_MAX_MODES, nullptr), O(T, nullptr);
         for (int t = 0; t < T; ++t) {
             for (int m = 0; m < S[t]->N; ++m) F[(size_t)t * BLCO_MAX_MODES + m] = S[t]->U[m];
@@ -530,36 +652,61 @@ int blco_batch_cpals(blco_batch* b, const blco_cpals_opts* o, double* const* U, 
             return cleanup(fail(BLCO_ENOMEM, "descriptor allocation failed"));
         if (!v.empty() && hipMemcpy(d_desc[n], v.data(), sizeof(BatchTensor) * v.size(), hipMemcpyHostToDevice) != hipSuccess)
             return cleanup(fail(BLCO_EHIP, "descriptor upload failed"));
-        rc = tune(b, d_desc[n], n, R, ft, &shape[n]);  // scribbles on the outputs, cleared below
+        rc = tune(b, d_desc[n], n, R, ft, &shape[n]);
         if (rc) return cleanup(rc);
+        for (int t : members(b, n)) {  // the tuning runs left their sums there
+            rc = launch_fill(S[t]->Mbuf, S[t]->m_bytes / (S[t]->mt == BLCO_F64 ? 8 : 4), S[t]->mt, 0.0, b->st);
+            if (rc) return cleanup(rc);
+        }
     }
-    if (hipStreamSynchronize(b->st) != hipSuccess) return cleanup(fail(BLCO_EHIP, "tuning failed"));
-
-    // the sweep: per mode clear outputs, one persistent MTTKRP, every ALS step
-    auto fork_each = [&](const std::vector<int>& who, auto&& body) -> int {
-        HIP_TRY(hipEventRecord(fork, b->st));
-        for (int t : who) {
-            HIP_TRY(hipStreamWaitEvent(S[t]->st, fork, 0));
-            int r = body(t);
+    const double eps = S[0]->eps;
+    auto sweep = [&](int which_norm) -> int {
+        for (int n = 0; n < b->maxN; ++n) {
+            int r = BLCO_OK;
+            for (const Group& g : groups[n]) {
+                r = launch_rows_batch(g.list, reinterpret_cast<const MttkrpArgs*>(d_pack + g.args), R, ft, b->st);
+                if (r) return r;
+            }
+            if (!by_rows[n]) r = launch_batch(b, d_desc[n], n, R, ft, shape[n].tpw, shape[n].waves, shape[n].wpc, b->st);
+            if (!r) r = launch_als_update(upd[n], ft, R, which_norm, eps, b->st);
             if (r) return r;
-            HIP_TRY(hipEventRecord(join[t], S[t]->st));
-            HIP_TRY(hipStreamWaitEvent(b->st, join[t], 0));
         }
         return BLCO_OK;
     };
-    std::vector<int> all(T);
-    for (int t = 0; t < T; ++t) all[t] = t;
-    auto sweep = [&](int which_norm) -> int {
-        for (int n = 0; n < b->maxN; ++n) {
-            const std::vector<int> mem = members(b, n);
-            int r = fork_each(mem, [&](int t) {
-                return launch_fill(S[t]->Mbuf, S[t]->d->dims[n] * (uint64_t)R, S[t]->mt, 0.0, S[t]->st);
-            });
-            if (!r) r = launch_batch(b, d_desc[n], n, R, ft, shape[n].tpw, shape[n].waves, shape[n].wpc, b->st);
-            if (!r) r = fork_each(mem, [&](int t) { return enqueue_step(S[t], n, which_norm, S[t]->st); });
-            if (r) return r;
+    // results of the tensors `who` (every sweep so far is done) to the caller
+    std::vector<double> host;
+    auto fetch = [&](const std::vector<int>& who) -> int {
+        if (who.empty()) return BLCO_OK;
+        try {
+            host.resize(export_at[T]);
+        } catch (const std::bad_alloc&) {
+            return fail(BLCO_ENOMEM, "host copy of the factors");
         }
-        return fork_each(all, [&](int t) { return enqueue_fit(S[t], S[t]->st); });
+        for (int t : who) {
+            int r = enqueue_export(S[t], d_export + export_at[t]);
+            if (r) return r;
+            HIP_TRY(hipMemcpyAsync(d_export + export_at[t + 1] - R, S[t]->lambda, sizeof(double) * R,
+                                   hipMemcpyDeviceToDevice, S[t]->st));
+        }
+        for (int t : who) HIP_TRY(hipStreamSynchronize(S[t]->st));
+        // neighbouring tensors in one copy
+        for (size_t i = 0; i < who.size();) {
+            size_t j = i + 1;
+            while (j < who.size() && who[j] == who[j - 1] + 1) ++j;
+            const uint64_t lo = export_at[who[i]], hi = export_at[who[j - 1] + 1];
+            HIP_TRY(hipMemcpy(host.data() + lo, d_export + lo, sizeof(double) * (hi - lo), hipMemcpyDeviceToHost));
+            i = j;
+        }
+        for (int t : who) {
+            const double* from = host.data() + export_at[t];
+            for (int m = 0; m < S[t]->N; ++m) {
+                const uint64_t n = S[t]->d->dims[m] * (uint64_t)R;
+                if (double* to = U[(size_t)t * BLCO_MAX_MODES + m]) std::memcpy(to, from, sizeof(double) * n);
+                from += n;
+            }
+            if (lambda) std::memcpy(lambda + (size_t)t * R, from, sizeof(double) * R);
+        }
+        return BLCO_OK;
     };
 
     std::vector<double> fit_old(T, 0.0);
@@ -570,7 +717,8 @@ int blco_batch_cpals(blco_batch* b, const blco_cpals_opts* o, double* const* U, 
     for (; it < o->max_iters && alive > 0; ++it) {
         HIP_TRY(hipEventRecord(it0, b->st));
         if (it == 0) {
-            rc = sweep(0);
+            rc = launch_als_begin(begin, R, eps, b->st);
+            if (!rc) rc = sweep(0);
             if (rc) return cleanup(rc);
         } else {
             if (!gexec) {
@@ -593,6 +741,7 @@ int blco_batch_cpals(blco_batch* b, const blco_cpals_opts* o, double* const* U, 
             ms_sum += ms;
             ++ms_n;
         }
+        std::vector<int> done;
         for (int t = 0; t < T; ++t) {
             if (stopped_at[t]) continue;
             const double f = h_fits[4 * t];
@@ -603,16 +752,18 @@ int blco_batch_cpals(blco_batch* b, const blco_cpals_opts* o, double* const* U, 
                 // this tensor's result is final: keep it before later sweeps move it
                 stopped_at[t] = it + 1;
                 --alive;
-                rc = blco_cpals_get(S[t], U + (size_t)t * BLCO_MAX_MODES, lambda ? lambda + (size_t)t * R : nullptr);
-                if (rc) return cleanup(rc);
+                done.push_back(t);
             }
         }
+        rc = fetch(done);
+        if (rc) return cleanup(rc);
     }
+    std::vector<int> never;  // max_iters == 0
+    for (int t = 0; t < T; ++t)
+        if (!stopped_at[t]) never.push_back(t);
+    rc = fetch(never);
+    if (rc) return cleanup(rc);
     for (int t = 0; t < T; ++t) {
-        if (!stopped_at[t]) {  // max_iters == 0
-            rc = blco_cpals_get(S[t], U + (size_t)t * BLCO_MAX_MODES, lambda ? lambda + (size_t)t * R : nullptr);
-            if (rc) return cleanup(rc);
-        }
         if (fits) fits[t] = fit_old[t];
         if (iters) iters[t] = stopped_at[t];
     }

@@ -16,17 +16,18 @@
 // Its Gram is formed from the stored factor and scaled by 1 / lambda on
 // both sides; the MTTKRP of a later mode then carries the product c of the
 // other factors' lambdas in its columns, and that mode's solve multiplies
-// M by c^{-1} (folded into F).  Mathematically the same step; each mode's
-// update is one MFMA kernel that reads M once and writes U_n once, forming
-// the Gram from the solve's registers (launch_solve_gram), instead of a
-// solve, an in-place rescale and a Gram pass.  blco_cpals_get applies
-// 1 / lambda.
+// M by c^{-1} (folded into F); blco_cpals_get applies 1 / lambda.  A mode's
+// update is one MFMA kernel that reads M once, writes U_n once, clears M for
+// the next MTTKRP and forms the Gram from the solve's registers, and a
+// one-workgroup kernel that turns the partial sums into lambda and G_n and
+// factors the next mode's V (launch_als_update).
 //
 // Everything stays on one stream with no host round trip inside a sweep;
-// the host reads back the fit (8 bytes) once per iteration.  With use_graph
+// the host reads back the fit (24 bytes) once per iteration.  With use_graph
 // one sweep (after iteration 0, whose norm differs) is captured into a
-// hipGraph and replayed; the output buffer is cleared by a fill kernel, never
-// by a memset node.
+// hipGraph and replayed; the output buffer is cleared by kernels, never by a
+// memset node.
+#include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -44,7 +45,7 @@ using namespace blco;
 
 namespace blco {
 
-void to_dtype(const double* src, void* dst, uint64_t n, int dt)
+static void to_dtype(const double* src, void* dst, uint64_t n, int dt)
 {
     if (dt == BLCO_F64) std::memcpy(dst, src, n * 8);
     else if (dt == BLCO_F32) {
@@ -62,119 +63,36 @@ void to_dtype(const double* src, void* dst, uint64_t n, int dt)
     }
 }
 
-void from_dtype(const void* src, double* dst, uint64_t n, int dt)
-{
-    if (dt == BLCO_F64) std::memcpy(dst, src, n * 8);
-    else if (dt == BLCO_F32) {
-        const float* f = (const float*)src;
-        for (uint64_t i = 0; i < n; ++i) dst[i] = f[i];
-    } else {
-        const uint16_t* b = (const uint16_t*)src;
-        for (uint64_t i = 0; i < n; ++i) {
-            uint32_t u = (uint32_t)b[i] << 16;
-            float x;
-            std::memcpy(&x, &u, 4);
-            dst[i] = x;
-        }
-    }
-}
-
-int enqueue_factorize(blco_cpals_state* s, int n, hipStream_t st)
-{
-    GramSet gs;
-    for (int m = 0; m < s->N; ++m) gs.g[m] = s->G[m];
-    // the pivot floor of f64 unless the caller asked for the factors' precision
-    const double eps = s->o.solve_floor ? gram_eps(s->ft) : gram_eps(BLCO_F64);
-    return launch_factorize(gs, s->N, n, s->R, eps, s->fac, s->work, s->status, st, s->dinv, s->colscale);
-}
-
-int enqueue_step(blco_cpals_state* s, int n, int which_norm, hipStream_t st)
-{
-    int rc = enqueue_factorize(s, n, st);
-    return rc ? rc : enqueue_update(s, n, which_norm, st);
-}
-
-int enqueue_update(blco_cpals_state* s, int n, int which_norm, hipStream_t st)
-{
-    const int N = s->N, R = s->R;
-    const uint64_t I = s->d->dims[n];
-    const int last = s->order[N - 1];
-    return launch_solve_gram(s->Mbuf, s->U[n], s->ft, I, R, s->fac, s->colscale, which_norm, n == last, s->stats,
-                             s->gram_part, s->lambda, s->inv, s->dinv + (size_t)n * R, s->G[n], s->ip, st);
-}
-
-int enqueue_fit(blco_cpals_state* s, hipStream_t st)
-{
-    GramSet gs;
-    for (int m = 0; m < s->N; ++m) gs.g[m] = s->G[m];
-    return launch_fit(gs, s->N, s->R, s->lambda, s->ip, s->normX2, s->fitbuf, st);
-}
-
-// Enqueues one ALS sweep (all modes) and the fit kernel.
+// Enqueues one ALS sweep: per mode the MTTKRP and the update, the last one
+// with the fit.
 static int enqueue_sweep(blco_cpals_state* s, int which_norm, bool timed)
 {
     blco_dev* d = s->d;
-    const int N = s->N, R = s->R;
-    for (int k = 0; k < N; ++k) {
+    for (int k = 0; k < s->N; ++k) {
         const int n = s->order[k];
-        // V_n's factorisation on the side stream, beside the MTTKRP
-        HIP_TRY(hipEventRecord(s->fork[n], s->st));
-        HIP_TRY(hipStreamWaitEvent(s->side, s->fork[n], 0));
-        int rc = enqueue_factorize(s, n, s->side);
-        if (rc) return rc;
-        HIP_TRY(hipEventRecord(s->join[n], s->side));
-        rc = launch_fill(s->Mbuf, d->dims[n] * (uint64_t)R, s->mt, 0.0, s->st);
-        if (rc) return rc;
         if (timed) HIP_TRY(hipEventRecord(s->ev0[n], s->st));
-        rc = mttkrp(d, n, R, s->ft, s->U, s->Mbuf, s->o.kernel, s->o.nprtn, s->o.thread_cf, s->st,
-                    &s->kern[n]);
+        int rc = mttkrp(d, n, s->R, s->ft, s->U, s->Mbuf, s->o.kernel, s->o.nprtn, s->o.thread_cf, s->st,
+                        &s->kern[n]);
         if (rc) return rc;
         if (timed) HIP_TRY(hipEventRecord(s->ev1[n], s->st));
-        HIP_TRY(hipStreamWaitEvent(s->st, s->join[n], 0));
-        rc = enqueue_update(s, n, which_norm, s->st);
+        rc = launch_als_update(s->upd[n], s->ft, s->R, which_norm, s->eps, s->st);
         if (rc) return rc;
     }
-    return enqueue_fit(s, s->st);
+    return BLCO_OK;
 }
 
-static double now_ms()
+int enqueue_export(blco_cpals_state* s, double* out)
 {
-    return std::chrono::duration<double, std::milli>(
-               std::chrono::steady_clock::now().time_since_epoch()).count();
-}
-
-}  // namespace blco
-
-extern "C" {
-
-void blco_cpals_free(blco_cpals_state* s)
-{
-    if (!s) return;
-    if (s->st) (void)hipStreamSynchronize(s->st);
-    if (s->side) (void)hipStreamSynchronize(s->side);
-    if (s->gexec) (void)hipGraphExecDestroy(s->gexec);
-    if (s->graph) (void)hipGraphDestroy(s->graph);
-    for (int m = 0; m < BLCO_MAX_MODES; ++m) {
-        if (s->U[m]) (void)hipFree(s->U[m]);
-        if (s->G[m]) (void)hipFree(s->G[m]);
-        if (s->ev0[m]) (void)hipEventDestroy(s->ev0[m]);
-        if (s->ev1[m]) (void)hipEventDestroy(s->ev1[m]);
-        if (s->fork[m]) (void)hipEventDestroy(s->fork[m]);
-        if (s->join[m]) (void)hipEventDestroy(s->join[m]);
+    for (int m = 0; m < s->N; ++m) {
+        const int rc = launch_export(s->U[m], s->ft, s->d->dims[m], s->R, s->dinv + (size_t)m * s->R, out, s->st);
+        if (rc) return rc;
+        out += s->d->dims[m] * (uint64_t)s->R;
     }
-    if (s->side) (void)hipStreamDestroy(s->side);
-    void* bufs[] = {s->Mbuf, s->lambda, s->inv, s->fac, s->work, s->status, s->gram_part,
-                    s->stats, s->ip, s->fitbuf, s->norm_part, s->dinv, s->colscale};
-    for (void* p : bufs)
-        if (p) (void)hipFree(p);
-    if (s->h_fit) (void)hipHostFree(s->h_fit);
-    if (s->it0) (void)hipEventDestroy(s->it0);
-    if (s->it1) (void)hipEventDestroy(s->it1);
-    delete s;
+    return BLCO_OK;
 }
 
-int blco_cpals_create(blco_dev* d, const blco_cpals_opts* o, const double* const* U,
-                      blco_cpals_state** out)
+int cpals_state_create(blco_dev* d, const blco_cpals_opts* o, const double* const* U, bool own_io,
+                       blco_cpals_state** out)
 {
     if (!d || !o || !U || !out) return fail(BLCO_EINVAL, "null argument");
     *out = nullptr;
@@ -207,46 +125,100 @@ int blco_cpals_create(blco_dev* d, const blco_cpals_opts* o, const double* const
         for (int i = 1; i < N; ++i)
             for (int j = i; j > 0 && d->dims[s->order[j]] > d->dims[s->order[j - 1]]; --j)
                 std::swap(s->order[j], s->order[j - 1]);
-    const int fsz = dtype_size(s->ft), msz = s->mt == BLCO_F64 ? 8 : 4;
-    uint64_t maxI = 0;
-    for (int m = 0; m < N; ++m) maxI = std::max(maxI, d->dims[m]);
-    std::vector<char> stage;
+    s->eps = o->solve_floor ? gram_eps(s->ft) : gram_eps(BLCO_F64);  // pivot floor: f64's unless asked for
+    const int fsz = dtype_size(s->ft), msz = s->mt == BLCO_F64 ? 8 : 4, nnorm = 1024;
+    uint64_t maxI = 0, parts = 1;
     for (int m = 0; m < N; ++m) {
-        uint64_t n = d->dims[m] * (uint64_t)R;
-        if (hipMalloc(&s->U[m], n * fsz) != hipSuccess || hipMalloc(&s->G[m], sizeof(double) * R * R) != hipSuccess)
-            return bad(fail(BLCO_ENOMEM, "factor allocation failed"));
-        stage.resize(n * fsz);
-        to_dtype(U[m], stage.data(), n, s->ft);
-        if (hipMemcpy(s->U[m], stage.data(), n * fsz, hipMemcpyHostToDevice) != hipSuccess)
+        int gp;
+        uint64_t rpw;
+        gram_parts(d->dims[m], &gp, &rpw);
+        maxI = std::max(maxI, d->dims[m]);
+        parts = std::max<uint64_t>(parts, std::max<uint64_t>((uint64_t)gp, solve_gram_parts(d->dims[m])));
+    }
+    // one allocation: offsets first, then the addresses
+    uint64_t total = 0;
+    auto take = [&](uint64_t bytes) {
+        const uint64_t at = total;
+        total += (bytes + 255) / 256 * 256;
+        return at;
+    };
+    uint64_t oU[BLCO_MAX_MODES], oG[BLCO_MAX_MODES];
+    for (int m = 0; m < N; ++m) oU[m] = take(d->dims[m] * (uint64_t)R * fsz);
+    const uint64_t factor_bytes = total;
+    for (int m = 0; m < N; ++m) oG[m] = take(sizeof(double) * R * R);
+    s->m_bytes = maxI * R * msz;
+    const uint64_t oM = take(s->m_bytes), olam = take(8 * R), ofac = take(8 * R * R),
+                   owork = take(8 * (2 * R * R + R)), ostat = take(sizeof(int)), opart = take(8 * parts * (R * R + R)),
+                   ostats = take(8 * parts * R), ofit = take(8 * 4), onorm = take(8 * (nnorm + 1)),
+                   odinv = take(8 * (uint64_t)N * R), ocs = take(8 * R), otask = take(sizeof(AlsTask) * N);
+    if (hipMalloc(&s->arena, total) != hipSuccess) return bad(fail(BLCO_ENOMEM, "solver allocation failed (%llu bytes)",
+                                                                   (unsigned long long)total));
+    char* base = static_cast<char*>(s->arena);
+    auto dbl = [&](uint64_t at) { return reinterpret_cast<double*>(base + at); };
+    for (int m = 0; m < N; ++m) {
+        s->U[m] = base + oU[m];
+        s->G[m] = dbl(oG[m]);
+    }
+    s->Mbuf = base + oM;
+    s->lambda = dbl(olam);
+    s->fac = dbl(ofac);
+    s->work = dbl(owork);
+    s->status = reinterpret_cast<int*>(base + ostat);
+    s->part = dbl(opart);
+    s->stats = dbl(ostats);
+    s->fitbuf = dbl(ofit);
+    s->norm_part = dbl(onorm);
+    s->dinv = dbl(odinv);
+    s->colscale = dbl(ocs);
+    // the factors in one copy (converted, and laid out as on the device)
+    {
+        std::vector<char> stage;
+        try {
+            stage.resize(factor_bytes);
+        } catch (const std::bad_alloc&) {
+            return bad(fail(BLCO_ENOMEM, "host staging of the factors"));
+        }
+        for (int m = 0; m < N; ++m) to_dtype(U[m], stage.data() + oU[m], d->dims[m] * (uint64_t)R, s->ft);
+        if (hipMemcpy(s->arena, stage.data(), factor_bytes, hipMemcpyHostToDevice) != hipSuccess)
             return bad(fail(BLCO_EHIP, "factor upload failed"));
-        if (hipEventCreate(&s->ev0[m]) != hipSuccess || hipEventCreate(&s->ev1[m]) != hipSuccess ||
-            hipEventCreateWithFlags(&s->fork[m], hipEventDisableTiming) != hipSuccess ||
-            hipEventCreateWithFlags(&s->join[m], hipEventDisableTiming) != hipSuccess)
+    }
+    if (own_io) {
+        for (int m = 0; m < N; ++m)
+            if (hipEventCreate(&s->ev0[m]) != hipSuccess || hipEventCreate(&s->ev1[m]) != hipSuccess)
+                return bad(fail(BLCO_EHIP, "event creation failed"));
+        if (hipHostMalloc((void**)&s->h_fit, sizeof(double) * 4, hipHostMallocDefault) != hipSuccess)
+            return bad(fail(BLCO_ENOMEM, "pinned allocation failed"));
+        if (hipEventCreate(&s->it0) != hipSuccess || hipEventCreate(&s->it1) != hipSuccess)
             return bad(fail(BLCO_EHIP, "event creation failed"));
     }
-    if (hipStreamCreateWithFlags(&s->side, hipStreamNonBlocking) != hipSuccess)
-        return bad(fail(BLCO_EHIP, "stream creation failed"));
-    const int gparts = GRAM_MAX_PARTS;  // upper bound of gram_parts() for any row count
-    uint32_t sparts = solve_parts(maxI);
-    const int nnorm = 1024;
-    if (hipMalloc(&s->Mbuf, maxI * R * msz) != hipSuccess ||
-        hipMalloc((void**)&s->lambda, sizeof(double) * R) != hipSuccess ||
-        hipMalloc((void**)&s->inv, sizeof(double) * R) != hipSuccess ||
-        hipMalloc((void**)&s->fac, sizeof(double) * R * R) != hipSuccess ||
-        hipMalloc((void**)&s->work, sizeof(double) * (2 * R * R + R)) != hipSuccess ||
-        hipMalloc((void**)&s->status, sizeof(int)) != hipSuccess ||
-        hipMalloc((void**)&s->gram_part, sizeof(double) * (size_t)gparts * (R * R + R)) != hipSuccess ||
-        hipMalloc((void**)&s->stats, sizeof(double) * (size_t)(sparts ? sparts : 1) * R) != hipSuccess ||
-        hipMalloc((void**)&s->ip, sizeof(double) * R) != hipSuccess ||
-        hipMalloc((void**)&s->fitbuf, sizeof(double) * 4) != hipSuccess ||
-        hipMalloc((void**)&s->norm_part, sizeof(double) * (nnorm + 1)) != hipSuccess ||
-        hipMalloc((void**)&s->dinv, sizeof(double) * (size_t)N * R) != hipSuccess ||
-        hipMalloc((void**)&s->colscale, sizeof(double) * R) != hipSuccess)
-        return bad(fail(BLCO_ENOMEM, "solver work allocation failed"));
-    if (hipHostMalloc((void**)&s->h_fit, sizeof(double) * 4, hipHostMallocDefault) != hipSuccess)
-        return bad(fail(BLCO_ENOMEM, "pinned allocation failed"));
-    if (hipEventCreate(&s->it0) != hipSuccess || hipEventCreate(&s->it1) != hipSuccess)
-        return bad(fail(BLCO_EHIP, "event creation failed"));
+    // each mode's task; its successor in the sweep is the mode factored next
+    for (int k = 0; k < N; ++k) {
+        const int n = s->order[k];
+        AlsTask& t = s->tasks[n];
+        t.M = s->Mbuf;
+        t.U = s->U[n];
+        t.rows = d->dims[n];
+        t.fac = s->fac;
+        t.colscale = s->colscale;
+        t.work = s->work;
+        t.stats = s->stats;
+        t.part = s->part;
+        t.lambda = s->lambda;
+        t.dinv = s->dinv;
+        for (int m = 0; m < N; ++m) t.G[m] = s->G[m];
+        t.fit = s->fitbuf;
+        t.normX2 = s->norm_part + nnorm;
+        t.status = s->status;
+        t.nmodes = N;
+        t.mode = n;
+        t.next = s->order[(k + 1) % N];
+        t.last = k == N - 1;
+        t.parts = solve_gram_parts(t.rows);
+        t.first = 0;
+        s->upd[n] = AlsLaunch{reinterpret_cast<AlsTask*>(base + otask) + n, 1, t.parts, t.parts};
+    }
+    if (hipMemcpy(base + otask, s->tasks, sizeof(AlsTask) * N, hipMemcpyHostToDevice) != hipSuccess)
+        return bad(fail(BLCO_EHIP, "task upload failed"));
     // lambda = 1 (KruskalModelRandomInit), ||X||^2, initial Grams
     int rc = launch_fill(s->lambda, R, BLCO_F64, 1.0, s->st);
     if (!rc) rc = launch_fill(s->dinv, (uint64_t)N * R, BLCO_F64, 1.0, s->st);
@@ -254,9 +226,7 @@ int blco_cpals_create(blco_dev* d, const blco_cpals_opts* o, const double* const
     if (d->nnz && !d->stream_data) {
         rc = launch_sumsq(d->d_vals, d->vdtype, d->nnz, s->norm_part, nnorm, s->norm_part + nnorm, s->st);
         if (rc) return bad(rc);
-        if (hipMemcpyAsync(&s->normX2, s->norm_part + nnorm, sizeof(double), hipMemcpyDeviceToHost, s->st) != hipSuccess)
-            return bad(fail(BLCO_EHIP, "norm read-back failed"));
-    } else if (d->nnz) {
+    } else {
         // streamed tensors: the values are in pinned host memory
         double acc = 0.0;
         if (d->vdtype == BLCO_F64) {
@@ -266,15 +236,53 @@ int blco_cpals_create(blco_dev* d, const blco_cpals_opts* o, const double* const
             const float* v = (const float*)d->h_vals;
             for (uint64_t i = 0; i < d->nnz; ++i) acc += (double)v[i] * (double)v[i];
         }
-        s->normX2 = acc;
+        if (hipMemcpy(s->norm_part + nnorm, &acc, sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
+            return bad(fail(BLCO_EHIP, "norm upload failed"));
     }
     for (int m = 0; m < N && !rc; ++m)
-        rc = launch_gram(s->U[m], s->ft, d->dims[m], R, nullptr, s->gram_part, s->G[m], nullptr, s->st);
+        rc = launch_gram(s->U[m], s->ft, d->dims[m], R, nullptr, s->part, s->G[m], nullptr, s->st);
     if (rc) return bad(rc);
-    if (hipStreamSynchronize(s->st) != hipSuccess) return bad(fail(BLCO_EHIP, "setup failed"));
-    // build the chunk table outside any capture
-    if (!chunk_table(d, s->o.thread_cf > 0 ? s->o.thread_cf : 4)) return bad(BLCO_ENOMEM);
     *out = s;
+    return BLCO_OK;
+}
+
+static double now_ms()
+{
+    return std::chrono::duration<double, std::milli>(
+               std::chrono::steady_clock::now().time_since_epoch()).count();
+}
+
+}  // namespace blco
+
+extern "C" {
+
+void blco_cpals_free(blco_cpals_state* s)
+{
+    if (!s) return;
+    if (s->st) (void)hipStreamSynchronize(s->st);
+    if (s->gexec) (void)hipGraphExecDestroy(s->gexec);
+    if (s->graph) (void)hipGraphDestroy(s->graph);
+    for (int m = 0; m < BLCO_MAX_MODES; ++m) {
+        if (s->ev0[m]) (void)hipEventDestroy(s->ev0[m]);
+        if (s->ev1[m]) (void)hipEventDestroy(s->ev1[m]);
+    }
+    if (s->arena) (void)hipFree(s->arena);
+    if (s->h_fit) (void)hipHostFree(s->h_fit);
+    if (s->it0) (void)hipEventDestroy(s->it0);
+    if (s->it1) (void)hipEventDestroy(s->it1);
+    delete s;
+}
+
+int blco_cpals_create(blco_dev* d, const blco_cpals_opts* o, const double* const* U,
+                      blco_cpals_state** out)
+{
+    int rc = cpals_state_create(d, o, U, true, out);
+    if (rc) return rc;
+    if (hipStreamSynchronize((*out)->st) != hipSuccess) {
+        blco_cpals_free(*out);
+        *out = nullptr;
+        return fail(BLCO_EHIP, "setup failed");
+    }
     return BLCO_OK;
 }
 
@@ -295,8 +303,17 @@ int blco_cpals_iterate(blco_cpals_state* s, int n_iters, double* fits, int* done
                 int rc = mttkrp_prepare(s->d, s->order[k], s->R, s->ft, s->o.kernel);
                 if (rc) return rc;
             }
+            // F of the first mode; every update factors the next mode's
+            AlsLaunch l = s->upd[s->order[s->N - 1]];
+            const int rc = launch_als_begin(l, s->R, s->eps, s->st);
+            if (rc) return rc;
         }
         HIP_TRY(hipEventRecord(s->it0, s->st));
+        if (s->m_dirty) {
+            const int rc = launch_fill(s->Mbuf, s->m_bytes / (s->mt == BLCO_F64 ? 8 : 4), s->mt, 0.0, s->st);
+            if (rc) return rc;
+        }
+        s->m_dirty = true;  // until the sweep is through
         if (use_graph) {
             if (!s->gexec) {
                 HIP_TRY(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
@@ -316,6 +333,7 @@ int blco_cpals_iterate(blco_cpals_state* s, int n_iters, double* fits, int* done
         HIP_TRY(hipMemcpyAsync(s->h_fit, s->fitbuf, sizeof(double) * 3, hipMemcpyDeviceToHost, s->st));
         HIP_TRY(hipEventRecord(s->it1, s->st));
         HIP_TRY(hipStreamSynchronize(s->st));
+        s->m_dirty = false;
         float ms = 0.f;
         HIP_TRY(hipEventElapsedTime(&ms, s->it0, s->it1));
         s->iter_ms += ms;
@@ -346,19 +364,32 @@ int blco_cpals_get(blco_cpals_state* s, double* const* U, double* lambda)
 {
     if (!s) return fail(BLCO_EINVAL, "null solver");
     HIP_TRY(hipStreamSynchronize(s->st));
-    const int fsz = dtype_size(s->ft), R = s->R;
-    std::vector<char> stage;
-    std::vector<double> dinv((size_t)s->N * R);
-    HIP_TRY(hipMemcpy(dinv.data(), s->dinv, sizeof(double) * dinv.size(), hipMemcpyDeviceToHost));
+    const int R = s->R;
+    // the stored factor carries lambda_m in its columns: scaled (and widened)
+    // on the GPU into the MTTKRP buffer, piece by piece
+    const uint64_t piece = std::max<uint64_t>(1, s->m_bytes / (8 * (uint64_t)R));
     for (int m = 0; m < s->N; ++m) {
         if (!U || !U[m]) continue;
-        uint64_t n = s->d->dims[m] * (uint64_t)R;
-        stage.resize(n * fsz);
-        HIP_TRY(hipMemcpy(stage.data(), s->U[m], n * fsz, hipMemcpyDeviceToHost));
-        from_dtype(stage.data(), U[m], n, s->ft);
-        // the stored factor carries lambda_m in its columns
-        const double* iv = dinv.data() + (size_t)m * R;
-        for (uint64_t e = 0; e < n; ++e) U[m][e] *= iv[e % R];
+        if (s->m_bytes < 8 * (uint64_t)R) {  // one float row: no room for a row of doubles
+            double* t = nullptr;
+            HIP_TRY(hipMalloc((void**)&t, 8 * (uint64_t)R * s->d->dims[m]));
+            const int rc = launch_export(s->U[m], s->ft, s->d->dims[m], R, s->dinv + (size_t)m * R, t, s->st);
+            hipError_t e = hipStreamSynchronize(s->st);
+            if (e == hipSuccess) e = hipMemcpy(U[m], t, 8 * (uint64_t)R * s->d->dims[m], hipMemcpyDeviceToHost);
+            (void)hipFree(t);
+            if (rc) return rc;
+            HIP_TRY(e);
+            continue;
+        }
+        s->m_dirty = true;
+        for (uint64_t r = 0; r < s->d->dims[m]; r += piece) {
+            const uint64_t rows = std::min(piece, s->d->dims[m] - r);
+            const char* from = static_cast<const char*>(s->U[m]) + r * R * dtype_size(s->ft);
+            const int rc = launch_export(from, s->ft, rows, R, s->dinv + (size_t)m * R, (double*)s->Mbuf, s->st);
+            if (rc) return rc;
+            HIP_TRY(hipStreamSynchronize(s->st));
+            HIP_TRY(hipMemcpy(U[m] + r * R, s->Mbuf, rows * R * 8, hipMemcpyDeviceToHost));
+        }
     }
     if (lambda) HIP_TRY(hipMemcpy(lambda, s->lambda, sizeof(double) * s->R, hipMemcpyDeviceToHost));
     return BLCO_OK;

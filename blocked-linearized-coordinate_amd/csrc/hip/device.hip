@@ -14,6 +14,7 @@
 #include <unistd.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <new>
 #include <vector>
@@ -653,6 +654,8 @@ static int ensure_row_ordered(blco_dev* d, int mode, int rank, int ftype)
     d->sfiber[mode] = use_fibers;
     d->sgrp_h[mode].swap(groups);
     d->srun_h[mode].swap(runs);
+    static std::atomic<uint64_t> copies{0};
+    d->copy_id[mode] = ++copies;
     return BLCO_OK;
 }
 
@@ -670,10 +673,8 @@ static int ensure_row_ordered(blco_dev* d, int mode, int rank, int ftype)
 // of workgroups and the XCD-contiguous workgroup numbering puts tile t on XCD t.
 constexpr uint64_t LONG_ROW = 32768, LONG_PIECE = 2 * WAVE * SORTED_TPW;
 
-static const ChunkTab* sorted_chunk_table(blco_dev* d, int mode, int tpw)
+static std::vector<Chunk> sorted_chunks(const blco_dev* d, int mode, int tpw)
 {
-    for (auto& t : d->stabs[mode])
-        if (t.tpw == tpw) return &t;
     const uint64_t base = (uint64_t)WAVE * tpw, cap = 2 * base;
     const int ntiles = std::max(1, d->stiles[mode]);
     std::vector<std::vector<Chunk>> tiles(ntiles);
@@ -744,6 +745,14 @@ static const ChunkTab* sorted_chunk_table(blco_dev* d, int mode, int tpw)
             h.resize(h.size() + (most - tl.size()), Chunk{0, 0, 0});
         }
     }
+    return h;
+}
+
+static const ChunkTab* sorted_chunk_table(blco_dev* d, int mode, int tpw)
+{
+    for (auto& t : d->stabs[mode])
+        if (t.tpw == tpw) return &t;
+    const std::vector<Chunk> h = sorted_chunks(d, mode, tpw);
     ChunkTab t;
     t.tpw = tpw;
     t.n = (uint32_t)h.size();
@@ -912,6 +921,56 @@ int mttkrp_prepare(blco_dev* d, int mode, int rank, int ftype, int kernel)
     return rc;
 }
 
+// The input modes (on a copy that the fiber form runs on, the inner one
+// first), then the output mode.
+static void gather_order(const blco_dev* d, int mode, int* order)
+{
+    int j = 0;
+    const int inner = d->sfiber[mode] ? d->sinner[mode] : -1;
+    if (inner >= 0) order[j++] = inner;
+    for (int m = 0; m < d->nmodes; ++m)
+        if (m != mode && m != inner) order[j++] = m;
+    order[j] = mode;
+}
+
+// 32-bit row offsets (and byte offsets into the factors' buffer resources)
+// reach every factor.
+static bool narrow_factors(const blco_dev* d, int rank, int ftype)
+{
+    for (int m = 0; m < d->nmodes; ++m)
+        if (d->dims[m] * (uint64_t)rank * dtype_size(ftype) >= FACTOR_BYTES_MAX) return false;
+    return true;
+}
+
+int rows_batch_prepare(blco_dev* d, int mode, int rank, int ftype)
+{
+    if (!narrow_factors(d, rank, ftype)) return BLCO_EUNSUPPORTED;
+    return d->nnz ? ensure_row_ordered(d, mode, rank, ftype) : BLCO_OK;
+}
+
+std::vector<Chunk> rows_batch_chunks(const blco_dev* d, int mode, int tpw)
+{
+    return d->nnz ? sorted_chunks(d, mode, tpw) : std::vector<Chunk>();
+}
+
+MttkrpArgs rows_batch_args(const blco_dev* d, int mode, int rank)
+{
+    MttkrpArgs a;
+    std::memset(&a, 0, sizeof a);
+    a.coords = d->d_scoords[mode];
+    a.vals = d->d_svals[mode];
+    a.bcoords = d->d_bcoords;
+    for (int m = 0; m < d->nmodes; ++m) {
+        a.mask[m] = d->masks[m];
+        a.pos[m] = d->pos[m];
+    }
+    a.nmodes = d->nmodes;
+    a.mode = mode;
+    a.rank = rank;
+    gather_order(d, mode, a.order);
+    return a;
+}
+
 int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, void* out, int kernel,
            int nprtn, int tpw, hipStream_t st, int* used_kernel)
 {
@@ -984,8 +1043,8 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
             return rc;
         }
     }
-    const ChunkTab* t = chunk_table(d, tpw);
-    if (!t) return BLCO_ENOMEM;
+    const ChunkTab* t = nullptr;  // kernels 14 and 12 have tables of their own
+    if (which != W_ROWS && which != W_WINDOW && !(t = chunk_table(d, tpw))) return BLCO_ENOMEM;
 
     MttkrpArgs a;
     std::memset(&a, 0, sizeof a);
@@ -1109,11 +1168,7 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
         a.coord_base = 0;
         const ChunkTab* stab = sorted_chunk_table(d, mode, tpw);
         if (!stab) return BLCO_ENOMEM;
-        // 32-bit row offsets (and byte offsets into the factors' buffer
-        // resources) when every factor holds fewer than FACTOR_BYTES_MAX bytes
-        bool wide = false;
-        for (int m = 0; m < d->nmodes; ++m)
-            wide |= d->dims[m] * (uint64_t)rank * dtype_size(ftype) >= FACTOR_BYTES_MAX;
+        const bool wide = !narrow_factors(d, rank, ftype);
         const bool fib = d->sfiber[mode];
         if (fib) a.inner = d->sinner[mode];
         if (wide) {
@@ -1127,11 +1182,7 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
             int kind = fib ? W_FIBER_LDS : W_SORTED_LDS;
             if (!lds) {
                 kind = tpw >= ROWS_LONG_TPW ? W_ROWS : W_ROWS_SHORT;
-                int j = 0;
-                if (fib) a.order[j++] = a.inner;
-                for (int m = 0; m < d->nmodes; ++m)
-                    if (m != mode && !(fib && m == a.inner)) a.order[j++] = m;
-                a.order[j] = mode;
+                gather_order(d, mode, a.order);
             }
             const uint32_t per_wg = WAVES_PER_WG * a.cpw;
             rc = launch_mttkrp(kind, a, ftype, (stab->n + per_wg - 1) / per_wg, lds, st);
@@ -1871,24 +1922,20 @@ int blco_solve(double* const* grams, int nmodes, int mode, int rank, const void*
     hipStream_t st = (hipStream_t)stream;
     GramSet gs;
     for (int m = 0; m < nmodes; ++m) gs.g[m] = grams[m];
-    double *fac = nullptr, *work = nullptr, *stats = nullptr;
+    double* fac = nullptr;
     int* status = nullptr;
-    uint32_t np = solve_parts(rows);
+    const size_t r2 = (size_t)rank * rank;
     auto release = [&]() {
         if (fac) (void)hipFree(fac);
-        if (work) (void)hipFree(work);
-        if (status) (void)hipFree(status);
-        if (stats) (void)hipFree(stats);
     };
-    if (hipMalloc(&fac, sizeof(double) * rank * rank) != hipSuccess ||
-        hipMalloc(&work, sizeof(double) * (2 * rank * rank + rank)) != hipSuccess ||
-        hipMalloc(&status, sizeof(int)) != hipSuccess ||
-        hipMalloc(&stats, sizeof(double) * (size_t)(np ? np : 1) * rank) != hipSuccess) {
+    // F, the fallback's 2 R^2 + R doubles, the status
+    if (hipMalloc(&fac, sizeof(double) * (3 * r2 + rank + 1)) != hipSuccess) {
         release();
         return fail(BLCO_ENOMEM, "solve work allocation failed");
     }
-    int rc = launch_factorize(gs, nmodes, mode, rank, gram_eps(BLCO_F64), fac, work, status, st);
-    if (!rc) rc = launch_solve_rows(M, U, dtype, rows, rank, fac, 0, stats, st);
+    status = reinterpret_cast<int*>(fac + 3 * r2 + rank);
+    int rc = launch_factorize(gs, nmodes, mode, rank, gram_eps(BLCO_F64), fac, fac + r2, status, st);
+    if (!rc) rc = launch_solve_rows(M, U, dtype, rows, rank, fac, st);
     int h_status = 0;
     hipError_t e = hipMemcpyAsync(&h_status, status, sizeof(int), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);

@@ -104,6 +104,7 @@ struct blco_dev {
     uint64_t* d_scoords[BLCO_MAX_MODES] = {};
     void* d_svals[BLCO_MAX_MODES] = {};
     bool sorted_failed[BLCO_MAX_MODES] = {};  // no device memory for the copy
+    uint64_t copy_id[BLCO_MAX_MODES] = {};    // of the copy, unlike any other copy's
     // groups of the copy in storage order (tile-major), the number of tiles
     // (1: untiled) and the positions where a run of equal (group, row)
     // starts, then nnz
@@ -169,6 +170,12 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
 // kernel) would do on its first call (kernel 14's row-ordered copy), without
 // a launch; a copy that does not fit leaves the mode to the row window.
 int mttkrp_prepare(blco_dev* d, int mode, int rank, int ftype, int kernel);
+// Kernel 14 over many tensors in one launch (k_mttkrp_rows_batch): builds the
+// copy (BLCO_EUNSUPPORTED for factors that need 64-bit offsets), its chunks,
+// and the kernel arguments without factors and output.
+int rows_batch_prepare(blco_dev* d, int mode, int rank, int ftype);
+std::vector<Chunk> rows_batch_chunks(const blco_dev* d, int mode, int tpw);
+MttkrpArgs rows_batch_args(const blco_dev* d, int mode, int rank);
 size_t rows_kernel_plan(blco_dev* d, int mode, int rank, int ftype, bool fib, MttkrpArgs* a);
 
 }  // namespace blco

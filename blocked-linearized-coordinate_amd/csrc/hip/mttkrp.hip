@@ -115,7 +115,7 @@ __global__ __launch_bounds__(WG) void k_fill(T* __restrict__ x, uint64_t n, T v)
 
 const void* mttkrp_kernel(int which, int nmodes, int ftype, int rank, int* C, int* L)
 {
-    const bool rows = which == W_ROWS || which == W_ROWS_SHORT;
+    const bool rows = which == W_ROWS || which == W_ROWS_SHORT || which == W_ROWS_BATCH;
     const Shape s = rows ? rows_shape(rank, dtype_size(ftype)) : pick_shape(rank, dtype_size(ftype));
     *C = s.C;
     *L = s.L;

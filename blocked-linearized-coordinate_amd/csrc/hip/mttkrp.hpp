@@ -25,6 +25,15 @@ struct SuperChunk {
     uint32_t block;
 };
 
+// A chunk of a tensor of a batch (an index into the launch's tensors).
+struct BatchChunk {
+    uint64_t begin;
+    uint32_t len;
+    uint32_t block;
+    uint32_t tensor;
+    uint32_t pad;
+};
+
 struct MttkrpArgs {
     const uint64_t* coords;  // element e lives at coords[e - coord_base]
     const void* vals;        // same indexing, f64 or f32
@@ -78,7 +87,7 @@ struct RowsPlan {
 };
 
 enum { W_LVL1 = 0, W_LVL3 = 1, W_ATOMIC = 2, W_WINDOW = 3, W_WINDOW64 = 4, W_SORTED64 = 5, W_FIBER64 = 6,
-       W_SORTED_LDS = 7, W_FIBER_LDS = 8, W_ROWS = 9, W_ROWS_SHORT = 10 };
+       W_SORTED_LDS = 7, W_FIBER_LDS = 8, W_ROWS = 9, W_ROWS_SHORT = 10, W_ROWS_BATCH = 11 };
 
 // The row-ordered and fiber kernels take 31-bit byte offsets into factors
 // of fewer bytes than this (bit 31 marks an offset into an LDS window).

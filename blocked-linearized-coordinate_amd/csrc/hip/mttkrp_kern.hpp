@@ -909,7 +909,8 @@ __device__ __forceinline__ void load_run(const T* p, T (&x)[Q])
 // 1206 / 1207 us; 10M nonzeros with BF16 factors 306 / 313 / 413 -> 110 / 118
 // / 109 us; 3.3M nonzeros at FP64 rank 10 117 -> 52 us.
 template <int N, typename FT, typename VT, int C, int L, int Q>
-__global__ __launch_bounds__(WG) void k_mttkrp_rows(MttkrpArgs a)
+__device__ __forceinline__ void rows_chunk(const MttkrpArgs& a, const Chunk& ch,
+                                           typename Acc<FT>::type (*s_stage)[C * L], uint32_t* s_row)
 {
     using AT = typename Acc<FT>::type;
     static_assert(C * L <= WAVE, "a staged row is added by at most one wave");
@@ -920,16 +921,9 @@ __global__ __launch_bounds__(WG) void k_mttkrp_rows(MttkrpArgs a)
     constexpr int PB = ROW_REGS <= 8 ? 4 : ROW_REGS <= 16 ? 2 : 1;
     constexpr int KS = PB < Q ? PB : Q;     // of one lane
     constexpr int LS = PB / KS;             // of consecutive lanes
-    constexpr int CAP = 2 * S;              // staged rows
     constexpr uint32_t NONE = 0x80000000u;  // past every factor: gathers zeros
-    __shared__ AT s_stage[WAVES_PER_WG][CAP][C * L];
-    __shared__ uint32_t s_row[WAVES_PER_WG][CAP];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const uint32_t c = (uint32_t)__builtin_amdgcn_readfirstlane(
-        (int)(xcd_remap(blockIdx.x, gridDim.x) * WAVES_PER_WG + w));
-    if (c >= a.nchunks) return;  // whole wave leaves; no block barriers below
-    const Chunk ch = a.chunks[a.chunk0 + c];
     if (ch.len == 0) return;
+    const int lane = threadIdx.x & 63;
     const int R = a.rank;
     const uint32_t row_bytes = (uint32_t)R * (uint32_t)sizeof(FT);
     // in the order of a.order: the input modes, then the output mode
@@ -967,7 +961,7 @@ __global__ __launch_bounds__(WG) void k_mttkrp_rows(MttkrpArgs a)
             for (int i = 0; i < staged; i += WAVE >> gsh) {
                 const int r = i + (lane >> gsh), col = lane & ((1 << gsh) - 1);
                 if (r < staged && col < width)
-                    atomic_add_global(out + (uint64_t)s_row[w][r] * R + cb + col, s_stage[w][r][col]);
+                    atomic_add_global(out + (uint64_t)s_row[r] * R + cb + col, s_stage[r][col]);
             }
             wave_lds_sync();
             staged = 0;
@@ -979,8 +973,8 @@ __global__ __launch_bounds__(WG) void k_mttkrp_rows(MttkrpArgs a)
                 const int at = staged + (int)__popcll(lanes & below_slots) / L;
                 #pragma unroll
                 for (int cc = 0; cc < C; ++cc)
-                    if (c0 + cc >= 0) s_stage[w][at][c0 + cc] = acc[cc];
-                if (sub == 0) s_row[w][at] = cur;
+                    if (c0 + cc >= 0) s_stage[at][c0 + cc] = acc[cc];
+                if (sub == 0) s_row[at] = cur;
             }
             staged += (int)__popcll(lanes) / L;
         };
@@ -1148,6 +1142,38 @@ __global__ __launch_bounds__(WG) void k_mttkrp_rows(MttkrpArgs a)
         stage((1ull << L) - 1);  // slot 0
         add_staged();
     }
+}
+
+template <int N, typename FT, typename VT, int C, int L, int Q>
+__global__ __launch_bounds__(WG) void k_mttkrp_rows(MttkrpArgs a)
+{
+    constexpr int CAP = 2 * (WAVE / L);  // staged rows
+    __shared__ typename Acc<FT>::type s_stage[WAVES_PER_WG][CAP][C * L];
+    __shared__ uint32_t s_row[WAVES_PER_WG][CAP];
+    const int w = threadIdx.x >> 6;
+    const uint32_t c = (uint32_t)__builtin_amdgcn_readfirstlane(
+        (int)(xcd_remap(blockIdx.x, gridDim.x) * WAVES_PER_WG + w));
+    if (c >= a.nchunks) return;  // whole wave leaves; no block barriers below
+    const Chunk ch = a.chunks[a.chunk0 + c];
+    rows_chunk<N, FT, VT, C, L, Q>(a, ch, s_stage[w], s_row[w]);
+}
+
+// The same over the chunks of many tensors of one order: chunk c belongs to
+// tensor chunks[c].tensor, whose arguments are tens[.].
+template <int N, typename FT, typename VT, int C, int L, int Q>
+__global__ __launch_bounds__(WG) void k_mttkrp_rows_batch(const MttkrpArgs* __restrict__ tens,
+                                                          const BatchChunk* __restrict__ chunks, uint32_t nchunks)
+{
+    constexpr int CAP = 2 * (WAVE / L);
+    __shared__ typename Acc<FT>::type s_stage[WAVES_PER_WG][CAP][C * L];
+    __shared__ uint32_t s_row[WAVES_PER_WG][CAP];
+    const int w = threadIdx.x >> 6;
+    const uint32_t c = (uint32_t)__builtin_amdgcn_readfirstlane(
+        (int)(xcd_remap(blockIdx.x, gridDim.x) * WAVES_PER_WG + w));
+    if (c >= nchunks) return;
+    const BatchChunk bc = chunks[c];
+    const MttkrpArgs& a = tens[__builtin_amdgcn_readfirstlane((int)bc.tensor)];
+    rows_chunk<N, FT, VT, C, L, Q>(a, Chunk{bc.begin, bc.len, bc.block}, s_stage[w], s_row[w]);
 }
 
 // MTTKRP over a row-ordered copy with the hot rows of two input modes in LDS
@@ -1545,6 +1571,7 @@ inline Shape rows_shape(int rank, int esize)
 template <int N, typename FT, typename VT, int C, int L>
 inline const void* rows_ptr(int which)
 {
+    if (which == W_ROWS_BATCH) return (const void*)&k_mttkrp_rows_batch<N, FT, VT, C, L, L == 16 ? 1 : 2>;
     // short runs take rounds of fewer positions
     if (which == W_ROWS_SHORT) return (const void*)&k_mttkrp_rows<N, FT, VT, C, L, L == 16 ? 1 : 2>;
     return (const void*)&k_mttkrp_rows<N, FT, VT, C, L, L == 16 ? 2 : 4>;
@@ -1575,7 +1602,7 @@ inline const void* select_rows(const Shape& s, int which)
 template <int N, typename FT, typename VT>
 inline const void* select_shape(const Shape& s, int which)
 {
-    if (which == W_ROWS || which == W_ROWS_SHORT) return select_rows<N, FT, VT>(s, which);
+    if (which == W_ROWS || which == W_ROWS_SHORT || which == W_ROWS_BATCH) return select_rows<N, FT, VT>(s, which);
     if (s.exact) {
         if (s.C == 1 && s.L == 8) return kernel_ptr<N, FT, VT, 1, 8, true>(which);
         if (s.C == 2 && s.L == 8) return kernel_ptr<N, FT, VT, 2, 8, true>(which);

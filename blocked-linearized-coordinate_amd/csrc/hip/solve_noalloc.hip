@@ -2,16 +2,14 @@
 // without any device allocation, for callers that cannot allocate (code
 // under HIP graph capture, tight serving loops, harnesses that forbid
 // hipMalloc).  It runs the kernels of blco_solve; their scratch (the R x R
-// factor, the Jacobi work area, the status flag and the per-workgroup column
-// statistics) lives in one file-scope device array instead of per-call
-// allocations.
+// factor, the Jacobi work area and the status flag) lives in one file-scope
+// device array instead of per-call allocations.
 //
 // The array exists once per GPU the library runs on and is held until the
 // process ends.  Every call on a GPU uses that GPU's copy, so calls that
 // overlap on one GPU (two streams, two host threads) race on it; callers
 // serialise them.  Nothing in the scratch has to start at zero: the
-// factorisation writes the status flag and the factor on both of its paths,
-// and the row solve writes every workgroup's statistics slot.
+// factorisation writes the status flag and the factor on both of its paths.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -24,8 +22,9 @@ namespace blco {
 namespace {
 
 constexpr int NOALLOC_MAX_RANK = 64;
-// fac (R^2) + Jacobi work (2 R^2 + R) + column statistics (at most
-// 2048 workgroups x R) in doubles, then the status flag
+// fac (R^2) + Jacobi work (2 R^2 + R) + 2048 R doubles, then the status flag.
+// The 2048 R are unused; they keep the size that
+// blco_solve_noalloc_scratch_bytes has always reported.
 constexpr size_t NOALLOC_FAC = (size_t)NOALLOC_MAX_RANK * NOALLOC_MAX_RANK;
 constexpr size_t NOALLOC_WORK = 2 * NOALLOC_FAC + NOALLOC_MAX_RANK;
 constexpr size_t NOALLOC_STATS = 2048 * (size_t)NOALLOC_MAX_RANK;
@@ -83,21 +82,17 @@ extern "C" int blco_solve_noalloc(double* const* grams, int nmodes, int mode, in
         return fail(BLCO_EUNSUPPORTED, "rank %d outside [1, %d]: the allocation-free solve's scratch holds "
                     "%llu bytes", rank, NOALLOC_MAX_RANK, (unsigned long long)NOALLOC_BYTES);
     if (dtype < BLCO_F64 || dtype > BLCO_BF16) return fail(BLCO_EINVAL, "factor dtype %d", dtype);
-    const uint32_t np = solve_parts(rows);
-    if ((size_t)np * rank > NOALLOC_STATS)
-        return fail(BLCO_EUNSUPPORTED, "%u row-solve workgroups exceed the scratch", np);
     void* base = nullptr;
     int rc = scratch_ptr(&base);
     if (rc) return rc;
     double* fac = static_cast<double*>(base);
     double* work = fac + (size_t)rank * rank;
-    double* stats = work + 2 * (size_t)rank * rank + rank;
     int* status = reinterpret_cast<int*>(static_cast<double*>(base) + NOALLOC_DOUBLES);
     hipStream_t st = (hipStream_t)stream;
     GramSet gs;
     for (int m = 0; m < nmodes; ++m) gs.g[m] = grams[m];
     rc = launch_factorize(gs, nmodes, mode, rank, gram_eps(BLCO_F64), fac, work, status, st);
-    if (!rc) rc = launch_solve_rows(M, U, dtype, rows, rank, fac, 0, stats, st);
+    if (!rc) rc = launch_solve_rows(M, U, dtype, rows, rank, fac, st);
     if (rc) return rc;
     if (used_fallback) {
         int h_status = 0;
