@@ -70,34 +70,49 @@ __global__ __launch_bounds__(WG) void k_gram(const UT* __restrict__ U, uint64_t 
     double ip[T];
     #pragma unroll
     for (int t = 0; t < T; ++t) ip[t] = 0.0;
-    for (uint64_t r0 = rb + (uint64_t)w * 4; r0 < re; r0 += WAVES_PER_WG * 4) {
-        const uint64_t row = r0 + k4;
-        AT a[T];
+    // UN row steps' loads are issued together (their MFMAs in row order): 1.8M
+    // rows at rank 32, FP32, 100 us with one step's loads at a time
+    constexpr int UN = 4;
+    for (uint64_t r0 = rb + (uint64_t)w * 4; r0 < re; r0 += UN * WAVES_PER_WG * 4) {
+        AT a[UN][T];
         #pragma unroll
-        for (int t = 0; t < T; ++t) {
-            const int col = t * 16 + i16;
-            AT x = 0;
-            if (row < re && col < R) {
-                x = (AT)as_f64(U[row * (uint64_t)R + col]);
-                if (M) {
-                    double mv = F64 ? reinterpret_cast<const double*>(M)[row * (uint64_t)R + col]
-                                    : (double)reinterpret_cast<const float*>(M)[row * (uint64_t)R + col];
-                    ip[t] += (double)x * mv;
+        for (int u = 0; u < UN; ++u) {
+            const uint64_t row = r0 + (uint64_t)u * WAVES_PER_WG * 4 + k4;
+            #pragma unroll
+            for (int t = 0; t < T; ++t) {
+                const int col = t * 16 + i16;
+                a[u][t] = (row < re && col < R) ? (AT)as_f64(U[row * (uint64_t)R + col]) : (AT)0;
+            }
+        }
+        if (M) {
+            #pragma unroll
+            for (int u = 0; u < UN; ++u) {
+                const uint64_t row = r0 + (uint64_t)u * WAVES_PER_WG * 4 + k4;
+                #pragma unroll
+                for (int t = 0; t < T; ++t) {
+                    const int col = t * 16 + i16;
+                    if (row < re && col < R) {
+                        const double mv = F64 ? reinterpret_cast<const double*>(M)[row * (uint64_t)R + col]
+                                              : (double)reinterpret_cast<const float*>(M)[row * (uint64_t)R + col];
+                        ip[t] += (double)a[u][t] * mv;
+                    }
                 }
             }
-            a[t] = x;
         }
-        int q = 0;
         #pragma unroll
-        for (int ti = 0; ti < T; ++ti)
+        for (int u = 0; u < UN; ++u) {
+            int q = 0;
             #pragma unroll
-            for (int tj = ti; tj < T; ++tj) {
-                if constexpr (F64)
-                    acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ti], a[tj], acc[q], 0, 0, 0);
-                else
-                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[ti], a[tj], acc[q], 0, 0, 0);
-                ++q;
-            }
+            for (int ti = 0; ti < T; ++ti)
+                #pragma unroll
+                for (int tj = ti; tj < T; ++tj) {
+                    if constexpr (F64)
+                        acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][ti], a[u][tj], acc[q], 0, 0, 0);
+                    else
+                        acc[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][ti], a[u][tj], acc[q], 0, 0, 0);
+                    ++q;
+                }
+        }
     }
     // combine the 4 waves in LDS, then write this workgroup's partial
     __shared__ double s_g[WAVES_PER_WG][T * 16][T * 16 + 1];
@@ -950,21 +965,45 @@ __global__ __launch_bounds__(WG) void k_hadamard(double* __restrict__ x, const d
 }
 
 // Per-workgroup column statistics of an existing factor (which 0: sum of
-// squares, 1: max seeded with 1), for the stand-alone column norm.
+// squares, 1: max seeded with 1), for the stand-alone column norm.  A
+// workgroup reads WG / R rows at a time, thread t the t-th element of them,
+// eight such loads in flight; bound by HBM (1.8M rows at rank 32, FP32: 700
+// us with one column's lane walking the rows alone).
 template <typename UT>
 __global__ __launch_bounds__(WG) void k_colstats(const UT* __restrict__ U, uint64_t rows, int R,
                                                  uint64_t rows_per_wg, int which,
                                                  double* __restrict__ stats)
 {
+    __shared__ double s_st[WG];
     const uint64_t rb = (uint64_t)blockIdx.x * rows_per_wg;
     const uint64_t re = min(rb + rows_per_wg, rows);
-    for (int c = threadIdx.x; c < R; c += WG) {
-        double x = (which == 0) ? 0.0 : 1.0;
-        for (uint64_t i = rb; i < re; ++i) {
-            double v = as_f64(U[i * (uint64_t)R + c]);
-            x = (which == 0) ? x + v * v : fmax(x, v);
+    const double seed = which == 0 ? 0.0 : 1.0;
+    for (int c0 = 0; c0 < R; c0 += WG) {  // one pass for R <= WG
+        const int width = min(R - c0, WG), groups = WG / width;
+        const int t = threadIdx.x, c = t % width, g = t / width;
+        double x = seed;
+        if (g < groups) {
+            uint64_t i = rb + g;
+            const uint64_t step = groups;
+            for (; i + 7 * step < re; i += 8 * step) {
+                double v[8];
+                #pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] = as_f64(U[(i + u * step) * (uint64_t)R + c0 + c]);
+                #pragma unroll
+                for (int u = 0; u < 8; ++u) x = (which == 0) ? x + v[u] * v[u] : fmax(x, v[u]);
+            }
+            for (; i < re; i += step) {
+                const double v = as_f64(U[i * (uint64_t)R + c0 + c]);
+                x = (which == 0) ? x + v * v : fmax(x, v);
+            }
         }
-        stats[(uint64_t)blockIdx.x * R + c] = x;
+        s_st[t] = x;
+        __syncthreads();
+        if (t < width) {
+            for (int q = 1; q < groups; ++q) x = which == 0 ? x + s_st[q * width + t] : fmax(x, s_st[q * width + t]);
+            stats[(uint64_t)blockIdx.x * R + c0 + t] = x;
+        }
+        __syncthreads();
     }
 }
 

@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <vector>
 
@@ -1819,6 +1820,7 @@ void blco_dev_free(blco_dev* d)
     if (d->copy_stream) (void)hipStreamDestroy(d->copy_stream);
     if (d->stream) (void)hipStreamDestroy(d->stream);
     delete d;
+    Workspace::release_all();
 }
 
 uint64_t blco_dev_bytes(const blco_dev* d) { return d ? d->bytes : 0; }
@@ -1885,10 +1887,10 @@ int blco_gram(const void* U, int dtype, uint64_t rows, int rank, double* G, void
     uint64_t rpw;
     gram_parts(rows, &nparts, &rpw);
     double* part = nullptr;
-    HIP_TRY(hipMalloc(&part, sizeof(double) * (size_t)nparts * (rank * rank + rank)));
-    int rc = launch_gram(U, dtype, rows, rank, nullptr, part, G, nullptr, st);
+    Workspace ws;
+    int rc = ws.get(sizeof(double) * (size_t)nparts * (rank * rank + rank), &part);
+    if (!rc) rc = launch_gram(U, dtype, rows, rank, nullptr, part, G, nullptr, st);
     hipError_t e = hipStreamSynchronize(st);
-    (void)hipFree(part);
     if (rc) return rc;
     HIP_TRY(e);
     return BLCO_OK;
@@ -1925,21 +1927,16 @@ int blco_solve(double* const* grams, int nmodes, int mode, int rank, const void*
     double* fac = nullptr;
     int* status = nullptr;
     const size_t r2 = (size_t)rank * rank;
-    auto release = [&]() {
-        if (fac) (void)hipFree(fac);
-    };
     // F, the fallback's 2 R^2 + R doubles, the status
-    if (hipMalloc(&fac, sizeof(double) * (3 * r2 + rank + 1)) != hipSuccess) {
-        release();
-        return fail(BLCO_ENOMEM, "solve work allocation failed");
-    }
+    Workspace ws;
+    int rc = ws.get(sizeof(double) * (3 * r2 + rank + 1), &fac);
+    if (rc) return rc;
     status = reinterpret_cast<int*>(fac + 3 * r2 + rank);
-    int rc = launch_factorize(gs, nmodes, mode, rank, gram_eps(BLCO_F64), fac, fac + r2, status, st);
+    rc = launch_factorize(gs, nmodes, mode, rank, gram_eps(BLCO_F64), fac, fac + r2, status, st);
     if (!rc) rc = launch_solve_rows(M, U, dtype, rows, rank, fac, st);
     int h_status = 0;
     hipError_t e = hipMemcpyAsync(&h_status, status, sizeof(int), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
-    release();
     if (rc) return rc;
     HIP_TRY(e);
     if (used_fallback) *used_fallback = h_status;
@@ -1964,14 +1961,15 @@ int blco_colnorm(void* U, int dtype, uint64_t rows, int rank, int which, double*
     hipStream_t st = (hipStream_t)stream;
     int np = (int)std::min<uint64_t>((rows + 1023) / 1024, 1024);
     if (np < 1) np = 1;
-    double *stats = nullptr, *inv = nullptr;
-    HIP_TRY(hipMalloc(&stats, sizeof(double) * (size_t)np * rank));
-    HIP_TRY(hipMalloc(&inv, sizeof(double) * rank));
-    int rc = launch_colstats(U, dtype, rows, rank, which, stats, np, st);
+    double* stats = nullptr;
+    Workspace ws;
+    int rc = ws.get(sizeof(double) * ((size_t)np + 1) * rank, &stats);
+    if (rc) return rc;
+    double* inv = stats + (size_t)np * rank;
+    rc = launch_colstats(U, dtype, rows, rank, which, stats, np, st);
     if (!rc) rc = launch_lambda(stats, np, rank, which, lambda, inv, st);
     if (!rc) rc = launch_scale(U, dtype, rows, rank, inv, st);
     hipError_t e = hipStreamSynchronize(st);
-    (void)hipFree(stats); (void)hipFree(inv);
     if (rc) return rc;
     HIP_TRY(e);
     return BLCO_OK;
@@ -1989,17 +1987,17 @@ int blco_fit(double* const* grams, int nmodes, int rank, const double* lambda, c
     int nparts;
     uint64_t rpw;
     gram_parts(rows, &nparts, &rpw);
-    double *part = nullptr, *G = nullptr, *ip = nullptr, *out = nullptr;
-    HIP_TRY(hipMalloc(&part, sizeof(double) * (size_t)nparts * (rank * rank + rank)));
-    HIP_TRY(hipMalloc(&G, sizeof(double) * rank * rank));
-    HIP_TRY(hipMalloc(&ip, sizeof(double) * rank));
-    HIP_TRY(hipMalloc(&out, sizeof(double) * 4));
-    int rc = launch_gram(U_last, dtype, rows, rank, M_last, part, G, ip, st);
+    double* part = nullptr;
+    Workspace ws;
+    const size_t w = (size_t)rank * rank + rank;
+    int rc = ws.get(sizeof(double) * ((size_t)nparts * w + w + 4), &part);
+    if (rc) return rc;
+    double *G = part + (size_t)nparts * w, *ip = G + (size_t)rank * rank, *out = ip + rank;
+    rc = launch_gram(U_last, dtype, rows, rank, M_last, part, G, ip, st);
     if (!rc) rc = launch_fit(gs, nmodes, rank, lambda, ip, normX2, out, st);
     double h[3] = {0, 0, 0};
     hipError_t e = hipMemcpyAsync(h, out, sizeof(double) * 3, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
-    (void)hipFree(part); (void)hipFree(G); (void)hipFree(ip); (void)hipFree(out);
     if (rc) return rc;
     HIP_TRY(e);
     *fit = h[0];
