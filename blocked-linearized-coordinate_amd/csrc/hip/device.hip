@@ -37,7 +37,7 @@ constexpr int DEFAULT_TPW = 4;                // tiles of 64 per wave
 constexpr int SORTED_TPW = 16;                // tiles of 64 per wave, row-ordered kernel (most)
 constexpr int ROWS_LONG_TPW = 8;              // chunks from here on take k_mttkrp_rows' long rounds
 constexpr int DEFAULT_NPRTN = 1;
-constexpr uint32_t LVL3_CHUNKS_PER_WG = 64;
+constexpr uint32_t LVL3_CHUNKS_PER_WG = 64;  // at most
 constexpr uint32_t HOT_EXCLUDE = 64;  // hot rows kept out of the row windows
 
 static int value_size(int vdt) { return vdt == BLCO_F64 ? 8 : 4; }
@@ -784,9 +784,10 @@ static int launch_range(blco_dev* d, int which, MttkrpArgs a, const ChunkTab* t,
     a.nchunks = c1 - c0;
     uint32_t grid;
     size_t lds = 0;
-    if (which == W_LVL3) {
-        a.chunks_per_wg = LVL3_CHUNKS_PER_WG;
-        grid = (a.nchunks + LVL3_CHUNKS_PER_WG - 1) / LVL3_CHUNKS_PER_WG;
+    if (which == W_LVL3 || which == W_LVL3_ROWS) {
+        // about 1024 workgroups, of at least one chunk a wave
+        a.chunks_per_wg = std::min(LVL3_CHUNKS_PER_WG, std::max<uint32_t>(WAVES_PER_WG, a.nchunks / 1024));
+        grid = (a.nchunks + a.chunks_per_wg - 1) / a.chunks_per_wg;
         lds = d->dims[a.mode] * (uint64_t)a.rank * (ftype == BLCO_F64 ? 8 : 4);
     } else {
         grid = (a.nchunks + WAVES_PER_WG - 1) / WAVES_PER_WG;
@@ -1063,7 +1064,15 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
     a.nprtn = which == W_LVL3 ? nprtn : 1;
     const int otype = ftype == BLCO_F64 ? BLCO_F64 : BLCO_F32;
     const uint64_t cells = d->dims[mode] * (uint64_t)rank;
-    if (which == W_LVL3 && nprtn > 1) {
+    const bool lvl3 = which == W_LVL3;
+    if (lvl3 && narrow_factors(d, rank, ftype)) {
+        which = W_LVL3_ROWS;
+        int j = 0;
+        for (int m = 0; m < d->nmodes; ++m)
+            if (m != mode) a.order[j++] = m;
+        a.order[j] = mode;
+    }
+    if (lvl3 && nprtn > 1) {
         size_t bytes = (size_t)nprtn * cells * (otype == BLCO_F64 ? 8 : 4);
         int rc = ensure_partials(d, bytes);
         if (rc) return rc;
@@ -1228,10 +1237,83 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
         }
     }
     if (rc) return rc;
-    if (which == W_LVL3 && nprtn > 1)
+    if (lvl3 && nprtn > 1)
         rc = launch_reduce_partials(out, d->partials, cells, nprtn, otype, st);
     return rc;
 }
+
+// Device scratch of the stand-alone ALS-step calls.  Each of them waits for
+// its stream before it returns, so a released buffer is idle; it is kept for
+// the next call on that GPU (an allocation and its free cost a call about 60
+// us) unless the kept ones would exceed KEPT_MAX bytes, and all idle ones are
+// freed with any device tensor (release_all).
+class Workspace {
+public:
+    ~Workspace()
+    {
+        if (!p_) return;
+        std::lock_guard<std::mutex> lk(mu());
+        if (kept() + n_ <= KEPT_MAX) idle().push_back({dev_, n_, p_});
+        else (void)hipFree(p_);
+    }
+    int get(size_t bytes, double** out)
+    {
+        HIP_TRY(hipGetDevice(&dev_));
+        {
+            std::lock_guard<std::mutex> lk(mu());
+            auto& v = idle();
+            for (size_t i = 0; i < v.size(); ++i)
+                if (v[i].dev == dev_ && v[i].n >= bytes) {
+                    p_ = v[i].p;
+                    n_ = v[i].n;
+                    v.erase(v.begin() + i);
+                    break;
+                }
+        }
+        if (!p_) {
+            n_ = (bytes + (1 << 20) - 1) >> 20 << 20;
+            if (hipMalloc(&p_, n_) != hipSuccess) {
+                p_ = nullptr;
+                return fail(BLCO_ENOMEM, "device scratch of %llu bytes", (unsigned long long)n_);
+            }
+        }
+        *out = static_cast<double*>(p_);
+        return BLCO_OK;
+    }
+    static void release_all()
+    {
+        std::lock_guard<std::mutex> lk(mu());
+        for (auto& b : idle()) (void)hipFree(b.p);
+        idle().clear();
+    }
+
+private:
+    struct Idle {
+        int dev;
+        size_t n;
+        void* p;
+    };
+    static constexpr size_t KEPT_MAX = 64u << 20;
+    static std::mutex& mu()
+    {
+        static std::mutex m;
+        return m;
+    }
+    static std::vector<Idle>& idle()
+    {
+        static std::vector<Idle> v;
+        return v;
+    }
+    static size_t kept()
+    {
+        size_t n = 0;
+        for (auto& b : idle()) n += b.n;
+        return n;
+    }
+    int dev_ = 0;
+    size_t n_ = 0;
+    void* p_ = nullptr;
+};
 
 static bool have_kfd() { return access("/dev/kfd", F_OK) == 0; }
 

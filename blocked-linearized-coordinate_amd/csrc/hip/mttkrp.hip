@@ -19,9 +19,10 @@
 // reference's match_any / labeled_partition / shuffle-scan counting sort,
 // which has no wave64 equivalent.
 //
-// lvl3 ("privatised"): the same per-tile segmentation, but segments are
-// added into a workgroup-private copy of the whole output held in LDS (short
-// modes only); at the end the workgroup adds its copy into partial matrix
+// lvl3 ("privatised"): every product is added into a workgroup-private copy of
+// the whole output held in LDS (short modes only), with the gathers of the
+// row-ordered kernel and no segmentation (factors of 2 GiB and more keep lvl1's
+// tiles and segments); at the end the workgroup adds its copy into partial matrix
 // (workgroup % nprtn) -- or straight into the output when nprtn == 1 -- and
 // a pull reduction sums the partial matrices (partial_matrix_reduction,
 // src/alto_dev.cu:1589-1601).
@@ -115,7 +116,7 @@ __global__ __launch_bounds__(WG) void k_fill(T* __restrict__ x, uint64_t n, T v)
 
 const void* mttkrp_kernel(int which, int nmodes, int ftype, int rank, int* C, int* L)
 {
-    const bool rows = which == W_ROWS || which == W_ROWS_SHORT || which == W_ROWS_BATCH;
+    const bool rows = which == W_ROWS || which == W_ROWS_SHORT || which == W_ROWS_BATCH || which == W_LVL3_ROWS;
     const Shape s = rows ? rows_shape(rank, dtype_size(ftype)) : pick_shape(rank, dtype_size(ftype));
     *C = s.C;
     *L = s.L;

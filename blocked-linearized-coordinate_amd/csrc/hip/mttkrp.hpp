@@ -87,7 +87,8 @@ struct RowsPlan {
 };
 
 enum { W_LVL1 = 0, W_LVL3 = 1, W_ATOMIC = 2, W_WINDOW = 3, W_WINDOW64 = 4, W_SORTED64 = 5, W_FIBER64 = 6,
-       W_SORTED_LDS = 7, W_FIBER_LDS = 8, W_ROWS = 9, W_ROWS_SHORT = 10, W_ROWS_BATCH = 11 };
+       W_SORTED_LDS = 7, W_FIBER_LDS = 8, W_ROWS = 9, W_ROWS_SHORT = 10, W_ROWS_BATCH = 11,
+       W_LVL3_ROWS = 12 };
 
 // The row-ordered and fiber kernels take 31-bit byte offsets into factors
 // of fewer bytes than this (bit 31 marks an offset into an LDS window).

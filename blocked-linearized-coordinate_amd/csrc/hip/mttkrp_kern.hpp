@@ -1176,6 +1176,131 @@ __global__ __launch_bounds__(WG) void k_mttkrp_rows_batch(const MttkrpArgs* __re
     rows_chunk<N, FT, VT, C, L, Q>(a, Chunk{bc.begin, bc.len, bc.block}, s_stage[w], s_row[w]);
 }
 
+// lvl3 for factors of fewer than FACTOR_BYTES_MAX bytes: rounds, gathers and
+// broadcasts as in rows_chunk over chunks in ALTO order; each product goes
+// straight to the workgroup's copy of the output in LDS (one LDS add per
+// element, about an eighth of what its gathers cost), without sorting tiles.
+// 3.3M nonzeros into 24 rows, FP64 rank 10: 635 us with sorted tiles,
+// single-element gathers and 202 workgroups.
+template <int N, typename FT, typename VT, int C, int L, int Q>
+__global__ __launch_bounds__(WG) void k_mttkrp_lvl3_rows(MttkrpArgs a)
+{
+    using AT = typename Acc<FT>::type;
+    constexpr int S = WAVE / L;
+    constexpr int P = L * Q;
+    constexpr int ROW_REGS = (N - 1) * C * (int)sizeof(AT) / 4;
+    constexpr int PB = ROW_REGS <= 8 ? 4 : ROW_REGS <= 16 ? 2 : 1;
+    constexpr int KS = PB < Q ? PB : Q;
+    constexpr int LS = PB / KS;
+    constexpr uint32_t NONE = 0x80000000u;
+    extern __shared__ __align__(16) unsigned char s_dyn[];
+    AT* s_out = reinterpret_cast<AT*>(s_dyn);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int R = a.rank;
+    const uint32_t cells = (uint32_t)(a.out_rows * (uint64_t)R);
+    for (uint32_t e = threadIdx.x; e < cells; e += WG) s_out[e] = 0;
+    __syncthreads();
+    const uint32_t row_bytes = (uint32_t)R * (uint32_t)sizeof(FT);
+    const int slot = lane / L, sub = lane % L;
+    __amdgpu_buffer_rsrc_t rs[N - 1];
+    uint64_t mk[N];
+    int ps[N];
+    #pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const int m = a.order[j];
+        if (j < N - 1) rs[j] = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.f[m]), 0, NONE, 0x00020000);
+        mk[j] = a.mask[m];
+        ps[j] = a.pos[m];
+    }
+    const uint32_t cbeg = a.chunk0 + blockIdx.x * a.chunks_per_wg;
+    const uint32_t cend = min(cbeg + a.chunks_per_wg, a.chunk0 + a.nchunks);
+    for (uint32_t c = cbeg + w; c < cend; c += WAVES_PER_WG) {
+        const Chunk ch = a.chunks[c];
+        uint32_t bc[N];
+        #pragma unroll
+        for (int j = 0; j < N; ++j) bc[j] = (uint32_t)a.bcoords[(uint64_t)ch.block * N + a.order[j]];
+        const VT* vals = reinterpret_cast<const VT*>(a.vals) + (ch.begin - a.coord_base);
+        const uint64_t* words = a.coords + (ch.begin - a.coord_base);
+        for (int cb = 0; cb < R; cb += C * L) {
+            const int width = min(R - cb, C * L);
+            const int c0 = min(sub * C, width - C);
+            const uint32_t colb = (uint32_t)(cb + c0) * (uint32_t)sizeof(FT);
+            for (uint32_t base = 0; base < ch.len;) {
+                const uint32_t run = min((uint32_t)P, (ch.len - base + S - 1) / S);
+                const uint32_t q = base + slot * run + sub * Q;
+                const int left = min((int)run - sub * Q, (int)ch.len - (int)q);
+                base += S * run;
+                uint64_t word[Q];
+                VT val[Q];
+                if (q + Q <= ch.len) {
+                    load_run<Q>(words + q, word);
+                    load_run<Q>(vals + q, val);
+                } else {
+                    #pragma unroll
+                    for (int k = 0; k < Q; ++k) {
+                        const uint32_t e = min(q + k, ch.len - 1);
+                        word[k] = words[e];
+                        val[k] = vals[e];
+                    }
+                }
+                uint32_t off[Q][N - 1], cell[Q];
+                AT v[Q];
+                #pragma unroll
+                for (int k = 0; k < Q; ++k) {
+                    const bool valid = k < left;
+                    #pragma unroll
+                    for (int j = 0; j < N - 1; ++j)
+                        off[k][j] = valid ? ((uint32_t)((word[k] >> ps[j]) & mk[j]) | bc[j]) * row_bytes : NONE;
+                    cell[k] = valid ? ((uint32_t)((word[k] >> ps[N - 1]) & mk[N - 1]) | bc[N - 1]) * (uint32_t)R : NONE;
+                    v[k] = valid ? (AT)val[k] : (AT)0;
+                }
+                unrolled<L / LS>([&](auto g) {
+                    if (g * LS * Q < run) {
+                        #pragma unroll
+                        for (int kb = 0; kb < Q; kb += KS) {
+                            AT x[PB][N - 1][C];
+                            unrolled<LS>([&](auto s) {
+                                constexpr int ln = g * LS + s;
+                                #pragma unroll
+                                for (int k = 0; k < KS; ++k) {
+                                    #pragma unroll
+                                    for (int j = 0; j < N - 1; ++j)
+                                        load_row_buf<FT, C>(rs[j], group_bcast<ln, L>(off[kb + k][j]) + colb,
+                                                            x[s * KS + k][j]);
+                                }
+                            });
+                            unrolled<LS>([&](auto s) {
+                                constexpr int ln = g * LS + s;
+                                #pragma unroll
+                                for (int k = 0; k < KS; ++k) {
+                                    const uint32_t at = group_bcast<ln, L>(cell[kb + k]);
+                                    const AT vb = group_bcast<ln, L>(v[kb + k]);
+                                    #pragma unroll
+                                    for (int cc = 0; cc < C; ++cc) {
+                                        AT t = vb;
+                                        #pragma unroll
+                                        for (int j = 0; j < N - 1; ++j) t *= x[s * KS + k][j][cc];
+                                        // columns that this lane repeats belong to the lane before
+                                        if (at != NONE && c0 + cc >= sub * C)
+                                            atomic_add_lds(s_out + at + cb + c0 + cc, t);
+                                    }
+                                }
+                            });
+                        }
+                    }
+                });
+            }
+        }
+    }
+    __syncthreads();
+    AT* dst = reinterpret_cast<AT*>(a.nprtn > 1 ? a.partials : a.out);
+    if (a.nprtn > 1) dst += (uint64_t)(blockIdx.x % (uint32_t)a.nprtn) * cells;
+    for (uint32_t e = threadIdx.x; e < cells; e += WG) {
+        const AT v = s_out[e];
+        if (v != (AT)0) atomic_add_global(dst + e, v);
+    }
+}
+
 // MTTKRP over a row-ordered copy with the hot rows of two input modes in LDS
 // windows and every round's decoded nonzeros staged in LDS.  Slots
 // and rounds are those of k_mttkrp_sorted: each lane decodes the nonzero of
@@ -1571,6 +1696,7 @@ inline Shape rows_shape(int rank, int esize)
 template <int N, typename FT, typename VT, int C, int L>
 inline const void* rows_ptr(int which)
 {
+    if (which == W_LVL3_ROWS) return (const void*)&k_mttkrp_lvl3_rows<N, FT, VT, C, L, L == 16 ? 1 : 2>;
     if (which == W_ROWS_BATCH) return (const void*)&k_mttkrp_rows_batch<N, FT, VT, C, L, L == 16 ? 1 : 2>;
     // short runs take rounds of fewer positions
     if (which == W_ROWS_SHORT) return (const void*)&k_mttkrp_rows<N, FT, VT, C, L, L == 16 ? 1 : 2>;
@@ -1602,7 +1728,8 @@ inline const void* select_rows(const Shape& s, int which)
 template <int N, typename FT, typename VT>
 inline const void* select_shape(const Shape& s, int which)
 {
-    if (which == W_ROWS || which == W_ROWS_SHORT || which == W_ROWS_BATCH) return select_rows<N, FT, VT>(s, which);
+    if (which == W_ROWS || which == W_ROWS_SHORT || which == W_ROWS_BATCH || which == W_LVL3_ROWS)
+        return select_rows<N, FT, VT>(s, which);
     if (s.exact) {
         if (s.C == 1 && s.L == 8) return kernel_ptr<N, FT, VT, 1, 8, true>(which);
         if (s.C == 2 && s.L == 8) return kernel_ptr<N, FT, VT, 2, 8, true>(which);
