@@ -217,29 +217,32 @@ __device__ __forceinline__ double lane_value(double x, int lane)
     return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
 }
 
-// X = L^{-1} (lower, row-major in s_x) of the Cholesky factor L of s_a, by one
-// wave and in registers (R <= RP): lane i holds row i of the matrix while it
-// is factored, then column i of X.  Right-looking in both parts, so every
-// entry's terms are subtracted in the order of dpotf2's column dot products.
-// No barriers (by a workgroup in LDS the factorisation took 42 us at R = 32
-// and 16 us at R = 16).
-// False when a pivot falls to `floor_piv` or below (the same for every lane).
+// V = s_a = L D L^T by one wave and in registers (R <= RP): X = L^{-1} (unit
+// lower, row-major) into s_x and D^{-1} X into s_a.  Lane i holds row i of
+// the matrix while it is factored, then column i of X.  Right-looking, so
+// every entry's terms are subtracted in the order of dpotf2's column dot
+// products; D_j is the pivot that dpotf2 would take the root of.  One
+// reciprocal a column, no root and no barriers: by a workgroup in LDS the
+// Cholesky form took 42 us at R = 32 and 16 us at R = 16.  False when a pivot
+// falls to `floor_piv` or below (the same for every lane).
 template <int RP>
-__device__ __forceinline__ bool chol_inverse_wave(const double* s_a, double* s_x, int R, double floor_piv)
+__device__ __forceinline__ bool ldl_inverse_wave(double* s_a, double* s_x, int R, double floor_piv)
 {
     const int lane = threadIdx.x & 63;
-    double a[RP];
+    double a[RP], rd[RP];
     #pragma unroll
     for (int k = 0; k < RP; ++k) a[k] = (lane < R && k < R) ? s_a[lane * R + k] : (lane == k ? 1.0 : 0.0);
     #pragma unroll
     for (int j = 0; j < RP; ++j) {
+        rd[j] = 1.0;
         if (j < R) {
             const double ajj = lane_value(a[j], j);
             if (!(ajj > floor_piv)) return false;
-            const double piv = sqrt(ajj);
-            a[j] = lane > j ? a[j] / piv : lane == j ? piv : 0.0;
+            rd[j] = 1.0 / ajj;
+            const double l = lane > j ? a[j] * rd[j] : 0.0;
             #pragma unroll
-            for (int k = j + 1; k < RP; ++k) a[k] -= a[j] * lane_value(a[j], k);
+            for (int k = j + 1; k < RP; ++k) a[k] -= l * lane_value(a[j], k);
+            a[j] = l;
         }
     }
     double x[RP];
@@ -248,17 +251,19 @@ __device__ __forceinline__ bool chol_inverse_wave(const double* s_a, double* s_x
     #pragma unroll
     for (int k = 0; k < RP; ++k) {
         if (k < R) {
-            x[k] /= lane_value(a[k], k);
             #pragma unroll
             for (int i = k + 1; i < RP; ++i) x[i] -= lane_value(a[k], i) * x[k];
-            if (lane < R) s_x[k * R + lane] = x[k];
+            if (lane < R) {
+                s_x[k * R + lane] = x[k];
+                s_a[k * R + lane] = x[k] * rd[k];
+            }
         }
     }
     return true;
 }
 
-// The same by the whole workgroup in LDS (s_a is overwritten), for ranks
-// whose rows do not fit a lane's registers.
+// X = L^{-1} of the Cholesky factor of s_a (overwritten) into s_x, by the
+// whole workgroup in LDS, for ranks whose rows do not fit a lane's registers.
 __device__ __forceinline__ bool chol_inverse_lds(double* s_a, double* s_x, int R, double floor_piv)
 {
     const int tid = threadIdx.x, nt = blockDim.x;
@@ -381,7 +386,7 @@ __device__ void jacobi_pinv(int R, double eps, double* __restrict__ work, double
 }
 
 // The whole workgroup: V = s_a (R x R, also kept in work), then fac = V^{-1}
-// = L^{-T} L^{-1} with status 0, or V^+ with status 1.
+// = X^T D^{-1} X with status 0, or V^+ with status 1.
 // A pivot at or below R * eps * max_i V_ii means V is singular to the working
 // precision its Grams carry: its Cholesky factor would carry pivots of
 // rounding noise (and the solve factors of that size), so the pseudo-inverse
@@ -402,8 +407,8 @@ __device__ __forceinline__ void factorize_block(double* s_a, double* s_x, int R,
     bool ok;
     if (R <= 32) {
         if (tid < WAVE) {
-            const bool r = R <= 16 ? chol_inverse_wave<16>(s_a, s_x, R, floor_piv)
-                                   : chol_inverse_wave<32>(s_a, s_x, R, floor_piv);
+            const bool r = R <= 16 ? ldl_inverse_wave<16>(s_a, s_x, R, floor_piv)
+                                   : ldl_inverse_wave<32>(s_a, s_x, R, floor_piv);
             if (tid == 0) s_ok = r;
         }
         __syncthreads();
@@ -412,10 +417,11 @@ __device__ __forceinline__ void factorize_block(double* s_a, double* s_x, int R,
         ok = chol_inverse_lds(s_a, s_x, R, floor_piv);
     }
     if (ok) {
+        const double* s_y = R <= 32 ? s_a : s_x;  // D^{-1} X, or X where L holds the roots
         for (int e = tid; e < R * R; e += nt) {
             const int a = e / R, b = e % R;
             double t = 0.0;
-            for (int k = a > b ? a : b; k < R; ++k) t += s_x[k * R + a] * s_x[k * R + b];
+            for (int k = a > b ? a : b; k < R; ++k) t += s_x[k * R + a] * s_y[k * R + b];
             fac[e] = t;
         }
         if (tid == 0) *status = 0;
@@ -550,21 +556,30 @@ __global__ __launch_bounds__(WG) void k_solve_rows(const MT* __restrict__ M, UT*
             b[ct][ks] = (k < R && j < R) ? fac[j * R + k] : 0.0;
         }
     const uint64_t tiles = (rows + 15) / 16, stride = (uint64_t)gridDim.x * WAVES_PER_WG;
-    for (uint64_t tile = (uint64_t)blockIdx.x * WAVES_PER_WG + w; tile < tiles; tile += stride) {
-        const uint64_t r0 = tile * 16, ra = r0 + i16;
-        d4 d[T];
-        #pragma unroll
-        for (int ct = 0; ct < T; ++ct) d[ct] = d4{0, 0, 0, 0};
-        double m[KS];
+    MT m[KS];  // the next tile's operands, loaded behind this one's MFMAs
+    auto load = [&](uint64_t tile) {
+        const uint64_t ra = tile * 16 + i16;
         #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             const int k = 4 * ks + k4;
-            m[ks] = (ra < rows && k < R) ? (double)M[ra * (uint64_t)R + k] : 0.0;
+            m[ks] = (ra < rows && k < R) ? M[ra * (uint64_t)R + k] : (MT)0;
         }
+    };
+    uint64_t tile = (uint64_t)blockIdx.x * WAVES_PER_WG + w;
+    load(tile);
+    for (; tile < tiles; tile += stride) {
+        const uint64_t r0 = tile * 16;
+        d4 d[T];
+        #pragma unroll
+        for (int ct = 0; ct < T; ++ct) d[ct] = d4{0, 0, 0, 0};
+        double x[KS];
+        #pragma unroll
+        for (int ks = 0; ks < KS; ++ks) x[ks] = (double)m[ks];
+        load(tile + stride);
         #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
             #pragma unroll
-            for (int ct = 0; ct < T; ++ct) d[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(m[ks], b[ct][ks], d[ct], 0, 0, 0);
+            for (int ct = 0; ct < T; ++ct) d[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[ks], b[ct][ks], d[ct], 0, 0, 0);
         #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const uint64_t row = r0 + k4 + 4 * v;
@@ -786,49 +801,65 @@ __global__ __launch_bounds__(FINISH_WG) void k_als_finish(const AlsTask* __restr
     __shared__ double s_red[FINISH_WG / WAVE];
     const int tid = threadIdx.x, W = R * R + R;
     const int np = (int)tk.parts <= FINISH_PARTS ? (int)tk.parts : RED_SPLIT;
-    const int mode = tk.mode, nmodes = tk.nmodes;
+    const int mode = tk.mode, nmodes = tk.nmodes, next = tk.next, last = tk.last;
+    // the Grams that this update leaves as they are: their product into s_v
+    for (int e = tid; e < R * R; e += FINISH_WG) {
+        double v = 1.0;
+        for (int m = 0; m < nmodes; ++m)
+            if (m != next && !(update && m == mode)) v *= tk.G[m][e];
+        s_v[e] = v;
+    }
     if (update) {
-        for (int c = tid; c < R; c += FINISH_WG) {
-            double y = tk.stats[c];
-            for (int p = 1; p < np; ++p) y = fold_op(which, y, tk.stats[(uint64_t)p * R + c]);
-            if (which == 0) y = sqrt(y);
-            const double iv = (y == 0.0) ? 0.0 : 1.0 / y;
-            s_lam[c] = y;
-            s_inv[c] = iv;
-            tk.lambda[c] = y;
-            tk.dinv[mode * R + c] = iv;
-        }
-        __syncthreads();
-        for (int e = tid; e < W; e += FINISH_WG) {
-            double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-            int p = 0;
-            for (; p + 4 <= np; p += 4) {
-                const double* q = tk.part + (uint64_t)p * W + e;
-                s0 += q[0];
-                s1 += q[W];
-                s2 += q[2 * W];
-                s3 += q[3 * W];
+        // sums over the partial rows, eight loads in flight: G and ip, then
+        // the statistics
+        for (int e = tid; e < W + R; e += FINISH_WG) {
+            const bool stat = e >= W;
+            const int op = stat ? which : 0;
+            const uint64_t width = stat ? R : W;
+            const double* q = stat ? tk.stats + (e - W) : tk.part + e;
+            double t = q[0];
+            int p = 1;
+            for (; p + 8 <= np; p += 8) {
+                double x[8];
+                #pragma unroll
+                for (int u = 0; u < 8; ++u) x[u] = q[(p + u) * width];
+                #pragma unroll
+                for (int u = 0; u < 8; ++u) t = fold_op(op, t, x[u]);
             }
-            for (; p < np; ++p) s0 += tk.part[(uint64_t)p * W + e];
-            double g = (s0 + s1) + (s2 + s3);
-            if (e < R * R) {
-                g *= s_inv[e / R] * s_inv[e % R];
-                tk.G[mode][e] = g;
-                s_g[e] = g;
+            {
+                double x[7];
+                #pragma unroll
+                for (int u = 0; u < 7; ++u) x[u] = p + u < np ? q[(p + u) * width] : (op == 0 ? 0.0 : t);
+                #pragma unroll
+                for (int u = 0; u < 7; ++u) t = fold_op(op, t, x[u]);
+            }
+            if (stat) {
+                const int c = e - W;
+                if (which == 0) t = sqrt(t);
+                const double iv = (t == 0.0) ? 0.0 : 1.0 / t;
+                s_lam[c] = t;
+                s_inv[c] = iv;
+                tk.lambda[c] = t;
+                tk.dinv[mode * R + c] = iv;
+            } else if (e < R * R) {
+                s_g[e] = t;
             } else {
-                const int r = e - R * R;
-                s_ip[r] = g * s_inv[r] * tk.colscale[r];
+                s_ip[e - R * R] = t * tk.colscale[e - R * R];
             }
         }
         __syncthreads();
-        if (tk.last) {
+        for (int e = tid; e < R * R; e += FINISH_WG) {
+            const double g = s_g[e] * (s_inv[e / R] * s_inv[e % R]);
+            tk.G[mode][e] = g;
+            s_g[e] = g;
+        }
+        if (last) {
             // fit = 1 - r / ||X||, as k_fit
             double sum = 0.0;
-            for (int e = tid; e < R * R; e += FINISH_WG) {
+            for (int e = tid; e < R * R; e += FINISH_WG) {  // this thread's own entries of s_g and s_v
                 const int i = e / R, j = e % R;
                 if (j > i) continue;
-                double t = s_lam[i] * s_lam[j];
-                for (int m = 0; m < nmodes; ++m) t *= m == mode ? s_g[e] : tk.G[m][e];
+                const double t = (s_lam[i] * s_lam[j]) * ((s_v[e] * tk.G[next][e]) * s_g[e]);
                 sum += j < i ? 2.0 * t : t;
             }
             #pragma unroll
@@ -838,7 +869,7 @@ __global__ __launch_bounds__(FINISH_WG) void k_als_finish(const AlsTask* __restr
             if (tid == 0) {
                 double model = 0.0, inner = 0.0;
                 for (int i = 0; i < FINISH_WG / WAVE; ++i) model += s_red[i];
-                for (int r = 0; r < R; ++r) inner += s_ip[r] * s_lam[r];
+                for (int r = 0; r < R; ++r) inner += (s_ip[r] * s_inv[r]) * s_lam[r];
                 model = fabs(model);
                 const double x2 = *tk.normX2;
                 double res = x2 + model - 2.0 * inner;
@@ -851,7 +882,6 @@ __global__ __launch_bounds__(FINISH_WG) void k_als_finish(const AlsTask* __restr
     }
     // the next mode's V, and the column scale its MTTKRP result carries: the
     // product of the other factors' pending inverse scales
-    const int next = tk.next;
     for (int k = tid; k < R; k += FINISH_WG) {
         double c = 1.0;
         for (int m = 0; m < nmodes; ++m)
@@ -859,9 +889,7 @@ __global__ __launch_bounds__(FINISH_WG) void k_als_finish(const AlsTask* __restr
         tk.colscale[k] = c;
     }
     for (int e = tid; e < R * R; e += FINISH_WG) {
-        double v = 1.0;
-        for (int m = 0; m < nmodes; ++m)
-            if (m != next) v *= update && m == mode ? s_g[e] : tk.G[m][e];
+        const double v = update ? s_v[e] * s_g[e] : s_v[e];
         s_v[e] = v;
         tk.work[e] = v;  // for the fallback
     }
