@@ -64,6 +64,15 @@ static int sorted_tpw(const blco_dev* d, int mode, int rank, int ftype)
     return t;
 }
 
+// Nonzeros of one streamed unit: a quarter of the tensor where that is below
+// the slot, so that copies and kernels of neighbouring units overlap (20M
+// nonzeros in slots of 2^24 were one unit of 16.8M, whose kernel nothing
+// overlapped, and one of 3.2M), but not so few that the copies' own cost shows.
+static uint64_t stream_unit(const blco_dev* d)
+{
+    return std::min(d->slot_nnz, std::max<uint64_t>(1ull << 21, (d->nnz + 3) / 4));
+}
+
 const ChunkTab* chunk_table(blco_dev* d, int tpw)
 {
     for (auto& t : d->tabs)
@@ -91,7 +100,7 @@ const ChunkTab* chunk_table(blco_dev* d, int tpw)
             uint32_t u0 = c0;
             uint64_t acc = 0;
             for (uint32_t c = c0; c < c1; ++c) {
-                if (acc + h[c].len > d->slot_nnz && c > u0) {
+                if (acc + h[c].len > stream_unit(d) && c > u0) {
                     t.units.push_back({u0, c, h[u0].begin, acc});
                     u0 = c;
                     acc = 0;
@@ -906,6 +915,70 @@ static size_t plan_rows(blco_dev* d, int mode, int rank, int ftype, bool fib, Mt
     return lds;
 }
 
+// The words of fine chunks from their packed form, a workgroup per chunk.
+__global__ __launch_bounds__(WG) void k_unpack(const PackChunk* __restrict__ pack, uint64_t first_dword,
+                                               uint64_t first_nz, const uint32_t* __restrict__ packed, BlcoPos pos,
+                                               int nmodes, uint64_t* __restrict__ coords)
+{
+    const PackChunk pc = pack[blockIdx.x];
+    const uint32_t* src = packed + (pc.at - first_dword);
+    uint64_t* dst = coords + (pc.begin - first_nz);
+    const uint32_t w = pc.width;
+    for (uint32_t i = threadIdx.x; i < pc.len; i += WG) {
+        const uint64_t bit = (uint64_t)i * w;
+        const uint32_t* q = src + (bit >> 5);
+        const uint32_t sh = (uint32_t)bit & 31;
+        // w <= 64 bits from bit sh on: at most three dwords (two lie past the
+        // last chunk's end at most; the packed buffers hold them)
+        uint64_t v = ((uint64_t)q[1] << 32 | q[0]) >> sh;
+        if (sh + w > 64) v |= (uint64_t)q[2] << (64 - sh);
+        uint64_t word = pc.base;
+        for (int m = 0; m < nmodes; ++m) {
+            const uint32_t b = pc.bits[m];
+            word += (v & (((uint64_t)1 << b) - 1)) << pos.p[m];
+            v >>= b;
+        }
+        dst[i] = word;
+    }
+}
+
+// Copies the nonzeros [begin, begin + cnt) of a streamed tensor into slot s
+// and makes `st` wait for them; *base is the nonzero at the slot's start.
+// Packed words travel in whole fine chunks and are unpacked on `st`: 20M
+// nonzeros over 48,000 x 18,000 x 18,000, FP32, 5.28 -> 3.45 ms a mode with
+// this and units of a quarter (stream_unit), bound by the link either way.
+static int stage_unit(blco_dev* d, int s, uint64_t begin, uint64_t cnt, hipStream_t st, uint64_t* base)
+{
+    const int vsz = value_size(d->vdtype);
+    HIP_TRY(hipStreamWaitEvent(d->copy_stream, d->ev_done[s], 0));
+    uint64_t f0 = 0, f1 = 0, lo = begin, hi = begin + cnt;
+    if (d->h_packed) {
+        const std::vector<uint64_t>& fb = d->fine_begin;
+        f0 = (uint64_t)(std::upper_bound(fb.begin(), fb.end(), begin) - fb.begin()) - 1;
+        f1 = (uint64_t)(std::lower_bound(fb.begin(), fb.end(), begin + cnt) - fb.begin());
+        lo = fb[f0];
+        hi = fb[f1 - 1] + d->fine_len[f1 - 1];
+        const uint64_t at = d->pack_h[f0].at, n = d->pack_h[f1].at - at;
+        if (hi - lo > d->slot_cap || n + 2 > d->packed_cap)
+            return fail(BLCO_EUNSUPPORTED, "a unit of %llu nonzeros exceeds the streaming slot", (unsigned long long)cnt);
+        HIP_TRY(hipMemcpyAsync(d->slot_packed[s], d->h_packed + at, n * 4, hipMemcpyHostToDevice, d->copy_stream));
+    } else {
+        HIP_TRY(hipMemcpyAsync(d->slot_coords[s], d->h_coords + lo, cnt * 8, hipMemcpyHostToDevice, d->copy_stream));
+    }
+    HIP_TRY(hipMemcpyAsync(d->slot_vals[s], (const char*)d->h_vals + lo * vsz, (hi - lo) * vsz, hipMemcpyHostToDevice,
+                           d->copy_stream));
+    HIP_TRY(hipEventRecord(d->ev_copied[s], d->copy_stream));
+    HIP_TRY(hipStreamWaitEvent(st, d->ev_copied[s], 0));
+    *base = lo;
+    if (!d->h_packed) return BLCO_OK;
+    BlcoPos pos;
+    for (int m = 0; m < BLCO_MAX_MODES; ++m) pos.p[m] = d->pos[m];
+    hipLaunchKernelGGL(k_unpack, dim3((uint32_t)(f1 - f0)), dim3(WG), 0, st, d->d_pack + f0, d->pack_h[f0].at, lo,
+                       d->slot_packed[s], pos, d->nmodes, d->slot_coords[s]);
+    HIP_TRY(hipGetLastError());
+    return BLCO_OK;
+}
+
 int mttkrp_prepare(blco_dev* d, int mode, int rank, int ftype, int kernel)
 {
     if (!d || mode < 0 || mode >= d->nmodes || !d->nnz || d->stream_data) return BLCO_OK;
@@ -1108,7 +1181,6 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
         for (int m = 0; m < d->nmodes; ++m) wide |= d->dims[m] > 0xFFFFFFFFull;
         const int wk = wide ? W_WINDOW64 : W_WINDOW;
         const bool per_block = kernel == BLCO_K_LVL2;
-        const int vsz = value_size(d->vdtype);
         if (!d->stream_data) {
             a.coords = d->d_coords;
             a.vals = d->d_vals;
@@ -1132,7 +1204,7 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
                 while (e < wt->first[b + 1] && !rc) {
                     uint32_t e1 = e;
                     uint64_t cnt = 0;
-                    while (e1 < wt->first[b + 1] && (e1 == e || cnt + wt->h_sc[e1].len <= d->slot_nnz)) {
+                    while (e1 < wt->first[b + 1] && (e1 == e || cnt + wt->h_sc[e1].len <= stream_unit(d))) {
                         cnt += wt->h_sc[e1].len;
                         ++e1;
                     }
@@ -1151,16 +1223,9 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
                         continue;
                     }
                     const int s = (int)(u & 1);
-                    HIP_TRY(hipStreamWaitEvent(d->copy_stream, d->ev_done[s], 0));
-                    HIP_TRY(hipMemcpyAsync(d->slot_coords[s], d->h_coords + begin, cnt * 8,
-                                           hipMemcpyHostToDevice, d->copy_stream));
-                    HIP_TRY(hipMemcpyAsync(d->slot_vals[s], (const char*)d->h_vals + begin * vsz,
-                                           cnt * vsz, hipMemcpyHostToDevice, d->copy_stream));
-                    HIP_TRY(hipEventRecord(d->ev_copied[s], d->copy_stream));
-                    HIP_TRY(hipStreamWaitEvent(st, d->ev_copied[s], 0));
+                    if ((rc = stage_unit(d, s, begin, cnt, st, &a.coord_base))) break;
                     a.coords = d->slot_coords[s];
                     a.vals = d->slot_vals[s];
-                    a.coord_base = begin;
                     rc = launch_mttkrp(wk, a, ftype, a.nchunks, lds, st);
                     HIP_TRY(hipEventRecord(d->ev_done[s], st));
                     ++u;
@@ -1210,7 +1275,6 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
     } else {
         // double-buffered streaming: the k-th unit beyond the resident
         // prefix goes through slot k % 2
-        const int vsz = value_size(d->vdtype);
         size_t k = 0;
         for (size_t u = 0; u < t->units.size() && !rc; ++u) {
             const StreamUnit& su = t->units[u];
@@ -1222,16 +1286,9 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
                 continue;
             }
             const int s = (int)(k++ & 1);
-            HIP_TRY(hipStreamWaitEvent(d->copy_stream, d->ev_done[s], 0));
-            HIP_TRY(hipMemcpyAsync(d->slot_coords[s], d->h_coords + su.begin, su.nnz * 8,
-                                   hipMemcpyHostToDevice, d->copy_stream));
-            HIP_TRY(hipMemcpyAsync(d->slot_vals[s], (const char*)d->h_vals + su.begin * vsz,
-                                   su.nnz * vsz, hipMemcpyHostToDevice, d->copy_stream));
-            HIP_TRY(hipEventRecord(d->ev_copied[s], d->copy_stream));
-            HIP_TRY(hipStreamWaitEvent(st, d->ev_copied[s], 0));
+            if ((rc = stage_unit(d, s, su.begin, su.nnz, st, &a.coord_base))) break;
             a.coords = d->slot_coords[s];
             a.vals = d->slot_vals[s];
-            a.coord_base = su.begin;
             rc = launch_range(d, which, a, t, su.c0, su.c1, ftype, st);
             HIP_TRY(hipEventRecord(d->ev_done[s], st));
         }
@@ -1560,12 +1617,34 @@ int create_device_tensor(int nmodes, const uint64_t* dims, const uint64_t* masks
             }
         }
     } else {
+        uint32_t widest = 0;
         if (nnz) {
-            if (hipHostMalloc((void**)&d->h_coords, nnz * 8, hipHostMallocDefault) != hipSuccess ||
-                hipHostMalloc(&d->h_vals, nnz * vsz, hipHostMallocDefault) != hipSuccess)
+            // packed words (no budget: they take slots of their own)
+            uint64_t dwords = 0;
+            bool packed = false;
+            try {
+                packed = !device_budget && pack_words(nmodes, d->masks, d->pos, nnz, coords, d->fine_begin, d->fine_len,
+                                                      &d->pack_h, &dwords, &widest);
+            } catch (const std::bad_alloc&) {
+                return cleanup(fail(BLCO_ENOMEM, "host tables of the packed words"));
+            }
+            const bool ok = packed ? hipHostMalloc((void**)&d->h_packed, (dwords + 2) * 4, hipHostMallocDefault) == hipSuccess
+                                   : hipHostMalloc((void**)&d->h_coords, nnz * 8, hipHostMallocDefault) == hipSuccess;
+            if (!ok || hipHostMalloc(&d->h_vals, nnz * vsz, hipHostMallocDefault) != hipSuccess)
                 return cleanup(fail(BLCO_ENOMEM, "pinned host allocation of %llu nonzeros failed",
                                     (unsigned long long)nnz));
-            std::memcpy(d->h_coords, coords, nnz * 8);
+            if (packed) {
+                write_packed(nmodes, d->masks, d->pos, coords, d->pack_h, d->h_packed);
+                const uint64_t nf = d->fine_begin.size();
+                if (hipMalloc(&d->d_pack, sizeof(PackChunk) * nf) != hipSuccess)
+                    return cleanup(fail(BLCO_ENOMEM, "device allocation failed (packed words' table)"));
+                if (hipMemcpy(d->d_pack, d->pack_h.data(), sizeof(PackChunk) * nf, hipMemcpyHostToDevice) != hipSuccess)
+                    return cleanup(fail(BLCO_EHIP, "upload of the packed words' table failed"));
+                d->bytes += sizeof(PackChunk) * nf;
+            } else {
+                d->pack_h.clear();
+                std::memcpy(d->h_coords, coords, nnz * 8);
+            }
             convert(0, nnz, d->h_vals);
         }
         if (res_nnz) {  // the resident prefix, from the pinned copy
@@ -1578,6 +1657,15 @@ int create_device_tensor(int nmodes, const uint64_t* dims, const uint64_t* masks
                 return cleanup(fail(BLCO_EHIP, "upload of the resident nonzeros failed"));
         }
         uint64_t cap = std::min<uint64_t>(slot_nnz, nnz ? nnz : 1);
+        if (d->h_packed) {  // whole fine chunks around a unit, and two dwords read past its end
+            cap = std::min<uint64_t>(std::min(slot_nnz, stream_unit(d)) + 2 * FINE_CHUNK, nnz);
+            d->packed_cap = (cap * widest + 31) / 32 + cap / FINE_CHUNK + nblocks + 4;
+            for (int s = 0; s < 2; ++s)
+                if (hipMalloc(&d->slot_packed[s], d->packed_cap * 4) != hipSuccess)
+                    return cleanup(fail(BLCO_ENOMEM, "device slot allocation failed"));
+            d->bytes += 2 * d->packed_cap * 4;
+        }
+        d->slot_cap = cap;
         for (int s = 0; s < 2; ++s) {
             if (hipMalloc(&d->slot_coords[s], cap * 8) != hipSuccess || hipMalloc(&d->slot_vals[s], cap * vsz) != hipSuccess)
                 return cleanup(fail(BLCO_ENOMEM, "device slot allocation failed"));
@@ -1893,11 +1981,14 @@ void blco_dev_free(blco_dev* d)
     if (d->partials) (void)hipFree(d->partials);
     for (int s = 0; s < 2; ++s) {
         if (d->slot_coords[s]) (void)hipFree(d->slot_coords[s]);
+        if (d->slot_packed[s]) (void)hipFree(d->slot_packed[s]);
         if (d->slot_vals[s]) (void)hipFree(d->slot_vals[s]);
         if (d->ev_copied[s]) (void)hipEventDestroy(d->ev_copied[s]);
         if (d->ev_done[s]) (void)hipEventDestroy(d->ev_done[s]);
     }
     if (d->h_coords) (void)hipHostFree(d->h_coords);
+    if (d->h_packed) (void)hipHostFree(d->h_packed);
+    if (d->d_pack) (void)hipFree(d->d_pack);
     if (d->h_vals) (void)hipHostFree(d->h_vals);
     if (d->copy_stream) (void)hipStreamDestroy(d->copy_stream);
     if (d->stream) (void)hipStreamDestroy(d->stream);

@@ -130,6 +130,12 @@ struct blco_dev {
     uint64_t res_nnz = 0;
     uint64_t budget = 0;  // device bytes for nonzeros, slots and copies (0: no cap)
     uint64_t* h_coords = nullptr;
+    // a streamed tensor without a budget keeps its words packed instead
+    uint32_t* h_packed = nullptr;
+    std::vector<blco::PackChunk> pack_h;  // per fine chunk
+    blco::PackChunk* d_pack = nullptr;
+    uint32_t* slot_packed[2] = {nullptr, nullptr};
+    uint64_t slot_cap = 0, packed_cap = 0;  // nonzeros and packed dwords a slot holds
     void* h_vals = nullptr;
     uint64_t* slot_coords[2] = {nullptr, nullptr};
     void* slot_vals[2] = {nullptr, nullptr};

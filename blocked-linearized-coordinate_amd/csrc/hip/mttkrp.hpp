@@ -100,6 +100,11 @@ constexpr uint32_t WINDOW_LDS_BYTES = 40 * 1024;  // hot area + row window per w
 constexpr int WIN_WAVES = 8;                      // waves per row-window workgroup
 constexpr int WIN_BATCH = 4;                      // positions whose gathers are issued together
 
+// Field positions of a tensor's words, as a kernel argument.
+struct BlcoPos {
+    int p[BLCO_MAX_MODES];
+};
+
 // Marks a reduce segment whose output row is split over several segments.
 constexpr uint64_t REDUCE_SHARED = 1ull << 63;
 

@@ -129,4 +129,26 @@ void build_blocks(const Layout& L, uint64_t nnz, const uint64_t* hi, uint64_t mb
 // start[0] = 0) and has upper half hival[r] (hival may be nullptr: 0).
 void build_blocks_runs(const Layout& L, uint64_t nnz, uint64_t nruns, const uint64_t* start, const uint64_t* hival,
                        uint64_t mbs, blco_host* h);
+// A fine chunk's words as they cross the host link of a streamed tensor: each
+// field less its smallest value in the chunk, bits[m] bits of it, the fields
+// side by side (width bits a nonzero, mode 0 lowest), from dword `at` of the
+// packed words.  Neighbours in ALTO order agree in their upper index bits, so
+// a chunk needs about as many bits as its share of the key space leaves.
+struct PackChunk {
+    uint64_t at;
+    uint64_t begin;  // first nonzero
+    uint64_t base;   // the word of the smallest fields
+    uint32_t len;
+    uint8_t bits[BLCO_MAX_MODES];
+    uint8_t width;
+};
+// The chunks' forms (and one more entry, whose `at` is the dword count), the
+// dwords and the widest width.  False when the fields overlap or packing
+// saves less than a byte per nonzero: the words stay as they are.
+bool pack_words(int nmodes, const uint64_t* masks, const int* pos, uint64_t nnz, const uint64_t* coords,
+                const std::vector<uint64_t>& fbeg, const std::vector<uint32_t>& flen, std::vector<PackChunk>* chunks,
+                uint64_t* dwords, uint32_t* widest);
+void write_packed(int nmodes, const uint64_t* masks, const int* pos, const uint64_t* coords,
+                  const std::vector<PackChunk>& chunks, uint32_t* out);
+
 }  // namespace blco
