@@ -11,7 +11,8 @@
 //              the f64 form D[l/16 + 4*v][l%16] (checked on the hardware).  Per-workgroup partial Grams are
 //              summed in a fixed order (deterministic).  Optionally the same
 //              pass forms the fit inner products sum_i U_ir M_ir.
-//   factorize  one workgroup: V = prod_{m != n} G_m (Hadamard), lower
+//   factorize  one workgroup: V = prod_{m != n} G_m (Hadamard), for R <= 32
+//              V = L D L^T and L^{-1} in one wave's registers, else lower
 //              Cholesky in LAPACK dpotf2 order in LDS; when a pivot falls to
 //              R * eps * max V_ii or below, cyclic Jacobi eigendecomposition
 //              of V and the pseudo-inverse V^+ = Q diag(1/w) Q^T with

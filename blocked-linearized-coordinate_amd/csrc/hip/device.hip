@@ -5,9 +5,10 @@
 // one contiguous allocation each, blocks back to back (block b occupies
 // [block_start[b], block_start[b] + block_nnz[b])); block coordinates
 // u64[nblocks][nmodes]; a chunk table per tiles-per-wave setting (one entry
-// per wave of work: begin, length, block).  Streamed tensors keep coords and
-// values in pinned host memory and pass them through two device slots of
-// slot_nnz nonzeros, copying on a side stream while the previous slot is
+// per wave of work: begin, length, block).  Streamed tensors keep words (packed,
+// host/pack.cpp, unless a device budget keeps part of them resident) and
+// values in pinned host memory and pass them through two device slots of at
+// most slot_nnz nonzeros, copying on a side stream while the previous slot is
 // being consumed (src/alto_dev.cu:1869-1874, 1987 stream one block per
 // launch through NUM_STREAMS slots).
 #include <sys/stat.h>
@@ -915,7 +916,10 @@ static size_t plan_rows(blco_dev* d, int mode, int rank, int ftype, bool fib, Mt
     return lds;
 }
 
-// The words of fine chunks from their packed form, a workgroup per chunk.
+// The words of fine chunks from their packed form, a workgroup per chunk: a
+// thread cuts its word's bits out of three dwords (neighbours share lines) and
+// adds the chunk's minima back.  Bound by the stores, 8 bytes a nonzero at HBM
+// rate, against the link's 4 to 8 bytes at 57 GB/s: hidden behind the copies.
 __global__ __launch_bounds__(WG) void k_unpack(const PackChunk* __restrict__ pack, uint64_t first_dword,
                                                uint64_t first_nz, const uint32_t* __restrict__ packed, BlcoPos pos,
                                                int nmodes, uint64_t* __restrict__ coords)

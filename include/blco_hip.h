@@ -325,9 +325,10 @@ int blco_batch_mttkrp(blco_batch* b, int mode, int rank, int factor_dtype,
                       void* const* factors, void* const* outs, int tpw,
                       int waves, int wgs_per_cu);
 /* CP-ALS of every tensor (cpals_blco_dev semantics per tensor, modes
- * 0..N-1): per mode one persistent MTTKRP for the whole batch, the ALS steps
- * of all tensors on their own streams, and after iteration 0 the sweep
- * replayed as one captured hipGraph.  U (host f64, U[t * BLCO_MAX_MODES + m],
+ * 0..N-1): per mode one MTTKRP launch for the whole batch (over row-ordered
+ * copies, built on first use; the persistent kernel where one does not fit),
+ * one update and one finish launch for all tensors, and after iteration 0 the
+ * sweep replayed as one captured hipGraph.  U (host f64, U[t * BLCO_MAX_MODES + m],
  * dims x rank) holds the initial factors and receives the results; lambda
  * (t * rank + r), fits[t] and iters[t] (may be NULL) receive each tensor's
  * result at its own stopping iteration.  *iter_ms: mean device time of one
