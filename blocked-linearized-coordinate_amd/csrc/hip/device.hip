@@ -678,16 +678,23 @@ static int ensure_row_ordered(blco_dev* d, int mode, int rank, int ftype)
 // chunks are shorter: it has waves enough so, and every piece ends in one add
 // per column to the same output row, which queue up (13 ns each) and, in
 // FP32, add their roundings (86,000 pieces of 128 nonzeros of one row: error
-// 1.6e-6 against 64 bits, 7,000 of 1500: 8e-7).  A tiled
+// 1.6e-6 against 64 bits, 7,000 of 1500: 8e-7).  Below 2^21 nonzeros the
+// pieces shrink to a PIECE_WAVES-th of the tensor, or the waves that hold them
+// run on alone: 2M nonzeros at rank 64, a row of 220,000, 147 us with pieces of
+// 2048, 92 of 1024, 88 of 256 (the last with an error of 3.8e-7 against 1.8e-7).
+// A tiled
 // copy pads every tile's chunk list with empty chunks to one common length, a
 // multiple of the waves per workgroup: the grid then has NUM_XCD equal ranges
 // of workgroups and the XCD-contiguous workgroup numbering puts tile t on XCD t.
-constexpr uint64_t LONG_ROW = 32768, LONG_PIECE = 2 * WAVE * SORTED_TPW;
+constexpr uint64_t LONG_ROW = 32768, LONG_PIECE = 2 * WAVE * SORTED_TPW, PIECE_WAVES = 1024;
 
 static std::vector<Chunk> sorted_chunks(const blco_dev* d, int mode, int tpw)
 {
     const uint64_t base = (uint64_t)WAVE * tpw, cap = 2 * base;
     const int ntiles = std::max(1, d->stiles[mode]);
+    uint64_t long_piece = LONG_PIECE;
+    while (long_piece > cap && long_piece * PIECE_WAVES > d->nnz) long_piece /= 2;
+    long_piece = std::max(long_piece, cap);
     std::vector<std::vector<Chunk>> tiles(ntiles);
     const std::vector<uint64_t>& runs = d->srun_h[mode];
     size_t r = 0;
@@ -702,7 +709,7 @@ static std::vector<Chunk> sorted_chunks(const blco_dev* d, int mode, int tpw)
             const uint64_t run_end = (r + 1 < runs.size()) ? std::min(runs[r + 1], end) : end;
             if (run_end - c0 > cap) {  // inside a long row
                 const uint64_t run_len = run_end - std::max(runs[r], g.start);
-                const uint64_t piece = run_len >= LONG_ROW ? std::max(cap, LONG_PIECE) : cap;
+                const uint64_t piece = run_len >= LONG_ROW ? long_piece : cap;
                 const uint64_t end_piece = std::min(c0 + piece, run_end);
                 emit(c0, end_piece);
                 c0 = end_piece;
@@ -723,7 +730,7 @@ static std::vector<Chunk> sorted_chunks(const blco_dev* d, int mode, int tpw)
         }
     }
     std::vector<Chunk> h;
-    if (ntiles == 1 && cap < LONG_PIECE) {
+    if (ntiles == 1 && cap < long_piece) {
         // the pieces of long rows hold many times the nonzeros of the other
         // chunks and lie together: they go to the XCDs with the fewest
         // nonzeros, ahead of each one's equal share of the rest
