@@ -859,12 +859,14 @@ size_t rows_kernel_plan(blco_dev* d, int mode, int rank, int ftype, bool fib, Mt
 }
 
 // k_mttkrp_rows takes one chunk per wave and keeps no windows.  The windowed
-// kernel (k_mttkrp_rows_lds) is slower wherever both were timed since the
-// former gathers with wide stream loads and coalesced adds: 40M nonzeros with
+// kernel (k_mttkrp_rows_lds) is slower, except in FP64 on 1.7B nonzeros of the
+// 4.8M-row shape in fiber order (42.4 / 43.4 / 43.5 ms with windows, 50.0 / 49.8 /
+// 49.6 without; FP32 24.1 / 24.7 / 24.4 and 22.6 / 22.6 / 22.4), since the former
+// gathers with wide stream loads and coalesced adds: 40M nonzeros with
 // Zipf(1.2) modes, FP32 rank 32, 821 / 840 / 667 us with windows and 574 /
 // 577 / 531 without, FP64 rank 16 1003 / 1020 / 761 and 628 / 634 / 622; the
 // 4.8M-row shape at 85M nonzeros 2360 / 1899 / 1880 and 1420 / 1398 / 1399.
-// It runs only where BLCO_FIBERS forces a form.  There the windows cover, for
+// It runs only where BLCO_FIBERS forces a form (=1 for that FP64 shape).  There the windows cover, for
 // the first two input modes (the inner and first outer mode with fibers, 2/3
 // and 1/3 of HOT_TABLE_BYTES' rows; else halves), the mode's consecutive rows
 // with the most nonzeros; a window that would hold fewer than 2% of the
