@@ -802,10 +802,26 @@ static int launch_range(blco_dev* d, int which, MttkrpArgs a, const ChunkTab* t,
     uint32_t grid;
     size_t lds = 0;
     if (which == W_LVL3 || which == W_LVL3_ROWS) {
-        // about 1024 workgroups, of at least one chunk a wave
-        a.chunks_per_wg = std::min(LVL3_CHUNKS_PER_WG, std::max<uint32_t>(WAVES_PER_WG, a.nchunks / 1024));
+        // through the row gathers: in FP64 about 1024 workgroups, of at least
+        // one chunk a wave; with floats in the output 16 (a whole tensor's), or
+        // as many as the chunks make at LVL3_CHUNKS_PER_WG each (lvl3_wg)
+        a.chunks_per_wg = LVL3_CHUNKS_PER_WG;
+        const bool f64 = ftype == BLCO_F64;
+        if (which == W_LVL3_ROWS && (f64 || a.nchunks == t->n)) {
+            const uint32_t waves = lvl3_wg(f64) / WAVE;
+            a.chunks_per_wg = std::min(LVL3_CHUNKS_PER_WG, std::max(waves, a.nchunks / (f64 ? 1024 : 16)));
+        }
         grid = (a.nchunks + a.chunks_per_wg - 1) / a.chunks_per_wg;
-        lds = d->dims[a.mode] * (uint64_t)a.rank * (ftype == BLCO_F64 ? 8 : 4);
+        if (which == W_LVL3_ROWS) {
+            // modes of few rows get several copies, or a wave's slots meet in
+            // the same row
+            const uint32_t rows = (uint32_t)d->dims[a.mode];
+            lds = sizeof(double) * lvl3_copy_stride(rows, a.rank);
+            a.lvl3_copies = std::max<uint32_t>(1, std::min<uint32_t>(16 / rows, (uint32_t)(LDS_OUT_MAX / lds)));
+            lds *= a.lvl3_copies;
+        } else {
+            lds = d->dims[a.mode] * (uint64_t)a.rank * (ftype == BLCO_F64 ? 8 : 4);
+        }
     } else {
         grid = (a.nchunks + WAVES_PER_WG - 1) / WAVES_PER_WG;
     }

@@ -133,7 +133,9 @@ int launch_mttkrp(int which, const MttkrpArgs& a, int ftype, uint32_t grid, size
     if (!k) return fail(BLCO_EUNSUPPORTED, "no MTTKRP kernel for %d modes, rank %d", a.nmodes, a.rank);
     MttkrpArgs args = a;
     void* params[] = {&args};
-    const int block = (which == W_WINDOW || which == W_WINDOW64) ? WIN_WAVES * WAVE : WG;
+    const int block = which == W_WINDOW || which == W_WINDOW64 ? WIN_WAVES * WAVE
+                      : which == W_LVL3_ROWS                  ? lvl3_wg(ftype == BLCO_F64)
+                                                              : WG;
     if (dyn_lds > 64 * 1024)
         HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn_lds));
     hipError_t e = hipLaunchKernel(k, dim3(grid), dim3(block), params, dyn_lds, st);

@@ -67,6 +67,8 @@ struct MttkrpArgs {
     int inner;
     // k_mttkrp_rows: the input modes in gather order, then the output mode
     int order[BLCO_MAX_MODES];
+    // k_mttkrp_lvl3_rows: copies of the output in LDS, slot s adds to s mod this
+    uint32_t lvl3_copies;
     // row-ordered kernels: chunks per wave (consecutive, or with
     // cpw_interleave one grid width apart), and for the first two input
     // modes (the inner and first outer mode with fibers) a window of rows
@@ -89,6 +91,23 @@ struct RowsPlan {
 enum { W_LVL1 = 0, W_LVL3 = 1, W_ATOMIC = 2, W_WINDOW = 3, W_WINDOW64 = 4, W_SORTED64 = 5, W_FIBER64 = 6,
        W_SORTED_LDS = 7, W_FIBER_LDS = 8, W_ROWS = 9, W_ROWS_SHORT = 10, W_ROWS_BATCH = 11,
        W_LVL3_ROWS = 12 };
+
+// Threads of a workgroup of k_mttkrp_lvl3_rows.  Every workgroup ends in one
+// add to each output element, and in FP32 each of those rounds: with floats in
+// the output a workgroup takes 64 chunks (16384 nonzeros, as many adds as the
+// tile-sorting kernel), and 16 waves to run them.  Workgroups of 1024 nonzeros
+// ran 300k nonzeros into 24 rows with an error of 2.6e-7 against 64 bits,
+// these 18 run it with 6.9e-8 (8.2e-8 with sorted tiles and sums in floats).
+constexpr int lvl3_wg(bool f64) { return f64 ? 4 * 64 : 16 * 64; }
+
+// Doubles from row to row and from copy to copy of k_mttkrp_lvl3_rows' output in
+// LDS: odd, so that the slots of a wave, which add to different rows, spread
+// over the banks (at rank 32 and a stride of 32 all of them met in 16 of 64).
+constexpr __host__ __device__ uint32_t lvl3_row_stride(int rank) { return (uint32_t)rank | 1; }
+constexpr __host__ __device__ uint32_t lvl3_copy_stride(uint32_t rows, int rank)
+{
+    return rows * lvl3_row_stride(rank) | 1;
+}
 
 // The row-ordered and fiber kernels take 31-bit byte offsets into factors
 // of fewer bytes than this (bit 31 marks an offset into an LDS window).

@@ -1178,13 +1178,18 @@ __global__ __launch_bounds__(WG) void k_mttkrp_rows_batch(const MttkrpArgs* __re
 
 // lvl3 for factors of fewer than FACTOR_BYTES_MAX bytes: rounds, gathers and
 // broadcasts as in rows_chunk over chunks in ALTO order; each product goes
-// straight to the workgroup's copy of the output in LDS (one LDS add per
-// element, about an eighth of what its gathers cost), without sorting tiles.
-// 3.3M nonzeros into 24 rows, FP64 rank 10: 635 us with sorted tiles,
+// straight to the workgroup's copies of the output in LDS, without sorting
+// tiles.  They hold doubles for every factor type: ds_add_f64 takes about
+// an eighth of the time of its gathers, ds_add_f32 four times as long as
+// ds_add_f64 (20M nonzeros into 24 rows, rank 32, FP32: 415 us, 3300 with
+// floats, 1467 with sorted tiles; rank 10: 217, 1036, 839), and a chain of
+// 16384 floats loses what the tiles' partial sums kept.
+// 3.3M nonzeros into 24 rows, FP64 rank 10: 58 us, 516 with sorted tiles,
 // single-element gathers and 202 workgroups.
 template <int N, typename FT, typename VT, int C, int L, int Q>
-__global__ __launch_bounds__(WG) void k_mttkrp_lvl3_rows(MttkrpArgs a)
+__global__ __launch_bounds__(lvl3_wg(std::is_same<FT, double>::value)) void k_mttkrp_lvl3_rows(MttkrpArgs a)
 {
+    constexpr int LVL3_WG = lvl3_wg(std::is_same<FT, double>::value);
     using AT = typename Acc<FT>::type;
     constexpr int S = WAVE / L;
     constexpr int P = L * Q;
@@ -1194,14 +1199,15 @@ __global__ __launch_bounds__(WG) void k_mttkrp_lvl3_rows(MttkrpArgs a)
     constexpr int LS = PB / KS;
     constexpr uint32_t NONE = 0x80000000u;
     extern __shared__ __align__(16) unsigned char s_dyn[];
-    AT* s_out = reinterpret_cast<AT*>(s_dyn);
+    double* s_out = reinterpret_cast<double*>(s_dyn);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int R = a.rank;
-    const uint32_t cells = (uint32_t)(a.out_rows * (uint64_t)R);
-    for (uint32_t e = threadIdx.x; e < cells; e += WG) s_out[e] = 0;
+    const uint32_t rows = (uint32_t)a.out_rows, stride = lvl3_row_stride(R), copy = lvl3_copy_stride(rows, R);
+    for (uint32_t e = threadIdx.x; e < copy * a.lvl3_copies; e += LVL3_WG) s_out[e] = 0;
     __syncthreads();
     const uint32_t row_bytes = (uint32_t)R * (uint32_t)sizeof(FT);
     const int slot = lane / L, sub = lane % L;
+    double* s_mine = s_out + (slot % a.lvl3_copies) * copy;
     __amdgpu_buffer_rsrc_t rs[N - 1];
     uint64_t mk[N];
     int ps[N];
@@ -1214,7 +1220,7 @@ __global__ __launch_bounds__(WG) void k_mttkrp_lvl3_rows(MttkrpArgs a)
     }
     const uint32_t cbeg = a.chunk0 + blockIdx.x * a.chunks_per_wg;
     const uint32_t cend = min(cbeg + a.chunks_per_wg, a.chunk0 + a.nchunks);
-    for (uint32_t c = cbeg + w; c < cend; c += WAVES_PER_WG) {
+    for (uint32_t c = cbeg + w; c < cend; c += LVL3_WG / WAVE) {
         const Chunk ch = a.chunks[c];
         uint32_t bc[N];
         #pragma unroll
@@ -1251,7 +1257,7 @@ __global__ __launch_bounds__(WG) void k_mttkrp_lvl3_rows(MttkrpArgs a)
                     #pragma unroll
                     for (int j = 0; j < N - 1; ++j)
                         off[k][j] = valid ? ((uint32_t)((word[k] >> ps[j]) & mk[j]) | bc[j]) * row_bytes : NONE;
-                    cell[k] = valid ? ((uint32_t)((word[k] >> ps[N - 1]) & mk[N - 1]) | bc[N - 1]) * (uint32_t)R : NONE;
+                    cell[k] = valid ? ((uint32_t)((word[k] >> ps[N - 1]) & mk[N - 1]) | bc[N - 1]) * stride : NONE;
                     v[k] = valid ? (AT)val[k] : (AT)0;
                 }
                 unrolled<L / LS>([&](auto g) {
@@ -1282,7 +1288,7 @@ __global__ __launch_bounds__(WG) void k_mttkrp_lvl3_rows(MttkrpArgs a)
                                         for (int j = 0; j < N - 1; ++j) t *= x[s * KS + k][j][cc];
                                         // columns that this lane repeats belong to the lane before
                                         if (at != NONE && c0 + cc >= sub * C)
-                                            atomic_add_lds(s_out + at + cb + c0 + cc, t);
+                                            atomic_add_lds(s_mine + at + cb + c0 + cc, (double)t);
                                     }
                                 }
                             });
@@ -1294,9 +1300,12 @@ __global__ __launch_bounds__(WG) void k_mttkrp_lvl3_rows(MttkrpArgs a)
     }
     __syncthreads();
     AT* dst = reinterpret_cast<AT*>(a.nprtn > 1 ? a.partials : a.out);
-    if (a.nprtn > 1) dst += (uint64_t)(blockIdx.x % (uint32_t)a.nprtn) * cells;
-    for (uint32_t e = threadIdx.x; e < cells; e += WG) {
-        const AT v = s_out[e];
+    if (a.nprtn > 1) dst += (uint64_t)(blockIdx.x % (uint32_t)a.nprtn) * rows * R;
+    for (uint32_t e = threadIdx.x; e < rows * R; e += LVL3_WG) {
+        const uint32_t at = e / R * stride + e % R;
+        double t = s_out[at];
+        for (uint32_t k = 1; k < a.lvl3_copies; ++k) t += s_out[k * copy + at];
+        const AT v = (AT)t;
         if (v != (AT)0) atomic_add_global(dst + e, v);
     }
 }
