@@ -43,26 +43,21 @@ constexpr uint32_t HOT_EXCLUDE = 64;  // hot rows kept out of the row windows
 
 static int value_size(int vdt) { return vdt == BLCO_F64 ? 8 : 4; }
 
-// Default tiles of 64 nonzeros per chunk of the row-ordered kernel.  A chunk
-// of 2 tiles runs in one or two rounds of the kernel: the most waves and the
-// closest neighbours in L1.  Longer chunks pay where a chunk's end, which
-// adds its open row to HBM, is dear: rows of more than 128 bytes (FP64 at
-// rank 32: 2055 / 2130 us with 2 tiles, 1506 / 1522 with 16 on the
-// 77M-nonzero modes), and for tensors from 2^22 nonzeros hot rows whose adds
-// queue up (nnz * hot / (64 tpw) adds of 13 ns each to one row: 401 rows of a
-// Zipf(0.8) mode at 34M nonzeros 671 us with 2 tiles, 560 with 8).  FP32 at
-// rank 32: 1221 / 1162 / 1164 us with 2 tiles and 1298 / 1273 / 1274 with 16
-// on the 4.8M-row shape at 85M nonzeros, 820 / 820 / 778 and 819 / 811 / 785
-// on the 77M-nonzero modes, 81 and 141 for 2M nonzeros at rank 64.
+// Default tiles of 64 nonzeros per chunk of k_mttkrp_rows.  A chunk of 2 tiles
+// runs in one or two rounds of the kernel: the most waves and the closest
+// neighbours in L1.  Longer chunks pay only where a chunk's end, which adds its
+// open row to HBM, is dear and seldom another row's end too: output rows of
+// more than 128 bytes and of a thousand nonzeros or so.  Times in us with 2, 8
+// and 16 tiles, FP64 at rank 32: 77M nonzeros over 12,092 rows 1583, 1512, 1506;
+// 200M over 2M rows 5381, 6086, 6820, over 600,000 rows 6088, 6149, 7451; 1.7B
+// over 4.8M rows 41938, 43263, 49704.  FP32 at rank 32: 77M 806, 798, 819; 1.7B
+// 20162, 19915, 22797.  Hot rows do not need them: their pieces are long at any
+// setting (LONG_ROW).
 static int sorted_tpw(const blco_dev* d, int mode, int rank, int ftype)
 {
     if (d->nnz < (1ull << 17)) return 1;  // 100k nonzeros: 5.4 us with 1, 6.3 with 2
-    if (d->nnz < (1ull << 22)) return 2;
-    const uint64_t row_bytes = (uint64_t)rank * (ftype == BLCO_F64 ? 8 : 4);
-    const uint64_t hottest = d->hot_cnt_h[mode].empty() ? 0 : d->hot_cnt_h[mode][0];
-    int t = row_bytes > 128 ? 8 : 2;
-    while (t < SORTED_TPW && hottest * row_bytes > (uint64_t)t * (2ull << 20) * 128) t *= 2;
-    return t;
+    if (d->nnz < (1ull << 22) || (uint64_t)rank * (ftype == BLCO_F64 ? 8 : 4) <= 128) return 2;
+    return d->nnz / 1024 < d->srun_h[mode].size() - 1 ? 2 : ROWS_LONG_TPW;
 }
 
 // Nonzeros of one streamed unit: a quarter of the tensor where that is below
@@ -875,14 +870,14 @@ size_t rows_kernel_plan(blco_dev* d, int mode, int rank, int ftype, bool fib, Mt
 }
 
 // k_mttkrp_rows takes one chunk per wave and keeps no windows.  The windowed
-// kernel (k_mttkrp_rows_lds) is slower, except in FP64 on 1.7B nonzeros of the
-// 4.8M-row shape in fiber order (42.4 / 43.4 / 43.5 ms with windows, 50.0 / 49.8 /
-// 49.6 without; FP32 24.1 / 24.7 / 24.4 and 22.6 / 22.6 / 22.4), since the former
-// gathers with wide stream loads and coalesced adds: 40M nonzeros with
-// Zipf(1.2) modes, FP32 rank 32, 821 / 840 / 667 us with windows and 574 /
-// 577 / 531 without, FP64 rank 16 1003 / 1020 / 761 and 628 / 634 / 622; the
-// 4.8M-row shape at 85M nonzeros 2360 / 1899 / 1880 and 1420 / 1398 / 1399.
-// It runs only where BLCO_FIBERS forces a form (=1 for that FP64 shape).  There the windows cover, for
+// kernel (k_mttkrp_rows_lds), which gathers an outer row once per fiber but adds
+// every row with its slot's lanes, is slower or within 2% on every shape timed:
+// FP64 at rank 32 in fiber order, 1.7B nonzeros of the 4.8M-row shape 42.4 /
+// 43.4 / 43.5 ms against 41.9 / 43.1 / 43.5, 340M 11.1 / 9.8 / 9.9 against 9.1 /
+// 8.8 / 8.8, 85M 4.5 / 3.8 / 3.9 against 2.8 / 2.6 / 2.6; FP32 at rank 32, 1.7B
+// 24.1 / 24.7 / 24.4 against 20.2; rank 64, 340M 10.7 / 8.7 / 8.7 against 8.7 /
+// 8.2 / 8.2.  It
+// runs only where BLCO_FIBERS forces a form.  There the windows cover, for
 // the first two input modes (the inner and first outer mode with fibers, 2/3
 // and 1/3 of HOT_TABLE_BYTES' rows; else halves), the mode's consecutive rows
 // with the most nonzeros; a window that would hold fewer than 2% of the
@@ -1132,7 +1127,7 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
             break;
         default: return fail(BLCO_EINVAL, "unknown kernel id %d", kernel);
     }
-    if (tpw <= 0) tpw = which == W_ROWS ? sorted_tpw(d, mode, rank, ftype) : DEFAULT_TPW;
+    if (tpw <= 0 && which != W_ROWS) tpw = DEFAULT_TPW;
     if (used_kernel) *used_kernel = kernel;
     if (d->nnz == 0) return BLCO_OK;
     if (which == W_ROWS) {
@@ -1270,6 +1265,7 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
         a.coords = d->d_scoords[mode];
         a.vals = d->d_svals[mode];
         a.coord_base = 0;
+        if (tpw <= 0) tpw = sorted_tpw(d, mode, rank, ftype);
         const ChunkTab* stab = sorted_chunk_table(d, mode, tpw);
         if (!stab) return BLCO_ENOMEM;
         const bool wide = !narrow_factors(d, rank, ftype);

@@ -57,3 +57,37 @@ def test_infinities_stay_in_their_rows(B, O, gpu):
         assert np.all(np.isinf(got[hit])) and np.all(np.isfinite(got[~hit]))
         assert np.linalg.norm(got[~hit] - want[~hit]) <= 2e-6 * np.linalg.norm(want[~hit])
     dev.free()
+
+
+@pytest.mark.parametrize("rank,dtype", [(32, 0), (33, 1), (32, 1)])
+def test_default_chunk_lengths_of_large_tensors(B, O, gpu, rank, dtype):
+    """Just past 2^22 nonzeros: output rows of more than 128 bytes in a mode
+    of many rows (chunks of 2 tiles) and in modes of long ones (8 tiles, the
+    kernel's long rounds), a most frequent row of over 32768 nonzeros (pieces
+    of 2048), and 128-byte rows (2 tiles everywhere)."""
+    dims, nnz = (100_000, 1500, 900), (1 << 22) + 4321
+    t = B.Coo.generate(dims, nnz, zipf=(0.3, 1.1, 0.0), gen_rank=4, seed=22, topup=True)
+    assert t.nnz == nnz and np.bincount(t.cidx[1].astype(int)).max() > 32768
+    at = O.Alto(dims, t.cidx, t.vals, nprtn=8)
+    dev = B.DeviceTensor(B.encode(t), value_dtype=B.F64 if dtype == 0 else B.F32)
+    U = [np.random.default_rng(m).random((d, rank)) for m, d in enumerate(dims)]
+    for m in range(3):
+        got, held = mttkrp(B, dev, U, m, dtype, 0)
+        want = at.mttkrp(held, m)
+        e = np.linalg.norm(got - want) / np.linalg.norm(want)
+        assert e <= TOL[dtype], (rank, dtype, m, e)
+    dev.free()
+
+
+def test_default_chunk_length_with_a_hot_row(B, gpu):
+    """A very frequent row (7% of 165M nonzeros) lengthens no chunks: the
+    default runs within 10% of the best of 2 and 8 tiles (16 tiles: 22% more)."""
+    dims, rank = (600_000, 400_000, 500_000), 32
+    dev = B.DeviceTensor.generate(dims, 165_000_000, zipf=(1.0, 1.0, 1.0), gen_rank=20, value_kind=1,
+                                  seed=1005, topup=True)
+    F = [B.DeviceArray((d, rank)) for d in dims]
+    out = B.DeviceArray((dims[1], rank))
+    ms = {tpw: min(B.mttkrp_time(dev, 1, rank, F, out, kernel=B.K_SORTED, reps=3, thread_cf=tpw)[0] for _ in range(3))
+          for tpw in (0, 2, 8)}
+    dev.free()
+    assert ms[0] <= 1.1 * min(ms[2], ms[8]), ms
