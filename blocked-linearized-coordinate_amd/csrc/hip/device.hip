@@ -36,12 +36,25 @@ constexpr uint64_t LDS_OUT_MAX = 48 * 1024;
 constexpr int LVL3_MAX_MODE_LENGTH = 100;     // src/utils.hpp:13
 constexpr int DEFAULT_TPW = 4;                // tiles of 64 per wave
 constexpr int SORTED_TPW = 16;                // tiles of 64 per wave, row-ordered kernel (most)
+constexpr uint64_t SORTED_TARGET_CHUNKS = 8192;
 constexpr int ROWS_LONG_TPW = 8;              // chunks from here on take k_mttkrp_rows' long rounds
 constexpr int DEFAULT_NPRTN = 1;
 constexpr uint32_t LVL3_CHUNKS_PER_WG = 64;  // at most
 constexpr uint32_t HOT_EXCLUDE = 64;  // hot rows kept out of the row windows
 
 static int value_size(int vdt) { return vdt == BLCO_F64 ? 8 : 4; }
+
+// Tiles of 64 nonzeros per chunk that leave 4096-8192 chunks of a tensor of up
+// to 2^22 nonzeros, and 16 from there on; 32 for FP64 rows of 256 bytes or more
+// from 2^26 nonzeros.  What the kernels that add a row with its slot's lanes
+// were timed with: fewer chunk ends, each of which adds its open rows to HBM.
+static int long_tpw(const blco_dev* d, int rank, int ftype)
+{
+    if (ftype == BLCO_F64 && rank >= 32 && d->nnz >= (1ull << 26)) return 32;
+    int t = 2;
+    while (t < SORTED_TPW && d->nnz > (uint64_t)WAVE * t * SORTED_TARGET_CHUNKS) t *= 2;
+    return t;
+}
 
 // Default tiles of 64 nonzeros per chunk of k_mttkrp_rows.  A chunk of 2 tiles
 // runs in one or two rounds of the kernel: the most waves and the closest
@@ -658,6 +671,7 @@ static int ensure_row_ordered(blco_dev* d, int mode, int rank, int ftype)
     d->stiles[mode] = ntiles;
     d->sinner[mode] = inner;
     d->sfiber[mode] = use_fibers;
+    d->sforced[mode] = fenv != nullptr;
     d->sgrp_h[mode].swap(groups);
     d->srun_h[mode].swap(runs);
     static std::atomic<uint64_t> copies{0};
@@ -823,7 +837,7 @@ static int launch_range(blco_dev* d, int which, MttkrpArgs a, const ChunkTab* t,
     return launch_mttkrp(which, a, ftype, grid, lds, st);
 }
 
-static size_t plan_rows(blco_dev* d, int mode, int rank, int ftype, bool fib, MttkrpArgs* a);
+static size_t plan_rows(blco_dev* d, int mode, int rank, int ftype, MttkrpArgs* a);
 
 // The best window of h consecutive rows of mode m (most nonzeros); its
 // start, and its nonzero count in *covered.
@@ -849,12 +863,13 @@ static uint64_t best_window(blco_dev* d, int m, uint64_t h, uint64_t* covered)
 }
 
 // Chunks per wave and the LDS windows of hot rows for the row-ordered
-// kernels (k_mttkrp_rows), into a; returns the dynamic LDS bytes.  Cached
-// per (mode, rank, factor type, form, chunk count).
-size_t rows_kernel_plan(blco_dev* d, int mode, int rank, int ftype, bool fib, MttkrpArgs* a)
+// kernels, into a (one chunk and no windows unless `windows` asks for them);
+// returns the dynamic LDS bytes.  Cached per (mode, rank, factor type, windows,
+// chunk count).
+size_t rows_kernel_plan(blco_dev* d, int mode, int rank, int ftype, bool windows, MttkrpArgs* a)
 {
     for (const RowsPlan& p : d->rows_plans[mode])
-        if (p.rank == rank && p.ftype == ftype && p.fib == fib && p.nchunks == a->nchunks) {
+        if (p.rank == rank && p.ftype == ftype && p.windows == windows && p.nchunks == a->nchunks) {
             a->cpw = p.cpw;
             a->cpw_interleave = p.interleave;
             for (int t = 0; t < 2; ++t) {
@@ -863,8 +878,12 @@ size_t rows_kernel_plan(blco_dev* d, int mode, int rank, int ftype, bool fib, Mt
             }
             return p.lds;
         }
-    const size_t lds = plan_rows(d, mode, rank, ftype, fib, a);
-    d->rows_plans[mode].push_back(RowsPlan{rank, ftype, fib, a->nchunks, a->cpw, a->cpw_interleave,
+    a->cpw = 1;
+    a->cpw_interleave = 0;
+    a->hot_lo[0] = a->hot_lo[1] = 0;
+    a->hot_n[0] = a->hot_n[1] = 0;
+    const size_t lds = windows ? plan_rows(d, mode, rank, ftype, a) : 0;
+    d->rows_plans[mode].push_back(RowsPlan{rank, ftype, windows, a->nchunks, a->cpw, a->cpw_interleave,
                                            {a->hot_lo[0], a->hot_lo[1]}, {a->hot_n[0], a->hot_n[1]}, lds});
     return lds;
 }
@@ -876,26 +895,21 @@ size_t rows_kernel_plan(blco_dev* d, int mode, int rank, int ftype, bool fib, Mt
 // 43.4 / 43.5 ms against 41.9 / 43.1 / 43.5, 340M 11.1 / 9.8 / 9.9 against 9.1 /
 // 8.8 / 8.8, 85M 4.5 / 3.8 / 3.9 against 2.8 / 2.6 / 2.6; FP32 at rank 32, 1.7B
 // 24.1 / 24.7 / 24.4 against 20.2; rank 64, 340M 10.7 / 8.7 / 8.7 against 8.7 /
-// 8.2 / 8.2.  It
-// runs only where BLCO_FIBERS forces a form.  There the windows cover, for
-// the first two input modes (the inner and first outer mode with fibers, 2/3
-// and 1/3 of HOT_TABLE_BYTES' rows; else halves), the mode's consecutive rows
-// with the most nonzeros; a window that would hold fewer than 2% of the
-// nonzeros is left out.  A workgroup fills its windows once, so its waves
-// take several chunks (as many as leave 1024 workgroups, at least half of the
-// cap): up to 4 consecutive ones each in the plain form, for rows of at most
-// 128 bytes; in the fiber form up to 8, with the grid walking the chunks in
-// step (chunk j of a wave is j grid widths on), and only when the inner
-// window holds a fifth of the nonzeros and the copy is not split into XCD
-// tiles.
-static size_t plan_rows(blco_dev* d, int mode, int rank, int ftype, bool fib, MttkrpArgs* a)
+// 8.2 / 8.2.  It runs on copies whose order BLCO_FIBERS forced (tests).  There
+// the windows cover, for the first two input modes (the inner and first outer
+// mode with fibers, 2/3 and 1/3 of HOT_TABLE_BYTES' rows; else halves), the
+// mode's consecutive rows with the most nonzeros; a window that would hold
+// fewer than 2% of the nonzeros is left out.  A workgroup fills its windows
+// once, so its waves take several chunks (as many as leave 1024 workgroups, at
+// least half of the cap): up to 4 consecutive ones each in the plain form, for
+// rows of at most 128 bytes; in the fiber form up to 8, with the grid walking
+// the chunks in step (chunk j of a wave is j grid widths on), and only when the
+// inner window holds a fifth of the nonzeros and the copy is not split into
+// XCD tiles.
+static size_t plan_rows(blco_dev* d, int mode, int rank, int ftype, MttkrpArgs* a)
 {
     const uint32_t n = a->nchunks;
-    a->cpw = 1;
-    a->cpw_interleave = 0;
-    a->hot_lo[0] = a->hot_lo[1] = 0;
-    a->hot_n[0] = a->hot_n[1] = 0;
-    if (!getenv("BLCO_FIBERS")) return 0;
+    const bool fib = d->sfiber[mode];
     const uint64_t row_bytes = (uint64_t)rank * dtype_size(ftype);
     // up to 8 (fibers) or 4 chunks per wave while 1024 workgroups remain
     const uint32_t cap = fib ? 8 : 4, fit = n / (1024u * WAVES_PER_WG);
@@ -1265,22 +1279,31 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
         a.coords = d->d_scoords[mode];
         a.vals = d->d_svals[mode];
         a.coord_base = 0;
-        if (tpw <= 0) tpw = sorted_tpw(d, mode, rank, ftype);
-        const ChunkTab* stab = sorted_chunk_table(d, mode, tpw);
-        if (!stab) return BLCO_ENOMEM;
-        const bool wide = !narrow_factors(d, rank, ftype);
         const bool fib = d->sfiber[mode];
         if (fib) a.inner = d->sinner[mode];
+        const bool wide = !narrow_factors(d, rank, ftype);
+        const ChunkTab* stab = nullptr;
+        size_t lds = 0;
+        if (!wide && d->sforced[mode]) {
+            stab = sorted_chunk_table(d, mode, tpw > 0 ? tpw : long_tpw(d, rank, ftype));
+            if (!stab) return BLCO_ENOMEM;
+            a.nchunks = stab->n;
+            lds = rows_kernel_plan(d, mode, rank, ftype, true, &a);
+        }
+        if (!lds) {
+            if (tpw <= 0) tpw = sorted_tpw(d, mode, rank, ftype);
+            stab = sorted_chunk_table(d, mode, tpw);
+            if (!stab) return BLCO_ENOMEM;
+        }
         if (wide) {
             rc = launch_range(d, fib ? W_FIBER64 : W_SORTED64, a, stab, 0, stab->n, ftype, st);
         } else if (stab->n) {
             a.chunks = stab->d;
             a.chunk0 = 0;
             a.nchunks = stab->n;
-            const size_t lds = rows_kernel_plan(d, mode, rank, ftype, fib, &a);
-            // the form with LDS windows only where the plan holds some
             int kind = fib ? W_FIBER_LDS : W_SORTED_LDS;
             if (!lds) {
+                rows_kernel_plan(d, mode, rank, ftype, false, &a);
                 kind = tpw >= ROWS_LONG_TPW ? W_ROWS : W_ROWS_SHORT;
                 gather_order(d, mode, a.order);
             }
@@ -1965,7 +1988,8 @@ int blco_dev_set_value_dtype(blco_dev* d, int value_dtype)
         d->sorted_failed[m] = false;
         d->stiles[m] = 0;
         d->sinner[m] = 0;
-        d->sfiber[m] = false;
+        d->sfiber[m] = d->sforced[m] = false;
+        d->rows_plans[m].clear();
     }
     d->sel_cache.clear();
     d->vdtype = value_dtype;

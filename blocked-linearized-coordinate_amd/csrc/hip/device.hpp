@@ -111,9 +111,9 @@ struct blco_dev {
     std::vector<blco::SGroup> sgrp_h[BLCO_MAX_MODES];
     int stiles[BLCO_MAX_MODES] = {};
     // fiber order of the copy: within a row by every input mode but sinner;
-    // sfiber: the fiber kernel runs on it (fibers long enough)
+    // sfiber: fibers long enough to gather by; sforced: BLCO_FIBERS chose the order
     int sinner[BLCO_MAX_MODES] = {};
-    bool sfiber[BLCO_MAX_MODES] = {};
+    bool sfiber[BLCO_MAX_MODES] = {}, sforced[BLCO_MAX_MODES] = {};
     std::vector<uint64_t> srun_h[BLCO_MAX_MODES];
     std::list<blco::ChunkTab> stabs[BLCO_MAX_MODES];  // row-aware chunks of the copy, per tpw
     // nonzeros per index of every mode, as prefix sums (dims + 1 entries),
@@ -182,6 +182,6 @@ int mttkrp_prepare(blco_dev* d, int mode, int rank, int ftype, int kernel);
 int rows_batch_prepare(blco_dev* d, int mode, int rank, int ftype);
 std::vector<Chunk> rows_batch_chunks(const blco_dev* d, int mode, int tpw);
 MttkrpArgs rows_batch_args(const blco_dev* d, int mode, int rank);
-size_t rows_kernel_plan(blco_dev* d, int mode, int rank, int ftype, bool fib, MttkrpArgs* a);
+size_t rows_kernel_plan(blco_dev* d, int mode, int rank, int ftype, bool windows, MttkrpArgs* a);
 
 }  // namespace blco

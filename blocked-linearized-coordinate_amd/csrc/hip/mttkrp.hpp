@@ -79,11 +79,11 @@ struct MttkrpArgs {
     uint32_t hot_n[2];
 };
 
-// Launch plan of a row-ordered kernel for one (rank, factor type, form,
+// Launch plan of a row-ordered kernel for one (rank, factor type, windows,
 // chunk count) of a mode: chunks per wave and the hot-row windows.
 struct RowsPlan {
     int rank, ftype;
-    bool fib;
+    bool windows;  // planned with windows, if any pay
     uint32_t nchunks, cpw, interleave, hot_lo[2], hot_n[2];
     size_t lds;
 };

@@ -91,3 +91,20 @@ def test_default_chunk_length_with_a_hot_row(B, gpu):
           for tpw in (0, 2, 8)}
     dev.free()
     assert ms[0] <= 1.1 * min(ms[2], ms[8]), ms
+
+
+def test_order_switch_after_the_copy_changes_nothing(B, gpu, monkeypatch):
+    """BLCO_FIBERS chooses the order of a copy, and windows for that copy, when
+    it is built; set later it reaches no launch."""
+    monkeypatch.delenv("BLCO_FIBERS", raising=False)
+    dims = (3000, 2000, 500)
+    dev = B.DeviceTensor.generate(dims, 2_000_000, zipf=(0.9, 0.9, 0.0), gen_rank=4, seed=3, topup=True,
+                                  value_dtype=B.F32)
+    for switch, rank in ((None, 32), ("0", 16)):
+        if switch:
+            monkeypatch.setenv("BLCO_FIBERS", switch)
+        F = [B.DeviceArray((d, rank), B.F32) for d in dims]
+        out = B.DeviceArray((dims[0], rank), B.F32)
+        B.mttkrp(dev, 0, rank, F, out, factor_dtype=B.F32, kernel=B.K_SORTED, thread_cf=1)
+        assert dev.rows_plan(0, rank, B.F32) == (1, False, 0)
+    dev.free()
