@@ -691,17 +691,17 @@ static int ensure_row_ordered(blco_dev* d, int mode, int rank, int ftype)
 // pieces shrink to a PIECE_WAVES-th of the tensor, or the waves that hold them
 // run on alone: 2M nonzeros at rank 64, a row of 220,000, 147 us with pieces of
 // 2048, 92 of 1024, 88 of 256 (the last with an error of 3.8e-7 against 1.8e-7).
-// A tiled
-// copy pads every tile's chunk list with empty chunks to one common length, a
+// Without long_rows every row is cut by the cap alone.
+// A tiled copy pads every tile's chunk list with empty chunks to one common length, a
 // multiple of the waves per workgroup: the grid then has NUM_XCD equal ranges
 // of workgroups and the XCD-contiguous workgroup numbering puts tile t on XCD t.
 constexpr uint64_t LONG_ROW = 32768, LONG_PIECE = 2 * WAVE * SORTED_TPW, PIECE_WAVES = 1024;
 
-static std::vector<Chunk> sorted_chunks(const blco_dev* d, int mode, int tpw)
+static std::vector<Chunk> sorted_chunks(const blco_dev* d, int mode, int tpw, bool long_rows)
 {
     const uint64_t base = (uint64_t)WAVE * tpw, cap = 2 * base;
     const int ntiles = std::max(1, d->stiles[mode]);
-    uint64_t long_piece = LONG_PIECE;
+    uint64_t long_piece = long_rows ? LONG_PIECE : cap;
     while (long_piece > cap && long_piece * PIECE_WAVES > d->nnz) long_piece /= 2;
     long_piece = std::max(long_piece, cap);
     std::vector<std::vector<Chunk>> tiles(ntiles);
@@ -775,13 +775,14 @@ static std::vector<Chunk> sorted_chunks(const blco_dev* d, int mode, int tpw)
     return h;
 }
 
-static const ChunkTab* sorted_chunk_table(blco_dev* d, int mode, int tpw)
+static const ChunkTab* sorted_chunk_table(blco_dev* d, int mode, int tpw, bool long_rows)
 {
     for (auto& t : d->stabs[mode])
-        if (t.tpw == tpw) return &t;
-    const std::vector<Chunk> h = sorted_chunks(d, mode, tpw);
+        if (t.tpw == tpw && t.long_rows == long_rows) return &t;
+    const std::vector<Chunk> h = sorted_chunks(d, mode, tpw, long_rows);
     ChunkTab t;
     t.tpw = tpw;
+    t.long_rows = long_rows;
     t.n = (uint32_t)h.size();
     if (t.n) {
         if (hipMalloc(&t.d, sizeof(Chunk) * t.n) != hipSuccess) {
@@ -1063,7 +1064,7 @@ int rows_batch_prepare(blco_dev* d, int mode, int rank, int ftype)
 
 std::vector<Chunk> rows_batch_chunks(const blco_dev* d, int mode, int tpw)
 {
-    return d->nnz ? sorted_chunks(d, mode, tpw) : std::vector<Chunk>();
+    return d->nnz ? sorted_chunks(d, mode, tpw, true) : std::vector<Chunk>();
 }
 
 MttkrpArgs rows_batch_args(const blco_dev* d, int mode, int rank)
@@ -1285,14 +1286,18 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
         const ChunkTab* stab = nullptr;
         size_t lds = 0;
         if (!wide && d->sforced[mode]) {
-            stab = sorted_chunk_table(d, mode, tpw > 0 ? tpw : long_tpw(d, rank, ftype));
+            stab = sorted_chunk_table(d, mode, tpw > 0 ? tpw : long_tpw(d, rank, ftype), true);
             if (!stab) return BLCO_ENOMEM;
             a.nchunks = stab->n;
             lds = rows_kernel_plan(d, mode, rank, ftype, true, &a);
         }
         if (!lds) {
-            if (tpw <= 0) tpw = sorted_tpw(d, mode, rank, ftype);
-            stab = sorted_chunk_table(d, mode, tpw);
+            // the per-slot adds of the wide kernels take long chunks, and below
+            // 2^22 nonzeros no long pieces: 3M nonzeros into 20,000 rows beside a
+            // factor of 2.2 GB, FP32, 106 us so, 167 with pieces (at 2 to 8
+            // tiles); 100M 2115 with 16 tiles, 2341 with 2
+            if (tpw <= 0) tpw = wide ? long_tpw(d, rank, ftype) : sorted_tpw(d, mode, rank, ftype);
+            stab = sorted_chunk_table(d, mode, tpw, !wide || d->nnz >= (1ull << 22));
             if (!stab) return BLCO_ENOMEM;
         }
         if (wide) {

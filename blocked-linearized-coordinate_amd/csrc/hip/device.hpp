@@ -56,6 +56,7 @@ struct SelCache {
 
 struct ChunkTab {
     int tpw = 0;
+    bool long_rows = false;  // of a row-ordered copy: long rows in long pieces
     Chunk* d = nullptr;
     uint32_t n = 0;
     std::vector<uint32_t> first;  // first chunk of each block (nblocks + 1)
@@ -115,7 +116,7 @@ struct blco_dev {
     int sinner[BLCO_MAX_MODES] = {};
     bool sfiber[BLCO_MAX_MODES] = {}, sforced[BLCO_MAX_MODES] = {};
     std::vector<uint64_t> srun_h[BLCO_MAX_MODES];
-    std::list<blco::ChunkTab> stabs[BLCO_MAX_MODES];  // row-aware chunks of the copy, per tpw
+    std::list<blco::ChunkTab> stabs[BLCO_MAX_MODES];  // row-aware chunks of the copy, per tpw and long_rows
     // nonzeros per index of every mode, as prefix sums (dims + 1 entries),
     // for the hot-row windows of the row-ordered kernels (built on first use)
     std::vector<uint64_t> idx_prefix[BLCO_MAX_MODES];

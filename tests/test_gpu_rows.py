@@ -108,3 +108,28 @@ def test_order_switch_after_the_copy_changes_nothing(B, gpu, monkeypatch):
         B.mttkrp(dev, 0, rank, F, out, factor_dtype=B.F32, kernel=B.K_SORTED, thread_cf=1)
         assert dev.rows_plan(0, rank, B.F32) == (1, False, 0)
     dev.free()
+
+
+@pytest.mark.parametrize("nnz", [3_000_000, (1 << 22) + 99])
+def test_wide_factors_with_a_long_row(B, O, gpu, nnz):
+    """A factor of more than 2 GiB (64-bit offsets) beside a mode whose most
+    frequent row has over 32768 nonzeros, below and above the size from which
+    that row's pieces are longer than the chunks."""
+    dims, rank = (17_000_000, 2000, 300), 32
+    assert dims[0] * rank * 4 >= 1 << 31
+    t = B.Coo.generate(dims, nnz, zipf=(0.9, 1.0, 0.0), gen_rank=2, seed=17, topup=True)
+    assert np.bincount(t.cidx[1].astype(int)).max() > 32768
+    dev = B.DeviceTensor(B.encode(t), value_dtype=B.F32)
+    U = [np.random.default_rng(m).random((d, rank), dtype=np.float32) for m, d in enumerate(dims)]
+    for m in (1, 2):
+        got, _ = mttkrp(B, dev, U, m, 1, 0)
+        want = np.zeros((dims[m], rank))
+        for at in range(0, nnz, 1 << 20):
+            i = [c[at:at + (1 << 20)].astype(np.int64) for c in t.cidx]
+            p = t.vals[at:at + (1 << 20), None] * U[0][i[0]]
+            p *= U[3 - m][i[3 - m]]
+            for c in range(rank):
+                want[:, c] += np.bincount(i[m], weights=p[:, c], minlength=dims[m])
+        e = np.linalg.norm(got - want) / np.linalg.norm(want)
+        assert e <= TOL[1], (nnz, m, e)
+    dev.free()
