@@ -59,18 +59,17 @@ static int long_tpw(const blco_dev* d, int rank, int ftype)
 // Default tiles of 64 nonzeros per chunk of k_mttkrp_rows.  A chunk of 2 tiles
 // runs in one or two rounds of the kernel: the most waves and the closest
 // neighbours in L1.  Longer chunks pay only where a chunk's end, which adds its
-// open row to HBM, is dear and seldom another row's end too: output rows of
-// more than 128 bytes and of a thousand nonzeros or so.  Times in us with 2, 8
-// and 16 tiles, FP64 at rank 32: 77M nonzeros over 12,092 rows 1583, 1512, 1506;
-// 200M over 2M rows 5381, 6086, 6820, over 600,000 rows 6088, 6149, 7451; 1.7B
-// over 4.8M rows 41938, 43263, 49704.  FP32 at rank 32: 77M 806, 798, 819; 1.7B
-// 20162, 19915, 22797.  Hot rows do not need them: their pieces are long at any
-// setting (LONG_ROW).
+// open row to HBM, is dear and rows long: output rows of more than 128 bytes on
+// copies in XCD tiles (xcd_tiles takes those with long rows).  Times in us with
+// 2, 8 and 16 tiles, FP64 at rank 32: 77M nonzeros over 12,092 rows in tiles
+// 1583, 1512, 1506; untiled, 200M over 2M rows 5381, 6086, 6820, over 600,000
+// 6088, 6149, 7451, 1.7B over 4.8M 41938, 43263, 49704.  FP32 at rank 32: 77M
+// 806, 798, 819; 1.7B 20162, 19915, 22797.  Hot rows do not need them: their
+// pieces are long at any setting (LONG_ROW).
 static int sorted_tpw(const blco_dev* d, int mode, int rank, int ftype)
 {
     if (d->nnz < (1ull << 17)) return 1;  // 100k nonzeros: 5.4 us with 1, 6.3 with 2
-    if (d->nnz < (1ull << 22) || (uint64_t)rank * (ftype == BLCO_F64 ? 8 : 4) <= 128) return 2;
-    return d->nnz / 1024 < d->srun_h[mode].size() - 1 ? 2 : ROWS_LONG_TPW;
+    return (uint64_t)rank * (ftype == BLCO_F64 ? 8 : 4) > 128 && d->stiles[mode] > 1 ? ROWS_LONG_TPW : 2;
 }
 
 // Nonzeros of one streamed unit: a quarter of the tensor where that is below

@@ -162,9 +162,8 @@ int blco_dev_set_value_dtype(blco_dev* d, int value_dtype);
  * BLCO_F64 factors, f32 otherwise; it is accumulated into (the caller
  * zeroes it, src/cpd_gpu.cu:155).  nprtn: lvl3 partial-matrix count (0 =
  * default); thread_cf: tiles of 64 nonzeros per wave (0 = default: 4, and
- * for kernel 14 2, or 1 for tensors of fewer than 2^17 nonzeros, or 8 from
- * 2^22 nonzeros for output rows of more than 128 bytes that average 1024
- * nonzeros). */
+ * for kernel 14 2, or 1 for tensors of fewer than 2^17 nonzeros, or 8 for
+ * output rows of more than 128 bytes on copies grouped by tiles). */
 int blco_mttkrp(blco_dev* d, int mode, int rank, int factor_dtype,
                 void* const* factors, void* out, int kernel, int nprtn,
                 int thread_cf, void* stream);

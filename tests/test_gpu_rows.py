@@ -61,10 +61,11 @@ def test_infinities_stay_in_their_rows(B, O, gpu):
 
 @pytest.mark.parametrize("rank,dtype", [(32, 0), (33, 1), (32, 1)])
 def test_default_chunk_lengths_of_large_tensors(B, O, gpu, rank, dtype):
-    """Just past 2^22 nonzeros: output rows of more than 128 bytes in a mode
-    of many rows (chunks of 2 tiles) and in modes of long ones (8 tiles, the
-    kernel's long rounds), a most frequent row of over 32768 nonzeros (pieces
-    of 2048), and 128-byte rows (2 tiles everywhere)."""
+    """Just past 2^22 nonzeros, from where copies are grouped by XCD tiles:
+    output rows of more than 128 bytes in a mode of many rows (untiled, chunks
+    of 2 tiles of 64) and in modes of long ones (8, the kernel's long rounds), a
+    most frequent row of over 32768 nonzeros (pieces of 2048), and 128-byte
+    rows (2 everywhere)."""
     dims, nnz = (100_000, 1500, 900), (1 << 22) + 4321
     t = B.Coo.generate(dims, nnz, zipf=(0.3, 1.1, 0.0), gen_rank=4, seed=22, topup=True)
     assert t.nnz == nnz and np.bincount(t.cidx[1].astype(int)).max() > 32768
@@ -73,6 +74,8 @@ def test_default_chunk_lengths_of_large_tensors(B, O, gpu, rank, dtype):
     U = [np.random.default_rng(m).random((d, rank)) for m, d in enumerate(dims)]
     for m in range(3):
         got, held = mttkrp(B, dev, U, m, dtype, 0)
+        # (FP32 copies are in fiber order here, whose outer factors L2 holds)
+        assert (dev.row_copy(m, rank, dtype)["tiles"] > 1) == (m > 0 and dtype == 0)
         want = at.mttkrp(held, m)
         e = np.linalg.norm(got - want) / np.linalg.norm(want)
         assert e <= TOL[dtype], (rank, dtype, m, e)
