@@ -303,7 +303,11 @@ int blco_cpals_iterate(blco_cpals_state* s, int n_iters, double* fits, int* done
                 int rc = mttkrp_prepare(s->d, s->order[k], s->R, s->ft, s->o.kernel);
                 if (rc) return rc;
             }
-            // F of the first mode; every update factors the next mode's
+        }
+        if (it == 0 || s->in_sweep) {
+            // F of the first mode; every update factors the next mode's.  After a
+            // sweep that ended half-way it is formed anew from the Grams, which
+            // are those of the factors as they are.
             AlsLaunch l = s->upd[s->order[s->N - 1]];
             const int rc = launch_als_begin(l, s->R, s->eps, s->st);
             if (rc) return rc;
@@ -313,7 +317,7 @@ int blco_cpals_iterate(blco_cpals_state* s, int n_iters, double* fits, int* done
             const int rc = launch_fill(s->Mbuf, s->m_bytes / (s->mt == BLCO_F64 ? 8 : 4), s->mt, 0.0, s->st);
             if (rc) return rc;
         }
-        s->m_dirty = true;  // until the sweep is through
+        s->m_dirty = s->in_sweep = true;  // until the sweep is through
         if (use_graph) {
             if (!s->gexec) {
                 HIP_TRY(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
@@ -333,7 +337,7 @@ int blco_cpals_iterate(blco_cpals_state* s, int n_iters, double* fits, int* done
         HIP_TRY(hipMemcpyAsync(s->h_fit, s->fitbuf, sizeof(double) * 3, hipMemcpyDeviceToHost, s->st));
         HIP_TRY(hipEventRecord(s->it1, s->st));
         HIP_TRY(hipStreamSynchronize(s->st));
-        s->m_dirty = false;
+        s->m_dirty = s->in_sweep = false;
         float ms = 0.f;
         HIP_TRY(hipEventElapsedTime(&ms, s->it0, s->it1));
         s->iter_ms += ms;

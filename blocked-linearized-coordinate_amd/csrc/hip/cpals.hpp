@@ -17,6 +17,9 @@ struct blco_cpals_state {
     void* arena = nullptr;  // one device allocation for everything below
     void* U[BLCO_MAX_MODES] = {};
     double* G[BLCO_MAX_MODES] = {};
+    // F (fac, colscale) belongs to the sweep's first mode between sweeps, and to
+    // a later one after a sweep that an error ended
+    bool in_sweep = false;
     // the MTTKRP's output, all zeros between a mode's update and the next
     // MTTKRP; m_dirty: an error or an export left something in it
     void* Mbuf = nullptr;

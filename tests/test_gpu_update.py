@@ -71,3 +71,25 @@ def test_factors_read_between_sweeps(B, gpu, graph):
     for a, b in zip(s.get()[0], whole.get()[0]):
         assert np.linalg.norm(a - b) <= 1e-9 * np.linalg.norm(b)
     dev.free()
+
+
+def test_iterate_after_a_failed_sweep(B, gpu):
+    """A sweep that an error ended (here values of the wrong type) leaves F to be
+    formed anew: the solver goes on as one that never failed."""
+    dims, R = (700, 300, 200), 9
+    t = B.Coo.generate(dims, 30000, gen_rank=3, value_kind=0, seed=4)
+    dev = B.DeviceTensor(B.encode(t))
+    U0 = B.init_factors(6, dims, R)
+    whole = B.CpAls(dev, U0, R)
+    want = whole.iterate(5)
+    s = B.CpAls(dev, U0, R)
+    got = list(s.iterate(2))
+    dev.set_value_dtype(B.F32)  # whole numbers: exact there and back
+    with pytest.raises(B.BlcoError):
+        s.iterate(1)
+    dev.set_value_dtype(B.F64)
+    got.extend(s.iterate(3))
+    assert np.allclose(got, want, rtol=0, atol=1e-10)
+    for a, b in zip(s.get()[0], whole.get()[0]):
+        assert np.linalg.norm(a - b) <= 1e-9 * np.linalg.norm(b)
+    dev.free()
