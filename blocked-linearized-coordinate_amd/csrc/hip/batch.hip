@@ -208,6 +208,7 @@ struct blco_batch {
     hipStream_t st = nullptr;
     std::list<ChunkList> lists;
     std::list<RowsList> rows_lists;
+    bool no_rows[BLCO_MAX_MODES][3] = {};  // no device memory for the copies of a mode (and factor type)
     std::vector<Tuned> tuned;
     BatchTensor* d_tens = nullptr;  // descriptors of blco_batch_mttkrp calls
     size_t tens_cap = 0;
@@ -426,6 +427,37 @@ int upload_descriptors(blco_batch* b, const std::vector<BatchTensor>& v)
     return BLCO_OK;
 }
 
+// What a blco_batch_cpals call holds, given back however it ends.
+struct BatchRun {
+    blco_batch* b;
+    std::vector<blco_cpals_state*> S;
+    std::vector<BatchTensor*> d_desc;
+    char* d_pack = nullptr;  // kernel arguments and ALS tasks of every mode
+    double *d_fits = nullptr, *h_fits = nullptr;
+    double* d_export = nullptr;  // every tensor's factors and lambda, f64
+    hipEvent_t it0 = nullptr, it1 = nullptr;
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t gexec = nullptr;
+
+    BatchRun(blco_batch* batch, int T) : b(batch), S(T, nullptr), d_desc(batch->maxN, nullptr) {}
+    ~BatchRun()
+    {
+        if (b->st) (void)hipStreamSynchronize(b->st);
+        if (gexec) (void)hipGraphExecDestroy(gexec);
+        if (graph) (void)hipGraphDestroy(graph);
+        for (blco_cpals_state* s : S)
+            if (s) blco_cpals_free(s);
+        for (BatchTensor* p : d_desc)
+            if (p) (void)hipFree(p);
+        if (d_pack) (void)hipFree(d_pack);
+        if (d_fits) (void)hipFree(d_fits);
+        if (d_export) (void)hipFree(d_export);
+        if (h_fits) (void)hipHostFree(h_fits);
+        for (hipEvent_t e : {it0, it1})
+            if (e) (void)hipEventDestroy(e);
+    }
+};
+
 }  // namespace
 }  // namespace blco
 
@@ -518,8 +550,8 @@ int blco_batch_mttkrp(blco_batch* b, int mode, int rank, int factor_dtype, void*
     return BLCO_OK;
 }
 
-int blco_batch_cpals(blco_batch* b, const blco_cpals_opts* o, double* const* U, double* lambda, double* fits,
-                     int* iters, double* iter_ms)
+static int batch_cpals(blco_batch* b, const blco_cpals_opts* o, double* const* U, double* lambda, double* fits,
+                       int* iters, double* iter_ms)
 {
     if (!b || !o || !U) return fail(BLCO_EINVAL, "null argument");
     const int T = (int)b->devs.size(), R = o->rank;
@@ -530,35 +562,19 @@ int blco_batch_cpals(blco_batch* b, const blco_cpals_opts* o, double* const* U, 
     o2.use_graph = 0;
     o2.mode_order = 0;  // modes 0..N-1 in every tensor
     o2.verbose = 0;
-    std::vector<blco_cpals_state*> S(T, nullptr);
-    std::vector<BatchTensor*> d_desc(b->maxN, nullptr);
-    char* d_pack = nullptr;     // kernel arguments and ALS tasks of every mode
-    double *d_fits = nullptr, *h_fits = nullptr;
-    double* d_export = nullptr;  // every tensor's factors and lambda, f64
-    hipEvent_t it0 = nullptr, it1 = nullptr;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t gexec = nullptr;
-    auto cleanup = [&](int code) {
-        if (b->st) (void)hipStreamSynchronize(b->st);
-        if (gexec) (void)hipGraphExecDestroy(gexec);
-        if (graph) (void)hipGraphDestroy(graph);
-        for (blco_cpals_state* s : S)
-            if (s) blco_cpals_free(s);
-        for (BatchTensor* p : d_desc)
-            if (p) (void)hipFree(p);
-        if (d_pack) (void)hipFree(d_pack);
-        if (d_fits) (void)hipFree(d_fits);
-        if (d_export) (void)hipFree(d_export);
-        if (h_fits) (void)hipHostFree(h_fits);
-        for (hipEvent_t e : {it0, it1})
-            if (e) (void)hipEventDestroy(e);
-        return code;
-    };
+    BatchRun run(b, T);
+    std::vector<blco_cpals_state*>& S = run.S;
+    std::vector<BatchTensor*>& d_desc = run.d_desc;
+    char*& d_pack = run.d_pack;
+    double *&d_fits = run.d_fits, *&h_fits = run.h_fits, *&d_export = run.d_export;
+    hipEvent_t &it0 = run.it0, &it1 = run.it1;
+    hipGraph_t& graph = run.graph;
+    hipGraphExec_t& gexec = run.gexec;
     for (int t = 0; t < T; ++t) {
         rc = cpals_state_create(b->devs[t], &o2, (const double* const*)(U + (size_t)t * BLCO_MAX_MODES), false, &S[t]);
-        if (rc) return cleanup(rc);
+        if (rc) return rc;
         rc = launch_fill(S[t]->Mbuf, S[t]->m_bytes / (S[t]->mt == BLCO_F64 ? 8 : 4), S[t]->mt, 0.0, S[t]->st);
-        if (rc) return cleanup(rc);
+        if (rc) return rc;
     }
     // every tensor's fit lands in one array: one read-back per iteration
     std::vector<uint64_t> export_at(T + 1, 0);
@@ -569,96 +585,126 @@ int blco_batch_cpals(blco_batch* b, const blco_cpals_opts* o, double* const* U, 
     if (hipMalloc((void**)&d_fits, sizeof(double) * 4 * T) != hipSuccess ||
         hipMalloc((void**)&d_export, sizeof(double) * export_at[T]) != hipSuccess ||
         hipHostMalloc((void**)&h_fits, sizeof(double) * 4 * T, hipHostMallocDefault) != hipSuccess)
-        return cleanup(fail(BLCO_ENOMEM, "batch result buffers"));
+        return fail(BLCO_ENOMEM, "batch result buffers");
     if (hipEventCreate(&it0) != hipSuccess || hipEventCreate(&it1) != hipSuccess)
-        return cleanup(fail(BLCO_EHIP, "event creation failed"));
+        return fail(BLCO_EHIP, "event creation failed");
     // per mode: the tensors of each order through kernel 14 over their copies,
     // or the mode's members through the tuned persistent kernel when a copy
     // cannot be had; then the members' update tasks
     struct Group { const RowsList* list; size_t args; };
-    std::vector<std::vector<Group>> groups(b->maxN);
-    std::vector<bool> by_rows(b->maxN, true);
+    std::vector<std::vector<Group>> groups;
+    std::vector<bool> by_rows;
     std::vector<Tuned> shape(b->maxN);
-    std::vector<char> pack;
-    auto append = [&](const void* p, size_t bytes) {
-        const size_t at = (pack.size() + 63) / 64 * 64;
-        pack.resize(at + bytes);
-        std::memcpy(pack.data() + at, p, bytes);
-        return at;
-    };
-    std::vector<AlsLaunch> upd(b->maxN);
-    std::vector<size_t> task_at(b->maxN + 1);
-    for (int n = 0; n < b->maxN; ++n) {
-        const std::vector<int> mem = members(b, n);
-        for (int t : mem) {
-            rc = rows_batch_prepare(b->devs[t], n, R, ft);
-            if (rc == BLCO_ENOMEM || rc == BLCO_EUNSUPPORTED) by_rows[n] = false;
-            else if (rc) return cleanup(rc);
-            if (!by_rows[n]) break;
-        }
-        std::vector<AlsTask> tasks;
-        for (int t : mem) {
-            AlsTask k = S[t]->tasks[n];
-            k.fit = d_fits + 4 * t;
-            k.first = upd[n].blocks;
-            upd[n].blocks += k.parts;
-            upd[n].most_parts = std::max(upd[n].most_parts, k.parts);
-            tasks.push_back(k);
-        }
-        upd[n].ntasks = (int)tasks.size();
-        task_at[n] = append(tasks.data(), sizeof(AlsTask) * tasks.size());
-        if (!by_rows[n]) continue;
-        for (int order = 2; order <= BLCO_MAX_MODES; ++order) {
-            std::vector<int> who;
-            for (int t : mem)
-                if (b->devs[t]->nmodes == order) who.push_back(t);
-            if (who.empty()) continue;
-            std::vector<MttkrpArgs> args;
-            for (int t : who) {
-                MttkrpArgs a = rows_batch_args(b->devs[t], n, R);
-                for (int m = 0; m < order; ++m) a.f[m] = S[t]->U[m];
-                a.out = S[t]->Mbuf;
-                args.push_back(a);
-            }
-            const RowsList* l = rows_list(b, n, order, who);
-            if (!l) return cleanup(BLCO_ENOMEM);
-            groups[n].push_back(Group{l, append(args.data(), sizeof(MttkrpArgs) * args.size())});
-        }
-    }
-    // the tasks of every tensor's last mode, whose successor is mode 0
+    std::vector<AlsLaunch> upd;
     AlsLaunch begin;
-    {
-        std::vector<AlsTask> tasks;
-        for (int t = 0; t < T; ++t) tasks.push_back(S[t]->tasks[S[t]->N - 1]);
-        begin.ntasks = T;
-        task_at[b->maxN] = append(tasks.data(), sizeof(AlsTask) * tasks.size());
-    }
-    if (hipMalloc((void**)&d_pack, pack.size()) != hipSuccess) return cleanup(fail(BLCO_ENOMEM, "batch descriptors"));
-    if (hipMemcpy(d_pack, pack.data(), pack.size(), hipMemcpyHostToDevice) != hipSuccess)
-        return cleanup(fail(BLCO_EHIP, "descriptor upload failed"));
-    for (int n = 0; n < b->maxN; ++n) upd[n].d_tasks = reinterpret_cast<const AlsTask*>(d_pack + task_at[n]);
-    begin.d_tasks = reinterpret_cast<const AlsTask*>(d_pack + task_at[b->maxN]);
-    for (int t = 0; t < T; ++t)
-        if (hipStreamSynchronize(S[t]->st) != hipSuccess) return cleanup(fail(BLCO_EHIP, "setup failed"));
-    for (int n = 0; n < b->maxN; ++n) {
-        if (by_rows[n]) continue;
-        std::vector<void*> F((size_t)T * BLCO_MAX_MODES, nullptr), O(T, nullptr);
-        for (int t = 0; t < T; ++t) {
-            for (int m = 0; m < S[t]->N; ++m) F[(size_t)t * BLCO_MAX_MODES + m] = S[t]->U[m];
-            O[t] = S[t]->Mbuf;
+    std::vector<std::pair<int, int>> built;  // (tensor, mode) of the copies that this call built
+    // drops the copies built since there were `keep` of them
+    auto drop_built = [&](size_t keep) {
+        for (; built.size() > keep; built.pop_back()) drop_row_copy(b->devs[built.back().first], built.back().second);
+    };
+    auto plan = [&](bool rows) -> int {
+        groups.assign(b->maxN, {});
+        by_rows.assign(b->maxN, rows);
+        upd.assign(b->maxN, AlsLaunch());
+        std::vector<char> pack;
+        auto append = [&](const void* p, size_t bytes) {
+            const size_t at = (pack.size() + 63) / 64 * 64;
+            pack.resize(at + bytes);
+            std::memcpy(pack.data() + at, p, bytes);
+            return at;
+        };
+        std::vector<size_t> task_at(b->maxN + 1);
+        for (int n = 0; n < b->maxN; ++n) {
+            const std::vector<int> mem = members(b, n);
+            if (b->no_rows[n][ft]) by_rows[n] = false;
+            const size_t before = built.size();
+            for (size_t i = 0; i < mem.size() && by_rows[n]; ++i) {
+                blco_dev* d = b->devs[mem[i]];
+                const bool had = d->d_scoords[n] != nullptr;
+                const int r = rows_batch_prepare(d, n, R, ft);
+                if (!had && d->d_scoords[n]) built.emplace_back(mem[i], n);
+                if (r == BLCO_ENOMEM || r == BLCO_EUNSUPPORTED) {
+                    // this mode's copies of the other tensors would only take room
+                    by_rows[n] = false;
+                    b->no_rows[n][ft] = r == BLCO_ENOMEM;
+                    drop_built(before);
+                } else if (r) {
+                    return r;
+                }
+            }
+            std::vector<AlsTask> tasks;
+            for (int t : mem) {
+                AlsTask k = S[t]->tasks[n];
+                k.fit = d_fits + 4 * t;
+                k.first = upd[n].blocks;
+                upd[n].blocks += k.parts;
+                upd[n].most_parts = std::max(upd[n].most_parts, k.parts);
+                tasks.push_back(k);
+            }
+            upd[n].ntasks = (int)tasks.size();
+            task_at[n] = append(tasks.data(), sizeof(AlsTask) * tasks.size());
+            if (!by_rows[n]) continue;
+            for (int order = 2; order <= BLCO_MAX_MODES; ++order) {
+                std::vector<int> who;
+                for (int t : mem)
+                    if (b->devs[t]->nmodes == order) who.push_back(t);
+                if (who.empty()) continue;
+                std::vector<MttkrpArgs> args;
+                for (int t : who) {
+                    MttkrpArgs a = rows_batch_args(b->devs[t], n, R);
+                    for (int m = 0; m < order; ++m) a.f[m] = S[t]->U[m];
+                    a.out = S[t]->Mbuf;
+                    args.push_back(a);
+                }
+                const RowsList* l = rows_list(b, n, order, who);
+                if (!l) return BLCO_ENOMEM;
+                groups[n].push_back(Group{l, append(args.data(), sizeof(MttkrpArgs) * args.size())});
+            }
         }
-        const std::vector<BatchTensor> v = descriptors(b, n, F.data(), O.data());
-        if (hipMalloc(&d_desc[n], sizeof(BatchTensor) * std::max<size_t>(1, v.size())) != hipSuccess)
-            return cleanup(fail(BLCO_ENOMEM, "descriptor allocation failed"));
-        if (!v.empty() && hipMemcpy(d_desc[n], v.data(), sizeof(BatchTensor) * v.size(), hipMemcpyHostToDevice) != hipSuccess)
-            return cleanup(fail(BLCO_EHIP, "descriptor upload failed"));
-        rc = tune(b, d_desc[n], n, R, ft, &shape[n]);
-        if (rc) return cleanup(rc);
-        for (int t : members(b, n)) {  // the tuning runs left their sums there
-            rc = launch_fill(S[t]->Mbuf, S[t]->m_bytes / (S[t]->mt == BLCO_F64 ? 8 : 4), S[t]->mt, 0.0, b->st);
-            if (rc) return cleanup(rc);
+        // the tasks of every tensor's last mode, whose successor is mode 0
+        {
+            std::vector<AlsTask> tasks;
+            for (int t = 0; t < T; ++t) tasks.push_back(S[t]->tasks[S[t]->N - 1]);
+            begin.ntasks = T;
+            task_at[b->maxN] = append(tasks.data(), sizeof(AlsTask) * tasks.size());
         }
+        if (d_pack) (void)hipFree(d_pack);
+        d_pack = nullptr;
+        if (hipMalloc((void**)&d_pack, pack.size()) != hipSuccess) return fail(BLCO_ENOMEM, "batch descriptors");
+        if (hipMemcpy(d_pack, pack.data(), pack.size(), hipMemcpyHostToDevice) != hipSuccess)
+            return fail(BLCO_EHIP, "descriptor upload failed");
+        for (int n = 0; n < b->maxN; ++n) upd[n].d_tasks = reinterpret_cast<const AlsTask*>(d_pack + task_at[n]);
+        begin.d_tasks = reinterpret_cast<const AlsTask*>(d_pack + task_at[b->maxN]);
+        for (int t = 0; t < T; ++t)
+            if (hipStreamSynchronize(S[t]->st) != hipSuccess) return fail(BLCO_EHIP, "setup failed");
+        for (int n = 0; n < b->maxN; ++n) {
+            if (by_rows[n]) continue;
+            std::vector<void*> F((size_t)T * BLCO_MAX_MODES, nullptr), O(T, nullptr);
+            for (int t = 0; t < T; ++t) {
+                for (int m = 0; m < S[t]->N; ++m) F[(size_t)t * BLCO_MAX_MODES + m] = S[t]->U[m];
+                O[t] = S[t]->Mbuf;
+            }
+            const std::vector<BatchTensor> v = descriptors(b, n, F.data(), O.data());
+            if (!d_desc[n] && hipMalloc(&d_desc[n], sizeof(BatchTensor) * std::max<size_t>(1, v.size())) != hipSuccess) {
+                d_desc[n] = nullptr;
+                return fail(BLCO_ENOMEM, "descriptor allocation failed");
+            }
+            if (!v.empty() && hipMemcpy(d_desc[n], v.data(), sizeof(BatchTensor) * v.size(), hipMemcpyHostToDevice) != hipSuccess)
+                return fail(BLCO_EHIP, "descriptor upload failed");
+            int r = tune(b, d_desc[n], n, R, ft, &shape[n]);
+            for (int t : members(b, n))  // the tuning runs left their sums there
+                if (!r) r = launch_fill(S[t]->Mbuf, S[t]->m_bytes / (S[t]->mt == BLCO_F64 ? 8 : 4), S[t]->mt, 0.0, b->st);
+            if (r) return r;
+        }
+        return BLCO_OK;
+    };
+    rc = plan(true);
+    if (rc == BLCO_ENOMEM && !built.empty()) {  // everything else fits without the copies
+        (void)hipStreamSynchronize(b->st);
+        drop_built(0);
+        rc = plan(false);
     }
+    if (rc) return rc;
     const double eps = S[0]->eps;
     auto sweep = [&](int which_norm) -> int {
         for (int n = 0; n < b->maxN; ++n) {
@@ -719,16 +765,16 @@ int blco_batch_cpals(blco_batch* b, const blco_cpals_opts* o, double* const* U, 
         if (it == 0) {
             rc = launch_als_begin(begin, R, eps, b->st);
             if (!rc) rc = sweep(0);
-            if (rc) return cleanup(rc);
+            if (rc) return rc;
         } else {
             if (!gexec) {
                 HIP_TRY(hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal));
                 rc = sweep(1);
                 hipError_t e = hipStreamEndCapture(b->st, &graph);
-                if (rc) return cleanup(rc);
-                if (e != hipSuccess) return cleanup(fail(BLCO_EHIP, "sweep capture failed: %s", hipGetErrorString(e)));
+                if (rc) return rc;
+                if (e != hipSuccess) return fail(BLCO_EHIP, "sweep capture failed: %s", hipGetErrorString(e));
                 if (hipGraphInstantiate(&gexec, graph, nullptr, nullptr, 0) != hipSuccess)
-                    return cleanup(fail(BLCO_EHIP, "graph instantiation failed"));
+                    return fail(BLCO_EHIP, "graph instantiation failed");
             }
             HIP_TRY(hipGraphLaunch(gexec, b->st));
         }
@@ -756,19 +802,29 @@ int blco_batch_cpals(blco_batch* b, const blco_cpals_opts* o, double* const* U, 
             }
         }
         rc = fetch(done);
-        if (rc) return cleanup(rc);
+        if (rc) return rc;
     }
     std::vector<int> never;  // max_iters == 0
     for (int t = 0; t < T; ++t)
         if (!stopped_at[t]) never.push_back(t);
     rc = fetch(never);
-    if (rc) return cleanup(rc);
+    if (rc) return rc;
     for (int t = 0; t < T; ++t) {
         if (fits) fits[t] = fit_old[t];
         if (iters) iters[t] = stopped_at[t];
     }
     if (iter_ms) *iter_ms = ms_n ? ms_sum / ms_n : 0.0;
-    return cleanup(BLCO_OK);
+    return BLCO_OK;
+}
+
+int blco_batch_cpals(blco_batch* b, const blco_cpals_opts* o, double* const* U, double* lambda, double* fits,
+                     int* iters, double* iter_ms)
+{
+    try {
+        return batch_cpals(b, o, U, lambda, fits, iters, iter_ms);
+    } catch (const std::bad_alloc&) {
+        return fail(BLCO_ENOMEM, "out of host memory");
+    }
 }
 
 }  // extern "C"

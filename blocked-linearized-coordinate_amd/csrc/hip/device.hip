@@ -1055,9 +1055,32 @@ static bool narrow_factors(const blco_dev* d, int rank, int ftype)
     return true;
 }
 
+void drop_row_copy(blco_dev* d, int mode)
+{
+    if (d->d_scoords[mode]) {
+        (void)hipFree(d->d_scoords[mode]);
+        d->d_scoords[mode] = nullptr;
+        d->bytes -= d->nnz * (8 + value_size(d->vdtype));
+    }
+    if (d->d_svals[mode]) (void)hipFree(d->d_svals[mode]);
+    d->d_svals[mode] = nullptr;
+    for (auto& t : d->stabs[mode]) {
+        if (t.d) (void)hipFree(t.d);
+        d->bytes -= sizeof(Chunk) * t.n;
+    }
+    d->stabs[mode].clear();
+    d->sgrp_h[mode].clear();
+    d->srun_h[mode].clear();
+    d->stiles[mode] = 0;
+    d->sinner[mode] = 0;
+    d->sfiber[mode] = d->sforced[mode] = false;
+    d->rows_plans[mode].clear();
+}
+
 int rows_batch_prepare(blco_dev* d, int mode, int rank, int ftype)
 {
     if (!narrow_factors(d, rank, ftype)) return BLCO_EUNSUPPORTED;
+    if (d->sorted_failed[mode]) return BLCO_ENOMEM;  // no room for it before
     return d->nnz ? ensure_row_ordered(d, mode, rank, ftype) : BLCO_OK;
 }
 
@@ -1973,28 +1996,13 @@ int blco_dev_set_value_dtype(blco_dev* d, int value_dtype)
         }
         (void)hipFree(d->d_vals);
         d->d_vals = nv;
-        d->bytes = d->bytes - n * old_sz + n * new_sz;
     }
     // the row-ordered copies hold values of the old type: rebuilt on next use
     for (int m = 0; m < BLCO_MAX_MODES; ++m) {
-        if (d->d_scoords[m]) {
-            (void)hipFree(d->d_scoords[m]);
-            d->d_scoords[m] = nullptr;
-            d->bytes -= n * (8 + old_sz);
-        }
-        if (d->d_svals[m]) (void)hipFree(d->d_svals[m]);
-        d->d_svals[m] = nullptr;
-        for (auto& t : d->stabs[m])
-            if (t.d) (void)hipFree(t.d);
-        d->stabs[m].clear();
-        d->sgrp_h[m].clear();
-        d->srun_h[m].clear();
+        drop_row_copy(d, m);
         d->sorted_failed[m] = false;
-        d->stiles[m] = 0;
-        d->sinner[m] = 0;
-        d->sfiber[m] = d->sforced[m] = false;
-        d->rows_plans[m].clear();
     }
+    if (n) d->bytes = d->bytes - n * old_sz + n * new_sz;
     d->sel_cache.clear();
     d->vdtype = value_dtype;
     return BLCO_OK;

@@ -177,6 +177,8 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
 // kernel) would do on its first call (kernel 14's row-ordered copy), without
 // a launch; a copy that does not fit leaves the mode to the row window.
 int mttkrp_prepare(blco_dev* d, int mode, int rank, int ftype, int kernel);
+// Frees a mode's row-ordered copy and what belongs to it; no launch may use it.
+void drop_row_copy(blco_dev* d, int mode);
 // Kernel 14 over many tensors in one launch (k_mttkrp_rows_batch): builds the
 // copy (BLCO_EUNSUPPORTED for factors that need 64-bit offsets), its chunks,
 // and the kernel arguments without factors and output.

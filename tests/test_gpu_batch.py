@@ -135,3 +135,32 @@ def test_batch_rejects_bad_input(B, gpu, small):
     bt.free()
     dev.free()
     streamed.free()
+
+
+def test_batch_without_room_for_a_copy(B, gpu):
+    """One tensor's device budget has no room for row-ordered copies: every mode
+    it has runs the persistent kernel, the copies built for the others are given
+    back, and the results are those of the tensors alone."""
+    shapes = [((300, 200, 100), 20000), ((120, 90, 80), 15000), ((60, 50, 40, 30), 12000)]
+    R, iters = 6, 3
+    devs, U0 = [], []
+    for k, (dims, nnz) in enumerate(shapes):
+        t = B.Coo.generate(dims, nnz, gen_rank=3, value_kind=1, seed=70 + k)
+        devs.append(B.DeviceTensor(B.encode(t), device_budget=t.nnz * 16 + 64 if k == 1 else 0))
+        assert devs[-1].residency()[:2] == (t.nnz, 0)
+        U0.append(B.init_factors(600 + k, dims, R))
+    bytes0 = [d.bytes() for d in devs]
+    bt = B.Batch(devs)
+    for _ in range(2):
+        U, lam, fits, its, _ = bt.cpals(U0, R, max_iters=iters, precision=B.F64)
+        held = [d.bytes() for d in devs]
+        # the third tensor's last mode is its own
+        assert held[:2] == bytes0[:2] and held[2] - bytes0[2] < 1.5 * devs[2].nnz * 16
+    for k, dev in enumerate(devs):
+        Us, ls, fs = B.cpals(dev, U0[k], R, iters)
+        assert abs(fits[k] - fs[-1]) <= 1e-9
+        for a, b in zip(U[k], Us):
+            assert np.linalg.norm(a - b) <= 1e-9 * np.linalg.norm(b), k
+    bt.free()
+    for d in devs:
+        d.free()
