@@ -1385,8 +1385,14 @@ public:
     {
         if (!p_) return;
         std::lock_guard<std::mutex> lk(mu());
-        if (kept() + n_ <= KEPT_MAX) idle().push_back({dev_, n_, p_});
-        else (void)hipFree(p_);
+        try {
+            if (kept() + n_ <= KEPT_MAX) {
+                idle().push_back({dev_, n_, p_});
+                return;
+            }
+        } catch (const std::bad_alloc&) {  // no room on the list
+        }
+        (void)hipFree(p_);
     }
     int get(size_t bytes, double** out)
     {
@@ -1405,8 +1411,11 @@ public:
         if (!p_) {
             n_ = (bytes + (1 << 20) - 1) >> 20 << 20;
             if (hipMalloc(&p_, n_) != hipSuccess) {
-                p_ = nullptr;
-                return fail(BLCO_ENOMEM, "device scratch of %llu bytes", (unsigned long long)n_);
+                release_all();  // the idle ones may be what is in the way
+                if (hipMalloc(&p_, n_) != hipSuccess) {
+                    p_ = nullptr;
+                    return fail(BLCO_ENOMEM, "device scratch of %llu bytes", (unsigned long long)n_);
+                }
             }
         }
         *out = static_cast<double*>(p_);
@@ -2170,9 +2179,10 @@ int blco_solve(double* const* grams, int nmodes, int mode, int rank, const void*
     if (!rc) rc = launch_solve_rows(M, U, dtype, rows, rank, fac, st);
     int h_status = 0;
     hipError_t e = hipMemcpyAsync(&h_status, status, sizeof(int), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    const hipError_t waited = hipStreamSynchronize(st);  // also when the copy failed: the scratch goes back idle
     if (rc) return rc;
     HIP_TRY(e);
+    HIP_TRY(waited);
     if (used_fallback) *used_fallback = h_status;
     return BLCO_OK;
 }
@@ -2231,9 +2241,10 @@ int blco_fit(double* const* grams, int nmodes, int rank, const double* lambda, c
     if (!rc) rc = launch_fit(gs, nmodes, rank, lambda, ip, normX2, out, st);
     double h[3] = {0, 0, 0};
     hipError_t e = hipMemcpyAsync(h, out, sizeof(double) * 3, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    const hipError_t waited = hipStreamSynchronize(st);  // also when the copy failed: the scratch goes back idle
     if (rc) return rc;
     HIP_TRY(e);
+    HIP_TRY(waited);
     *fit = h[0];
     return BLCO_OK;
 }

@@ -93,3 +93,41 @@ def test_iterate_after_a_failed_sweep(B, gpu):
     for a, b in zip(s.get()[0], whole.get()[0]):
         assert np.linalg.norm(a - b) <= 1e-9 * np.linalg.norm(b)
     dev.free()
+
+
+def test_step_calls_from_threads(B, gpu):
+    """The stand-alone step calls share idle scratch between calls, not between
+    calls that run at the same time: threads with sizes and streams of their
+    own."""
+    import ctypes
+    import threading
+
+    create = B.lib().hipStreamCreate  # of the HIP runtime that the library is linked to
+    create.restype = ctypes.c_int
+    ran, wrong = [], []
+
+    def work(k):
+        R, rows = 5 + 9 * k, 3000 * (k + 1) + k
+        rng = np.random.default_rng(k)
+        U, M = rng.standard_normal((rows, R)), rng.standard_normal((rows, R))
+        grams = [u.T @ u for u in (rng.standard_normal((4 * R + 9, R)) for _ in range(2))]
+        st = ctypes.c_void_p()
+        assert create(ctypes.byref(st)) == 0
+        Ud, Md = B.DeviceArray.from_numpy(U), B.DeviceArray.from_numpy(M)
+        Gd, X = B.DeviceArray((R, R)), B.DeviceArray((rows, R))
+        gd = [B.DeviceArray.from_numpy(g) for g in grams]
+        for _ in range(20):
+            B.gram(Ud, B.F64, rows, R, Gd, stream=st.value)
+            B.solve(gd + [Gd], 2, R, Md, X, B.F64, rows, stream=st.value)
+            want = np.linalg.solve(grams[0] * grams[1], M.T).T
+            if np.linalg.norm(Gd.numpy() - U.T @ U) > 1e-12 * np.linalg.norm(U.T @ U) * np.sqrt(rows) or \
+               np.linalg.norm(X.numpy() - want) > 1e-10 * np.linalg.norm(want):
+                wrong.append(k)
+        ran.append(k)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(5)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert sorted(ran) == list(range(5)) and not wrong
