@@ -37,7 +37,7 @@ constexpr int LVL3_MAX_MODE_LENGTH = 100;     // src/utils.hpp:13
 constexpr int DEFAULT_TPW = 4;                // tiles of 64 per wave
 constexpr int SORTED_TPW = 16;                // tiles of 64 per wave, row-ordered kernel (most)
 constexpr uint64_t SORTED_TARGET_CHUNKS = 8192;
-constexpr int ROWS_LONG_TPW = 8;              // chunks from here on take k_mttkrp_rows' long rounds
+constexpr int ROWS_LONG_TPW = 8;              // mean chunks from here on take k_mttkrp_rows' long rounds
 constexpr int DEFAULT_NPRTN = 1;
 constexpr uint32_t LVL3_CHUNKS_PER_WG = 64;  // at most
 constexpr uint32_t HOT_EXCLUDE = 64;  // hot rows kept out of the row windows
@@ -48,12 +48,16 @@ static int value_size(int vdt) { return vdt == BLCO_F64 ? 8 : 4; }
 // to 2^22 nonzeros, and 16 from there on; 32 for FP64 rows of 256 bytes or more
 // from 2^26 nonzeros.  What the kernels that add a row with its slot's lanes
 // were timed with: fewer chunk ends, each of which adds its open rows to HBM.
+static int long_tpw(uint64_t nnz)
+{
+    int t = 2;
+    while (t < SORTED_TPW && nnz > (uint64_t)WAVE * t * SORTED_TARGET_CHUNKS) t *= 2;
+    return t;
+}
+
 static int long_tpw(const blco_dev* d, int rank, int ftype)
 {
-    if (ftype == BLCO_F64 && rank >= 32 && d->nnz >= (1ull << 26)) return 32;
-    int t = 2;
-    while (t < SORTED_TPW && d->nnz > (uint64_t)WAVE * t * SORTED_TARGET_CHUNKS) t *= 2;
-    return t;
+    return ftype == BLCO_F64 && rank >= 32 && d->nnz >= (1ull << 26) ? 32 : long_tpw(d->nnz);
 }
 
 // Default tiles of 64 nonzeros per chunk of k_mttkrp_rows.  A chunk of 2 tiles
@@ -690,11 +694,15 @@ static int ensure_row_ordered(blco_dev* d, int mode, int rank, int ftype)
 // pieces shrink to a PIECE_WAVES-th of the tensor, or the waves that hold them
 // run on alone: 2M nonzeros at rank 64, a row of 220,000, 147 us with pieces of
 // 2048, 92 of 1024, 88 of 256 (the last with an error of 3.8e-7 against 1.8e-7).
+// Shorter rows beyond the cap are cut into about MID_PIECES, of at most the
+// length that long_tpw gives chunks: 30M nonzeros over 3000 x 4000 x 2000, FP32
+// at rank 32, 8.8e-8 to 1.2e-7 against 64 bits and 371 us in pieces of 256,
+// 5.7e-8 to 6.5e-8 and 350 to 358 us so.
 // Without long_rows every row is cut by the cap alone.
 // A tiled copy pads every tile's chunk list with empty chunks to one common length, a
 // multiple of the waves per workgroup: the grid then has NUM_XCD equal ranges
 // of workgroups and the XCD-contiguous workgroup numbering puts tile t on XCD t.
-constexpr uint64_t LONG_ROW = 32768, LONG_PIECE = 2 * WAVE * SORTED_TPW, PIECE_WAVES = 1024;
+constexpr uint64_t LONG_ROW = 32768, LONG_PIECE = 2 * WAVE * SORTED_TPW, PIECE_WAVES = 1024, MID_PIECES = 4;
 
 static std::vector<Chunk> sorted_chunks(const blco_dev* d, int mode, int tpw, bool long_rows)
 {
@@ -703,6 +711,8 @@ static std::vector<Chunk> sorted_chunks(const blco_dev* d, int mode, int tpw, bo
     uint64_t long_piece = long_rows ? LONG_PIECE : cap;
     while (long_piece > cap && long_piece * PIECE_WAVES > d->nnz) long_piece /= 2;
     long_piece = std::max(long_piece, cap);
+    // pieces of the rows between the two
+    const uint64_t mid_piece = long_rows ? std::max<uint64_t>(cap, 2 * WAVE * long_tpw(d->nnz)) : cap;
     std::vector<std::vector<Chunk>> tiles(ntiles);
     const std::vector<uint64_t>& runs = d->srun_h[mode];
     size_t r = 0;
@@ -717,7 +727,8 @@ static std::vector<Chunk> sorted_chunks(const blco_dev* d, int mode, int tpw, bo
             const uint64_t run_end = (r + 1 < runs.size()) ? std::min(runs[r + 1], end) : end;
             if (run_end - c0 > cap) {  // inside a long row
                 const uint64_t run_len = run_end - std::max(runs[r], g.start);
-                const uint64_t piece = run_len >= LONG_ROW ? long_piece : cap;
+                const uint64_t piece = run_len >= LONG_ROW ? long_piece
+                                                           : std::min(std::max(cap, run_len / MID_PIECES), mid_piece);
                 const uint64_t end_piece = std::min(c0 + piece, run_end);
                 emit(c0, end_piece);
                 c0 = end_piece;
@@ -738,7 +749,7 @@ static std::vector<Chunk> sorted_chunks(const blco_dev* d, int mode, int tpw, bo
         }
     }
     std::vector<Chunk> h;
-    if (ntiles == 1 && cap < long_piece) {
+    if (ntiles == 1 && cap < std::max(long_piece, mid_piece)) {
         // the pieces of long rows hold many times the nonzeros of the other
         // chunks and lie together: they go to the XCDs with the fewest
         // nonzeros, ahead of each one's equal share of the rest
@@ -782,6 +793,7 @@ static const ChunkTab* sorted_chunk_table(blco_dev* d, int mode, int tpw, bool l
     ChunkTab t;
     t.tpw = tpw;
     t.long_rows = long_rows;
+    t.filled = (uint32_t)std::count_if(h.begin(), h.end(), [](const Chunk& c) { return c.len > 0; });
     t.n = (uint32_t)h.size();
     if (t.n) {
         if (hipMalloc(&t.d, sizeof(Chunk) * t.n) != hipSuccess) {
@@ -1331,7 +1343,7 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
             int kind = fib ? W_FIBER_LDS : W_SORTED_LDS;
             if (!lds) {
                 rows_kernel_plan(d, mode, rank, ftype, false, &a);
-                kind = tpw >= ROWS_LONG_TPW ? W_ROWS : W_ROWS_SHORT;
+                kind = d->nnz >= (uint64_t)WAVE * ROWS_LONG_TPW * stab->filled ? W_ROWS : W_ROWS_SHORT;
                 gather_order(d, mode, a.order);
             }
             const uint32_t per_wg = WAVES_PER_WG * a.cpw;

@@ -58,7 +58,7 @@ struct ChunkTab {
     int tpw = 0;
     bool long_rows = false;  // of a row-ordered copy: long rows in long pieces
     Chunk* d = nullptr;
-    uint32_t n = 0;
+    uint32_t n = 0, filled = 0;   // chunks; of a row-ordered copy, those that are not empty
     std::vector<uint32_t> first;  // first chunk of each block (nblocks + 1)
     std::vector<StreamUnit> units;
 };

@@ -136,3 +136,25 @@ def test_wide_factors_with_a_long_row(B, O, gpu, nnz):
         e = np.linalg.norm(got - want) / np.linalg.norm(want)
         assert e <= TOL[1], (nnz, m, e)
     dev.free()
+
+
+@pytest.mark.parametrize("dims,nnz,tpw", [((160, 6000, 5000), 2_000_000, 4), ((300, 3000, 2000), 4_300_000, 16)])
+@pytest.mark.parametrize("dtype", [1, 2])
+def test_float_error_of_rows_cut_into_pieces(B, O, gpu, dims, nnz, tpw, dtype):
+    """Every piece of a row ends in a float add to the output.  Rows of 12,500
+    and 14,300 nonzeros are cut no finer than by chunks of the length that
+    leaves 4096 to 8192 of them (`tpw` tiles): the default's error against the
+    oracle is that of those chunks, to the tenth that the order of the adds
+    moves it by at most (pieces of 256 nonzeros: 1.4 and 1.8 times)."""
+    R = 32
+    t = B.Coo.generate(dims, nnz, gen_rank=3, value_kind=0, seed=12)
+    at = O.Alto(dims, t.cidx, t.vals, nprtn=8)
+    dev = B.DeviceTensor(B.encode(t), value_dtype=B.F32)
+    U = [np.random.default_rng(m).random((d, R)) for m, d in enumerate(dims)]
+    error = {}
+    for cf in (0, tpw):
+        got, held = mttkrp(B, dev, U, 0, dtype, cf)
+        want = at.mttkrp(held, 0)
+        error[cf] = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert error[0] <= 1.1 * error[tpw], (dims, dtype, error)
+    dev.free()
