@@ -698,13 +698,13 @@ static int ensure_row_ordered(blco_dev* d, int mode, int rank, int ftype)
 // length that long_tpw gives chunks: 30M nonzeros over 3000 x 4000 x 2000, FP32
 // at rank 32, 8.8e-8 to 1.2e-7 against 64 bits and 371 us in pieces of 256,
 // 5.7e-8 to 6.5e-8 and 350 to 358 us so.
-// Without long_rows every row is cut by the cap alone.
+// Without long_rows and mid_rows such rows are cut by the cap alone.
 // A tiled copy pads every tile's chunk list with empty chunks to one common length, a
 // multiple of the waves per workgroup: the grid then has NUM_XCD equal ranges
 // of workgroups and the XCD-contiguous workgroup numbering puts tile t on XCD t.
 constexpr uint64_t LONG_ROW = 32768, LONG_PIECE = 2 * WAVE * SORTED_TPW, PIECE_WAVES = 1024, MID_PIECES = 4;
 
-static std::vector<Chunk> sorted_chunks(const blco_dev* d, int mode, int tpw, bool long_rows)
+static std::vector<Chunk> sorted_chunks(const blco_dev* d, int mode, int tpw, bool long_rows, bool mid_rows)
 {
     const uint64_t base = (uint64_t)WAVE * tpw, cap = 2 * base;
     const int ntiles = std::max(1, d->stiles[mode]);
@@ -712,7 +712,7 @@ static std::vector<Chunk> sorted_chunks(const blco_dev* d, int mode, int tpw, bo
     while (long_piece > cap && long_piece * PIECE_WAVES > d->nnz) long_piece /= 2;
     long_piece = std::max(long_piece, cap);
     // pieces of the rows between the two
-    const uint64_t mid_piece = long_rows ? std::max<uint64_t>(cap, 2 * WAVE * long_tpw(d->nnz)) : cap;
+    const uint64_t mid_piece = mid_rows ? std::max<uint64_t>(cap, 2 * WAVE * long_tpw(d->nnz)) : cap;
     std::vector<std::vector<Chunk>> tiles(ntiles);
     const std::vector<uint64_t>& runs = d->srun_h[mode];
     size_t r = 0;
@@ -789,7 +789,7 @@ static const ChunkTab* sorted_chunk_table(blco_dev* d, int mode, int tpw, bool l
 {
     for (auto& t : d->stabs[mode])
         if (t.tpw == tpw && t.long_rows == long_rows) return &t;
-    const std::vector<Chunk> h = sorted_chunks(d, mode, tpw, long_rows);
+    const std::vector<Chunk> h = sorted_chunks(d, mode, tpw, long_rows, long_rows);
     ChunkTab t;
     t.tpw = tpw;
     t.long_rows = long_rows;
@@ -1098,7 +1098,7 @@ int rows_batch_prepare(blco_dev* d, int mode, int rank, int ftype)
 
 std::vector<Chunk> rows_batch_chunks(const blco_dev* d, int mode, int tpw)
 {
-    return d->nnz ? sorted_chunks(d, mode, tpw, true) : std::vector<Chunk>();
+    return d->nnz ? sorted_chunks(d, mode, tpw, true, false) : std::vector<Chunk>();
 }
 
 MttkrpArgs rows_batch_args(const blco_dev* d, int mode, int rank)
