@@ -37,6 +37,7 @@ constexpr int LVL3_MAX_MODE_LENGTH = 100;     // src/utils.hpp:13
 constexpr int DEFAULT_TPW = 4;                // tiles of 64 per wave
 constexpr int SORTED_TPW = 16;                // tiles of 64 per wave, row-ordered kernel (most)
 constexpr uint64_t SORTED_TARGET_CHUNKS = 8192;
+constexpr uint64_t WINDOW_MAX_FINE = 256;     // fine chunks per entry of kernel 12 (most)
 constexpr int ROWS_LONG_TPW = 8;              // mean chunks from here on take k_mttkrp_rows' long rounds
 constexpr int DEFAULT_NPRTN = 1;
 constexpr uint32_t LVL3_CHUNKS_PER_WG = 64;  // at most
@@ -76,13 +77,29 @@ static int sorted_tpw(const blco_dev* d, int mode, int rank, int ftype)
     return (uint64_t)rank * (ftype == BLCO_F64 ? 8 : 4) > 128 && d->stiles[mode] > 1 ? ROWS_LONG_TPW : 2;
 }
 
-// Nonzeros of one streamed unit: a quarter of the tensor where that is below
-// the slot, so that copies and kernels of neighbouring units overlap (20M
-// nonzeros in slots of 2^24 were one unit of 16.8M, whose kernel nothing
-// overlapped, and one of 3.2M), but not so few that the copies' own cost shows.
-static uint64_t stream_unit(const blco_dev* d)
+// Units that a block of a streamed tensor passes through the slots in.  What
+// the copies do not hide is a unit's kernel that outlasts the copy of the next
+// unit, so a block that at least half as many nonzeros follow stays whole as
+// far as a slot holds it (5 modes, 4.4M nonzeros in blocks of 2.24M, 0.9M, 0.9M
+// and 0.36M, FP64: 7.4 ms whole, 7.8 with the first in two, 8.8 with it cut at
+// 2^21: a slot is filled again only when its kernel is through, and the copy of
+// 0.15M nonzeros does not cover the kernel of 2.1M).  Other blocks take equal
+// units of at most a quarter of the tensor, but not of so few nonzeros that the
+// copies' own cost shows (one block of 2.5M, FP32: 6.6 ms whole, 5.8 cut at
+// 2^21, 4.6 in halves).
+static uint64_t stream_units(const blco_dev* d, uint64_t b)
 {
-    return std::min(d->slot_nnz, std::max<uint64_t>(1ull << 21, (d->nnz + 3) / 4));
+    const uint64_t n = d->bnnz[b], after = d->nnz - d->bstart[b] - n;
+    const uint64_t unit = std::min(d->slot_nnz, after >= n / 2 ? n : std::max<uint64_t>(1ull << 21, (d->nnz + 3) / 4));
+    return n ? (n + unit - 1) / unit : 1;
+}
+
+// Where the unit that starts `at` nonzeros into its block ends (a piece that
+// crosses the end still belongs to it).
+static uint64_t stream_unit_end(const blco_dev* d, uint64_t b, uint64_t at)
+{
+    const uint64_t units = stream_units(d, b), n = d->bnnz[b];
+    return n * (at * units / n + 1) / units;
 }
 
 const ChunkTab* chunk_table(blco_dev* d, int tpw)
@@ -112,7 +129,8 @@ const ChunkTab* chunk_table(blco_dev* d, int tpw)
             uint32_t u0 = c0;
             uint64_t acc = 0;
             for (uint32_t c = c0; c < c1; ++c) {
-                if (acc + h[c].len > stream_unit(d) && c > u0) {
+                const uint64_t at = h[u0].begin - d->bstart[b];
+                if (c > u0 && (at + acc >= stream_unit_end(d, b, at) || acc + h[c].len > d->slot_nnz)) {
                     t.units.push_back({u0, c, h[u0].begin, acc});
                     u0 = c;
                     acc = 0;
@@ -256,7 +274,7 @@ static void choose_window(const blco_dev* d, int mode, uint32_t total, uint64_t 
     int best_k = 0, last_k = 0;
     uint32_t best_h = 0;
     double best_cost = -1.0;
-    for (int k = 0; k <= 8; ++k) {
+    for (int k = 0; 1u << k <= WINDOW_MAX_FINE; ++k) {
         for (uint32_t hot : {H, 0u}) {
             const uint64_t cap = total - hot;
             double cost = 0.0;
@@ -1277,7 +1295,9 @@ int mttkrp(blco_dev* d, int mode, int rank, int ftype, void* const* factors, voi
                 while (e < wt->first[b + 1] && !rc) {
                     uint32_t e1 = e;
                     uint64_t cnt = 0;
-                    while (e1 < wt->first[b + 1] && (e1 == e || cnt + wt->h_sc[e1].len <= stream_unit(d))) {
+                    const uint64_t at = wt->h_sc[e].begin - d->bstart[b], end = stream_unit_end(d, b, at);
+                    while (e1 < wt->first[b + 1] &&
+                           (e1 == e || (at + cnt < end && cnt + wt->h_sc[e1].len <= d->slot_nnz))) {
                         cnt += wt->h_sc[e1].len;
                         ++e1;
                     }
@@ -1720,7 +1740,9 @@ int create_device_tensor(int nmodes, const uint64_t* dims, const uint64_t* masks
             bool packed = false;
             try {
                 packed = !device_budget && pack_words(nmodes, d->masks, d->pos, nnz, coords, d->fine_begin, d->fine_len,
-                                                      &d->pack_h, &dwords, &widest);
+                                                      &d->pack_h, &dwords, &widest) &&
+                         // a unit's unpacking is a launch of its own: worth 2^20 bytes of copies
+                         nnz * 8 - dwords * 4 >= (nblocks - 1) << 20;
             } catch (const std::bad_alloc&) {
                 return cleanup(fail(BLCO_ENOMEM, "host tables of the packed words"));
             }
@@ -1754,7 +1776,10 @@ int create_device_tensor(int nmodes, const uint64_t* dims, const uint64_t* masks
         }
         uint64_t cap = std::min<uint64_t>(slot_nnz, nnz ? nnz : 1);
         if (d->h_packed) {  // whole fine chunks around a unit, and two dwords read past its end
-            cap = std::min<uint64_t>(std::min(slot_nnz, stream_unit(d)) + 2 * FINE_CHUNK, nnz);
+            uint64_t unit = 0;
+            for (uint64_t b = 0; b < nblocks; ++b)
+                unit = std::max(unit, block_nnz[b] / stream_units(d, b) + 1);
+            cap = std::min<uint64_t>(std::min(slot_nnz, unit + WINDOW_MAX_FINE * FINE_CHUNK) + 2 * FINE_CHUNK, nnz);
             d->packed_cap = (cap * widest + 31) / 32 + cap / FINE_CHUNK + nblocks + 4;
             for (int s = 0; s < 2; ++s)
                 if (hipMalloc(&d->slot_packed[s], d->packed_cap * 4) != hipSuccess)

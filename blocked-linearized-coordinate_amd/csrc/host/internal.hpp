@@ -144,7 +144,7 @@ struct PackChunk {
 };
 // The chunks' forms (and one more entry, whose `at` is the dword count), the
 // dwords and the widest width.  False when the fields overlap or packing
-// saves less than a byte per nonzero: the words stay as they are.
+// saves less than two bytes per nonzero: the words stay as they are.
 bool pack_words(int nmodes, const uint64_t* masks, const int* pos, uint64_t nnz, const uint64_t* coords,
                 const std::vector<uint64_t>& fbeg, const std::vector<uint32_t>& flen, std::vector<PackChunk>* chunks,
                 uint64_t* dwords, uint32_t* widest);

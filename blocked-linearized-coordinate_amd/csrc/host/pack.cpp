@@ -50,7 +50,7 @@ bool pack_words(int nmodes, const uint64_t* masks, const int* pos, uint64_t nnz,
         *widest = std::max<uint32_t>(*widest, pc.width);
     }
     *dwords = at;
-    return *widest <= 60 && bits <= nnz * 56;
+    return *widest <= 60 && bits <= nnz * 48;
 }
 
 void write_packed(int nmodes, const uint64_t* masks, const int* pos, const uint64_t* coords,
