@@ -628,8 +628,10 @@ def write_selector(path, widths, params, xmean, xstd):
 
 
 class Batch:
-    """Many resident device tensors decomposed together (one persistent
-    MTTKRP kernel per mode, graph-captured ALS sweeps)."""
+    """Many resident device tensors decomposed together: `cpals` runs one MTTKRP
+    launch per mode and order over row-ordered copies (the persistent kernel
+    where they do not fit) in graph-captured sweeps, `mttkrp` and `tune` the
+    persistent kernel."""
 
     def __init__(self, devs):
         self.devs = list(devs)

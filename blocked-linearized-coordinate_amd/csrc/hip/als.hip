@@ -789,7 +789,7 @@ __global__ __launch_bounds__(WG) void k_als_fold(const AlsTask* __restrict__ tas
 // partial rows, then the factorisation for the mode that comes next.  One
 // launch in place of six and of a factorisation on a side stream: a sweep of
 // a small tensor is bound by its launches, and the factorisation takes a few
-// microseconds (chol_inverse_wave).  With nothing to finish (update = 0) only
+// microseconds (ldl_inverse_wave).  With nothing to finish (update = 0) only
 // the factorisation, for the first mode of the first sweep.
 constexpr int FINISH_WG = 512;
 

@@ -449,16 +449,18 @@ constexpr uint64_t XCD_TILE_MIN_NNZ = 1ull << 22;
 constexpr uint64_t XCD_TILE_MIN_FACTOR = 2ull << 20;
 constexpr uint64_t XCD_TILE_RUN_RATIO = 256;
 constexpr double XCD_TILE_SLACK = 1.15;
-// The fiber kernel runs on a fiber-ordered copy whose fibers average at
-// least this many nonzeros (below, the plain row-ordered kernel runs on it).
-// BLCO_FIBERS=0 keeps the ALTO order within rows (no fibers), =1 runs the
-// fiber kernel whatever the fiber length (tests).
+// The fiber kernels (k_mttkrp_fiber for factors of 2 GiB and more, and the
+// windowed form on copies that BLCO_FIBERS=1 ordered) run on a fiber-ordered copy
+// whose fibers average at least this many nonzeros, and k_mttkrp_rows gathers
+// such a copy's inner rows first; below it the plain row-ordered kernels run on
+// it.  BLCO_FIBERS=0 keeps the ALTO order within rows (no fibers), =1 takes the
+// fiber order whatever the fiber length (tests).
 constexpr double FIBER_MIN_LEN = 1.25;
 // Fiber order is chosen only when the inner factor holds at least this many
-// bytes at the first call's rank and type (smaller ones stay in L2, where
-// the gathers the fibers save are cheap).  The FP64 fiber kernel holds 108
-// VGPRs (4 waves per SIMD against 5 for the plain kernel), so for FP64
-// factors it pays only once most inner gathers miss the caches.
+// bytes at the first call's rank and type: smaller ones stay in L2.  The lines
+// were drawn with fiber kernels that gathered an outer row once per fiber, in
+// FP64 with 108 VGPRs; k_mttkrp_rows, which gathers it for every nonzero, was
+// not timed on either side of them.
 constexpr uint64_t FIBER_MIN_INNER = 2ull << 20;
 constexpr uint64_t FIBER_MIN_INNER_F64 = 64ull << 20;
 

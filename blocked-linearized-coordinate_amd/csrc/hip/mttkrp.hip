@@ -20,9 +20,9 @@
 // which has no wave64 equivalent.
 //
 // lvl3 ("privatised"): every product is added into a workgroup-private copy of
-// the whole output held in LDS (short modes only), with the gathers of the
-// row-ordered kernel and no segmentation (factors of 2 GiB and more keep lvl1's
-// tiles and segments); at the end the workgroup adds its copy into partial matrix
+// the whole output held in LDS as doubles (short modes only), with the gathers of
+// the row-ordered kernel and no segmentation (factors of 2 GiB and more keep
+// lvl1's tiles and segments); at the end the workgroup adds its copy into partial matrix
 // (workgroup % nprtn) -- or straight into the output when nprtn == 1 -- and
 // a pull reduction sums the partial matrices (partial_matrix_reduction,
 // src/alto_dev.cu:1589-1601).

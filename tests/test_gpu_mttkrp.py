@@ -99,9 +99,10 @@ def test_row_ordered_all_shapes(B, O, gpu, tensors, name):
 @pytest.mark.parametrize("nnz", [1_500_000, 3_000_000])
 def test_row_ordered_default_chunk_lengths(B, O, gpu, nnz):
     """Kernel 14 at its default chunk length for tensors between 2^20 and
-    2^22 nonzeros (4 and 8 tiles of 64 per wave; the small shapes above take
-    2 and the 40M-nonzero tensor 16), FP64 at rank 32 and FP32 at rank 20,
-    on a 4-mode tensor with Zipf-skewed modes."""
+    2^22 nonzeros (2 tiles of 64 per wave, rows of thousands of nonzeros in
+    longer pieces; the small shapes above take 1 tile, larger tensors are in
+    test_gpu_rows.py), FP64 at rank 32 and FP32 at rank 20, on a 4-mode tensor
+    with Zipf-skewed modes."""
     dims = (3000, 2000, 500, 40)
     t = B.Coo.generate(dims, nnz, zipf=(1.1, 0.8, 0.0, 0.0), gen_rank=5, value_kind=1, seed=nnz % 9973,
                        topup=True)
@@ -132,9 +133,10 @@ def test_row_ordered_xcd_tiles(B, O, gpu, tensors, name, monkeypatch):
 @pytest.mark.parametrize("name", [n for n in CASES if n != "order2"])
 @pytest.mark.parametrize("tiles", ["0", "1"])
 def test_fiber_kernel(B, O, gpu, tensors, name, tiles, monkeypatch):
-    """The fiber kernel (forced on: these small tensors have short fibers)
-    over fiber-ordered copies, untiled and with 8 forced tiles, for every
-    precision and for ranks that do not fill a lane group."""
+    """Fiber-ordered copies (forced: these small tensors have short fibers), whose
+    windowed fiber kernel gives way to k_mttkrp_rows where no window pays,
+    untiled and with 8 forced tiles, for every precision and for ranks that do
+    not fill a lane group."""
     monkeypatch.setenv("BLCO_FIBERS", "1")
     monkeypatch.setenv("BLCO_XCD_TILES", tiles)
     check(B, O, tensors, name, 0, B.K_SORTED, 32)
